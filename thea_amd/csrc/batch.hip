@@ -188,23 +188,21 @@ __device__ __forceinline__ uint32_t batch_key(float3 p, const int *__restrict__ 
 
 __global__ void __launch_bounds__(BB) k_bkeys(const float4 *__restrict__ center, const MeshInfo *__restrict__ mi, int nm,
                                               const int *__restrict__ mb, int mesh_bits, int64_t n,
-                                              uint32_t *__restrict__ keys, uint32_t *__restrict__ vals) {
+                                              uint32_t *__restrict__ keys) {
   int64_t e = (int64_t)blockIdx.x * BB + threadIdx.x;
   if (e >= n) return;
   int m = mesh_of(mi, nm, e, false, false);
   float4 c = center[e];
   keys[e] = batch_key(f3(c.x, c.y, c.z), mb, m, mesh_bits, true);
-  vals[e] = (uint32_t)e;
 }
 
 __global__ void __launch_bounds__(BB) k_bqkeys(const float *__restrict__ q, const MeshInfo *__restrict__ mi, int nm,
                                                const int *__restrict__ mb, int mesh_bits, int64_t n,
-                                               uint32_t *__restrict__ keys, uint32_t *__restrict__ vals) {
+                                               uint32_t *__restrict__ keys) {
   int64_t j = (int64_t)blockIdx.x * BB + threadIdx.x;
   if (j >= n) return;
   int m = mesh_of(mi, nm, j, true, false);
   keys[j] = batch_key(f3(q[3 * j], q[3 * j + 1], q[3 * j + 2]), mb, m, mesh_bits, false);
-  vals[j] = (uint32_t)j;
 }
 
 // Common prefix of sorted keys at global positions i, j of one mesh [a, b); -1 outside.
@@ -359,10 +357,10 @@ static void plan_pipeline(BatchPlan &P, hipStream_t s, hipEvent_t mid = nullptr)
                        mi, P.d_tchunks.as<int4>(), P.center.as<float4>(), P.blo.as<float4>(), P.bhi.as<float4>(), mb);
     launch_check("k_bprep");
     hipLaunchKernelGGL(k_bkeys, dim3(ceil_div(P.NT, BB)), dim3(BB), 0, s, P.center.as<float4>(), mi, nm, mb, P.mesh_bits,
-                       P.NT, P.keys.as<uint32_t>(), P.vals.as<uint32_t>());
+                       P.NT, P.keys.as<uint32_t>());
     launch_check("k_bkeys");
-    radix_sort_pairs(P.keys.as<uint32_t>(), P.vals.as<uint32_t>(), P.tk.as<uint32_t>(), P.tv.as<uint32_t>(),
-                     P.hist.as<uint32_t>(), P.NT, 0, 32, s);
+    radix_sort_iota(P.keys.as<uint32_t>(), P.vals.as<uint32_t>(), P.tk.as<uint32_t>(), P.tv.as<uint32_t>(),
+                    P.hist.as<uint32_t>(), P.NT, 0, 32, s);
     hipLaunchKernelGGL(k_bkarras, dim3(ceil_div(P.NT, BB)), dim3(BB), 0, s, P.keys.as<uint32_t>(), mi, nm, P.NT,
                        P.left.as<int32_t>(), P.right.as<int32_t>(), P.rfirst.as<int32_t>(), P.rlast.as<int32_t>(),
                        P.nparent.as<int32_t>(), P.lparent.as<int32_t>());
@@ -391,14 +389,13 @@ static void plan_pipeline(BatchPlan &P, hipStream_t s, hipEvent_t mid = nullptr)
   if (P.NQ > 0) {
     // queries: reuse the key/value buffers (the element order is no longer needed after the records)
     hipLaunchKernelGGL(k_bqkeys, dim3(ceil_div(P.NQ, BB)), dim3(BB), 0, s, P.queries.as<float>(), mi, nm, mb, P.mesh_bits,
-                       P.NQ, P.keys.as<uint32_t>(), P.vals.as<uint32_t>());
+                       P.NQ, P.keys.as<uint32_t>());
     launch_check("k_bqkeys");
-    radix_sort_pairs(P.keys.as<uint32_t>(), P.vals.as<uint32_t>(), P.tk.as<uint32_t>(), P.tv.as<uint32_t>(),
-                     P.hist.as<uint32_t>(), P.NQ, 0, 32, s);
+    const uint32_t *qorder = radix_sort_order(P.keys.as<uint32_t>(), P.vals.as<uint32_t>(), P.tk.as<uint32_t>(),
+                                              P.tv.as<uint32_t>(), P.hist.as<uint32_t>(), P.NQ, 0, 32, false, s);
     hipLaunchKernelGGL(k_bsegs, dim3(ceil_div(nm, BB)), dim3(BB), 0, s, mi, nm, mb, P.fidx.as<uint32_t>(), P.nsmall,
                        P.nodes.as<BNode>(), P.recs.as<TriRec>(), P.screen.as<ScreenRec>(), P.queries.as<float>(),
-                       P.vals.as<uint32_t>(),
-                       P.out_idx.as<int32_t>(), P.out_dist.as<float>(), P.seg.as<SegDesc>());
+                       qorder, P.out_idx.as<int32_t>(), P.out_dist.as<float>(), P.seg.as<SegDesc>());
     launch_check("k_bsegs");
     hipLaunchKernelGGL(k_bempty, dim3(ceil_div(P.NQ, BB)), dim3(BB), 0, s, mi, nm, P.NQ, P.out_idx.as<int32_t>(),
                        P.out_dist.as<float>());

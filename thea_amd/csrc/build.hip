@@ -113,12 +113,11 @@ __device__ __forceinline__ uint32_t morton30(float3 c, float3 lo, float3 inv) {
 }
 
 __global__ void __launch_bounds__(B_BLOCK) k_morton(const float4 *__restrict__ center, int64_t n, float3 lo, float3 inv,
-                                                    uint32_t *__restrict__ keys, uint32_t *__restrict__ vals) {
+                                                    uint32_t *__restrict__ keys) {
   int64_t i = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
   if (i >= n) return;
   float4 c = center[i];
   keys[i] = morton30(f3(c.x, c.y, c.z), lo, inv);
-  vals[i] = (uint32_t)i;
 }
 
 // Common prefix length of sorted (code, position) keys i and j; -1 outside [0, n).
@@ -815,9 +814,9 @@ void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool 
   float3 cext = f3(f[9] - f[6], f[10] - f[7], f[11] - f[8]);
   float3 inv = f3(cext.x > 0 ? 1.0f / cext.x : 0.0f, cext.y > 0 ? 1.0f / cext.y : 0.0f, cext.z > 0 ? 1.0f / cext.z : 0.0f);
   hipLaunchKernelGGL(k_morton, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, center.as<float4>(), n, clo, inv,
-                     keys.as<uint32_t>(), vals.as<uint32_t>());
+                     keys.as<uint32_t>());
   launch_check("k_morton");
-  radix_sort_pairs(keys.as<uint32_t>(), vals.as<uint32_t>(), tk.as<uint32_t>(), tv.as<uint32_t>(), hist.as<uint32_t>(), n,
+  radix_sort_iota(keys.as<uint32_t>(), vals.as<uint32_t>(), tk.as<uint32_t>(), tv.as<uint32_t>(), hist.as<uint32_t>(), n,
                    0, 32, s);
   const uint32_t *sorted = vals.as<uint32_t>();
 

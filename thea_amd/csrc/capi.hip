@@ -71,6 +71,8 @@ void check_tri_indices(const int32_t *tris, int64_t nt, int64_t nv, hipStream_t 
 // the library's load on that device until the process ends.
 constexpr size_t NOALLOC_WORDS = 4 * (size_t)THG_NOALLOC_MAX_QUERIES +
                                  256 * (((size_t)THG_NOALLOC_MAX_QUERIES + 4095) / 4096) + 256;
+static_assert((size_t)THG_NOALLOC_MAX_QUERIES / RS_TILE_LARGE >= RS_SMALL_MAX / RS_TILE_SMALL,
+              "a smaller batch's histograms may need more words");
 static __device__ __align__(256) uint32_t scratch[NOALLOC_WORDS];
 
 constexpr int NOALLOC_DEVICES = 64;

@@ -102,11 +102,46 @@ inline void launch_check(const char *name) {
 
 inline uint32_t ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-// Radix sort of (key, value) pairs over key bits [begin_bit, end_bit), stable, LSD with 8-bit
-// digits. keys/vals are sorted in place (using tmp_keys/tmp_vals as the ping-pong partner);
-// `hist` must hold radix_hist_words(n) uint32.
-void radix_sort_pairs(uint32_t *keys, uint32_t *vals, uint32_t *tmp_keys, uint32_t *tmp_vals, uint32_t *hist,
-                      int64_t n, int begin_bit, int end_bit, hipStream_t s);
+// Radix sort (radix_sort.hip): 8-bit digits, tiles of 1,024 pairs up to 2^20 pairs (a tile of 4,096
+// would leave most CUs idle: 25 workgroups for 100,000 pairs) and of 4,096 above (runs of equal
+// digits four times as long to write).
+constexpr int RS_BLOCK = 256;
+constexpr int RS_ITEMS_SMALL = 4, RS_ITEMS_LARGE = 16;
+constexpr uint64_t RS_TILE_SMALL = RS_BLOCK * RS_ITEMS_SMALL, RS_TILE_LARGE = RS_BLOCK * RS_ITEMS_LARGE;
+constexpr int64_t RS_SMALL_MAX = (int64_t)1 << 20;
+
+// Digit counts of one tile, in LDS. A key kernel that processes whole tiles in 256-thread blocks
+// fills one (clear, count every key, store) and so saves the sort its first histogram pass.
+struct RadixHist {
+  uint32_t h[256];
+  __device__ __forceinline__ void clear() {
+    h[threadIdx.x] = 0;
+    __syncthreads();
+  }
+  __device__ __forceinline__ void count(uint32_t key, int shift) { atomicAdd(&h[(key >> shift) & 0xFF], 1u); }
+  __device__ __forceinline__ void store(uint32_t *__restrict__ hist, uint32_t tiles) {
+    __syncthreads();
+    hist[(size_t)threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
+  }
+};
+inline int radix_items(int64_t n) { return n <= RS_SMALL_MAX ? RS_ITEMS_SMALL : RS_ITEMS_LARGE; }
+inline uint32_t radix_tiles(int64_t n) { return ceil_div((uint64_t)n, (uint64_t)RS_BLOCK * radix_items(n)); }
+
+// Where a sort left its results.
+struct RadixResult {
+  const uint32_t *keys, *vals;
+};
+
+// The stable order of n keys by bits [begin_bit, end_bit): returns the positions in that order, in
+// vals or tmp_vals. vals needs no input; the keys' own order is lost. first_hist: the caller's key
+// kernel has stored the first digit's histograms (RadixHist) in hist. `hist` must hold
+// radix_hist_words(n) words.
+const uint32_t *radix_sort_order(uint32_t *keys, uint32_t *vals, uint32_t *tmp_keys, uint32_t *tmp_vals,
+                                 uint32_t *hist, int64_t n, int begin_bit, int end_bit, bool first_hist,
+                                 hipStream_t s);
+// The same order with the sorted keys in `keys` and the positions in `vals`.
+void radix_sort_iota(uint32_t *keys, uint32_t *vals, uint32_t *tmp_keys, uint32_t *tmp_vals, uint32_t *hist,
+                     int64_t n, int begin_bit, int end_bit, hipStream_t s);
 size_t radix_hist_words(int64_t n);
 
 }  // namespace thg

@@ -2251,35 +2251,45 @@ __device__ __forceinline__ uint32_t spread10q(uint32_t v) {
   return v;
 }
 
-__global__ void __launch_bounds__(256) k_query_keys(const float *__restrict__ q, int64_t n, float3 lo, float3 inv,
-                                                    uint32_t *__restrict__ keys, uint32_t *__restrict__ vals) {
-  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  float3 p = load_q(q, i);
+__device__ __forceinline__ uint32_t query_key(float3 p, float3 lo, float3 inv) {
   float x = (p.x - lo.x) * inv.x, y = (p.y - lo.y) * inv.y, z = (p.z - lo.z) * inv.z;
   // NaN coordinates map to cell 0 (fmaxf drops NaN).
   uint32_t ix = (uint32_t)fminf(fmaxf(x * 1024.0f, 0.0f), 1023.0f);
   uint32_t iy = (uint32_t)fminf(fmaxf(y * 1024.0f, 0.0f), 1023.0f);
   uint32_t iz = (uint32_t)fminf(fmaxf(z * 1024.0f, 0.0f), 1023.0f);
-  keys[i] = (spread10q(ix) << 2) | (spread10q(iy) << 1) | spread10q(iz);
-  vals[i] = (uint32_t)i;
+  return (spread10q(ix) << 2) | (spread10q(iy) << 1) | spread10q(iz);
 }
 
 // Ray tracing order key: the direction's octant (3 bits) above the 27-bit Morton code of the
 // origin (9 bits per axis), so that a wave takes rays of one octant from nearby origins.
-__global__ void __launch_bounds__(256) k_ray_keys(const float *__restrict__ o, const float *__restrict__ d, int64_t n,
-                                                  float3 lo, float3 inv, uint32_t *__restrict__ keys,
-                                                  uint32_t *__restrict__ vals) {
-  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  float3 p = load_q(o, i), v = load_q(d, i);
+__device__ __forceinline__ uint32_t ray_key(float3 p, float3 v, float3 lo, float3 inv) {
   float x = (p.x - lo.x) * inv.x, y = (p.y - lo.y) * inv.y, z = (p.z - lo.z) * inv.z;
   uint32_t ix = (uint32_t)fminf(fmaxf(x * 512.0f, 0.0f), 511.0f);
   uint32_t iy = (uint32_t)fminf(fmaxf(y * 512.0f, 0.0f), 511.0f);
   uint32_t iz = (uint32_t)fminf(fmaxf(z * 512.0f, 0.0f), 511.0f);
   const uint32_t oct = (v.x < 0 ? 4u : 0u) | (v.y < 0 ? 2u : 0u) | (v.z < 0 ? 1u : 0u);
-  keys[i] = (oct << 27) | (spread10q(ix) << 2) | (spread10q(iy) << 1) | spread10q(iz);
-  vals[i] = (uint32_t)i;
+  return (oct << 27) | (spread10q(ix) << 2) | (spread10q(iy) << 1) | spread10q(iz);
+}
+
+// Order keys of a batch and the histograms of their first sorted digit, one sort tile per block
+// (d null: query keys of q, else ray keys).
+template <int ITEMS>
+__global__ void __launch_bounds__(RS_BLOCK) k_order_keys(const float *__restrict__ q, const float *__restrict__ d,
+                                                         int64_t n, float3 lo, float3 inv, int shift, uint32_t tiles,
+                                                         uint32_t *__restrict__ keys, uint32_t *__restrict__ hist) {
+  __shared__ RadixHist h;
+  h.clear();
+  const int64_t base = (int64_t)blockIdx.x * (RS_BLOCK * ITEMS);
+#pragma unroll 4
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t i = base + (int64_t)r * RS_BLOCK + threadIdx.x;
+    if (i < n) {
+      const uint32_t key = d ? ray_key(load_q(q, i), load_q(d, i), lo, inv) : query_key(load_q(q, i), lo, inv);
+      keys[i] = key;
+      h.count(key, shift);
+    }
+  }
+  h.store(hist, tiles);
 }
 
 //--------------------------------------------------------------------------------------------------
@@ -2305,10 +2315,13 @@ int group_lanes_log2(int64_t n, int depth) {
   return lg;
 }
 
-// Lowest Morton bit the query sort uses (THG_ORDER_BITS = number of top bits of the 30, default 24).
-static int order_bits_lo() {
+// Lowest key bit an order of n queries sorts by (THG_ORDER_BITS = number of top bits of the 30).
+// 24 bits (cells of 1/256 of the scene per axis, 3 radix passes) serve millions of queries (30 bits,
+// 4 passes, is no faster on C3); below 2^18 queries 16 bits already give about a cell per query, and
+// each pass saved is three launches.
+int order_bits_lo(int64_t n) {
   static const char *env = getenv("THG_ORDER_BITS");
-  int bits = env ? atoi(env) : 24;  // 3 radix passes; 30 bits (4 passes) is no faster on C3
+  int bits = env ? atoi(env) : (n < ((int64_t)1 << 18) ? 16 : 24);
   bits = bits < 8 ? 8 : (bits > 30 ? 30 : bits);
   return 30 - bits;
 }
@@ -2329,19 +2342,29 @@ QueryScratch::Sort QueryScratch::sort_memory(int64_t n, hipStream_t s) {
   return Sort{keys.as<uint32_t>(), vals.as<uint32_t>(), tk.as<uint32_t>(), tv.as<uint32_t>(), hist.as<uint32_t>()};
 }
 
-void order_queries(const Bvh &b, const float *q, int64_t n, QueryScratch &ws, hipStream_t s) {
+// Spatial order of n queries (d null) or rays into ws.order.
+static void order_batch(const Bvh &b, const float *q, const float *d, int64_t n, QueryScratch &ws, hipStream_t s) {
   ws.order = nullptr;
   if (n < ORDER_MIN_QUERIES) return;
   KernelTimer kt(ws.timer_ctx(b.ctx), s, "order");
   const QueryScratch::Sort m = ws.sort_memory(n, s);
   float3 ext = f3(b.hi.x - b.lo.x, b.hi.y - b.lo.y, b.hi.z - b.lo.z);
   float3 inv = f3(ext.x > 0 ? 1.0f / ext.x : 0.0f, ext.y > 0 ? 1.0f / ext.y : 0.0f, ext.z > 0 ? 1.0f / ext.z : 0.0f);
-  hipLaunchKernelGGL(k_query_keys, dim3(ceil_div(n, 256)), dim3(256), 0, s, q, n, b.lo, inv, m.keys, m.vals);
-  launch_check("k_query_keys");
-  // The top 24 of the 30 code bits give cells of 1/256 of the scene per axis: enough coherence.
-  radix_sort_pairs(m.keys, m.vals, m.tk, m.tv, m.hist, n, order_bits_lo(), 30, s);
-  ws.order = m.vals;
+  const uint32_t tiles = radix_tiles(n);
+  const int lo_bit = order_bits_lo(n);
+  if (radix_items(n) == RS_ITEMS_SMALL)
+    hipLaunchKernelGGL(k_order_keys<RS_ITEMS_SMALL>, dim3(tiles), dim3(RS_BLOCK), 0, s, q, d, n, b.lo, inv, lo_bit,
+                       tiles, m.keys, m.hist);
+  else
+    hipLaunchKernelGGL(k_order_keys<RS_ITEMS_LARGE>, dim3(tiles), dim3(RS_BLOCK), 0, s, q, d, n, b.lo, inv, lo_bit,
+                       tiles, m.keys, m.hist);
+  launch_check("k_order_keys");
+  ws.order = radix_sort_order(m.keys, m.vals, m.tk, m.tv, m.hist, n, lo_bit, 30, true, s);
   kt.stop();
+}
+
+void order_queries(const Bvh &b, const float *q, int64_t n, QueryScratch &ws, hipStream_t s) {
+  order_batch(b, q, nullptr, n, ws, s);
 }
 
 // Tracing order of a ray batch: direction octant, then origin Morton code (THG_RAY_ORDER=origin:
@@ -2352,21 +2375,7 @@ void order_rays(const Bvh &b, const float *o, const float *d, int64_t n, QuerySc
     const char *e = getenv("THG_RAY_ORDER");
     return e && std::string(e) == "origin";
   }();
-  if (by_origin) {
-    order_queries(b, o, n, ws, s);
-    return;
-  }
-  ws.order = nullptr;
-  if (n < ORDER_MIN_QUERIES) return;
-  KernelTimer kt(ws.timer_ctx(b.ctx), s, "order");
-  const QueryScratch::Sort m = ws.sort_memory(n, s);
-  float3 ext = f3(b.hi.x - b.lo.x, b.hi.y - b.lo.y, b.hi.z - b.lo.z);
-  float3 inv = f3(ext.x > 0 ? 1.0f / ext.x : 0.0f, ext.y > 0 ? 1.0f / ext.y : 0.0f, ext.z > 0 ? 1.0f / ext.z : 0.0f);
-  hipLaunchKernelGGL(k_ray_keys, dim3(ceil_div(n, 256)), dim3(256), 0, s, o, d, n, b.lo, inv, m.keys, m.vals);
-  launch_check("k_ray_keys");
-  radix_sort_pairs(m.keys, m.vals, m.tk, m.tv, m.hist, n, order_bits_lo(), 30, s);
-  ws.order = m.vals;
-  kt.stop();
+  order_batch(b, o, by_origin ? nullptr : d, n, ws, s);
 }
 
 static float prev_float(float x) { return std::nextafter(x, -INFINITY); }

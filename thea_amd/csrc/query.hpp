@@ -68,6 +68,7 @@ void check_tri_indices(const int32_t *tris, int64_t nt, int64_t nv, hipStream_t 
 void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool points, int leaf_size, hipStream_t s);
 // The 4-wide quantized ray tree (Bvh::qnodes) of a built mesh BVH; synchronises `s`.
 void build_qbvh4(Bvh &b, hipStream_t s);
+int order_bits_lo(int64_t n);
 void order_queries(const Bvh &b, const float *q, int64_t n, QueryScratch &ws, hipStream_t s);
 void order_rays(const Bvh &b, const float *o, const float *d, int64_t n, QueryScratch &ws, hipStream_t s);
 float bound_to_best(double dist_bound);

@@ -83,7 +83,7 @@ __device__ __forceinline__ uint32_t spread10_64(uint32_t v) {
 
 // Morton key of each double query (rounded to float) in the scene box, for the spatial sort.
 __global__ void __launch_bounds__(256) k_query_keys64(const double *__restrict__ q, int64_t n, float3 lo, float3 inv,
-                                                      uint32_t *__restrict__ keys, uint32_t *__restrict__ vals) {
+                                                      uint32_t *__restrict__ keys) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const float px = (float)q[3 * i], py = (float)q[3 * i + 1], pz = (float)q[3 * i + 2];
@@ -92,7 +92,6 @@ __global__ void __launch_bounds__(256) k_query_keys64(const double *__restrict__
   const uint32_t iy = (uint32_t)fminf(fmaxf(y * 1024.0f, 0.0f), 1023.0f);
   const uint32_t iz = (uint32_t)fminf(fmaxf(z * 1024.0f, 0.0f), 1023.0f);
   keys[i] = (spread10_64(ix) << 2) | (spread10_64(iy) << 1) | spread10_64(iz);
-  vals[i] = (uint32_t)i;
 }
 
 __global__ void __launch_bounds__(B64) k_closest64(const BNode *__restrict__ nodes, const PointRecD *__restrict__ pr,
@@ -277,10 +276,9 @@ void order_queries64(const Bvh &b, const double *q, int64_t n, QueryScratch &ws,
   const float3 ext = f3(b.hi.x - b.lo.x, b.hi.y - b.lo.y, b.hi.z - b.lo.z);
   const float3 inv =
       f3(ext.x > 0 ? 1.0f / ext.x : 0.0f, ext.y > 0 ? 1.0f / ext.y : 0.0f, ext.z > 0 ? 1.0f / ext.z : 0.0f);
-  hipLaunchKernelGGL(k_query_keys64, dim3(ceil_div(n, 256)), dim3(256), 0, s, q, n, b.lo, inv, m.keys, m.vals);
+  hipLaunchKernelGGL(k_query_keys64, dim3(ceil_div(n, 256)), dim3(256), 0, s, q, n, b.lo, inv, m.keys);
   launch_check("k_query_keys64");
-  radix_sort_pairs(m.keys, m.vals, m.tk, m.tv, m.hist, n, 6, 30, s);
-  ws.order = m.vals;
+  ws.order = radix_sort_order(m.keys, m.vals, m.tk, m.tv, m.hist, n, order_bits_lo(n), 30, false, s);
 }
 
 double bound_to_best64(double dist_bound) {

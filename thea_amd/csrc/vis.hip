@@ -71,8 +71,7 @@ __device__ __forceinline__ uint32_t vis_spread7(uint32_t v) {  // 7 bits -> ever
 // points rather than 64 random directions from one point (74.4 -> 67.6 ms per 100M C3 rays; an
 // 8 x 8 octahedral direction grid over a 6-bit-per-axis origin code measured 70.9 ms).
 __global__ void __launch_bounds__(256) k_vis_keys(const float *__restrict__ org, const float *__restrict__ dir,
-                                                  int64_t m, float3 lo, float3 inv, uint32_t *__restrict__ keys,
-                                                  uint32_t *__restrict__ vals) {
+                                                  int64_t m, float3 lo, float3 inv, uint32_t *__restrict__ keys) {
   const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (g >= m) return;
   const float x = (org[3 * g] - lo.x) * inv.x, y = (org[3 * g + 1] - lo.y) * inv.y, z = (org[3 * g + 2] - lo.z) * inv.z;
@@ -81,7 +80,6 @@ __global__ void __launch_bounds__(256) k_vis_keys(const float *__restrict__ org,
   const uint32_t iz = (uint32_t)fminf(fmaxf(z * 128.0f, 0.0f), 127.0f);
   const uint32_t oct = (dir[3 * g] < 0 ? 4u : 0u) | (dir[3 * g + 1] < 0 ? 2u : 0u) | (dir[3 * g + 2] < 0 ? 1u : 0u);
   keys[g] = (oct << 21) | (vis_spread7(ix) << 2) | (vis_spread7(iy) << 1) | vis_spread7(iz);
-  vals[g] = (uint32_t)g;
 }
 
 // One thread per point: the fraction of its rays that escaped.
@@ -151,12 +149,12 @@ extern "C" int thg_visibility(thg_bvh mesh_bvh, const float *positions, int64_t 
                          org.as<float>(), dir.as<float>());
       launch_check("k_vis_rays");
       hipLaunchKernelGGL(k_vis_keys, dim3(ceil_div(m, 256)), dim3(256), 0, s, org.as<float>(), dir.as<float>(), m, b->lo,
-                         inv, keys.as<uint32_t>(), vals.as<uint32_t>());
+                         inv, keys.as<uint32_t>());
       launch_check("k_vis_keys");
-      radix_sort_pairs(keys.as<uint32_t>(), vals.as<uint32_t>(), tk.as<uint32_t>(), tv.as<uint32_t>(),
-                       hist.as<uint32_t>(), m, 0, 24, s);
+      const uint32_t *order = radix_sort_order(keys.as<uint32_t>(), vals.as<uint32_t>(), tk.as<uint32_t>(),
+                                               tv.as<uint32_t>(), hist.as<uint32_t>(), m, 0, 24, false, s);
       launch_ray(*b, org.as<float>(), dir.as<float>(), m, -1.0f, true, nullptr, nullptr, nullptr, hit.as<uint8_t>(), ws,
-                 s, /*sort_rays=*/false, vals.as<uint32_t>());
+                 s, /*sort_rays=*/false, order);
       hipLaunchKernelGGL(k_vis_count, dim3(ceil_div(np, 256)), dim3(256), 0, s, hit.as<uint8_t>(), np, R,
                          d_vis + p0);
       launch_check("k_vis_count");
