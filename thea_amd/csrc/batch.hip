@@ -35,7 +35,7 @@ struct MeshInfo {  // per mesh, device side
   int32_t leaf, small_slot;  // small_slot >= 0: index of its single-leaf root node
   uint64_t wave_begin;       // first 64-query wave of the mesh within its traversal group
   int32_t seg_slot;          // row of the segment table (wave-cooperative meshes first)
-  int32_t lane;              // > 0: log2 lanes per query (sparse queries), 0: wave-cooperative
+  int32_t lane;              // > 0: work queue, log2 lanes per query; 0: wave-cooperative
   int32_t child_order;       // visiting order of the closest-point kernel on this mesh (CHILD_*)
 };
 
@@ -402,19 +402,8 @@ static void plan_pipeline(BatchPlan &P, hipStream_t s, hipEvent_t mid = nullptr)
     launch_check("k_bempty");
     launch_closest_multi(P.seg.as<SegDesc>(), P.nwave_meshes, P.total_waves, false, s, false, P.block_waves,
                          P.spill_build);
-    launch_closest_group_multi(P.seg.as<SegDesc>() + P.nwave_meshes, nm - P.nwave_meshes, P.lane_waves, false, 64, s);
+    launch_closest_queue_multi(P.seg.as<SegDesc>() + P.nwave_meshes, nm - P.nwave_meshes, P.lane_waves, s);
   }
-}
-
-// Sparse meshes of a plan share each query among 2-64 lanes when THG_BATCH_LANE=1 (default: every
-// mesh uses the wave-cooperative kernel; the per-query kernel must reserve a 64-entry stack here
-// because the depth is known only after the captured build).
-static bool batch_lane_split() {
-  static const bool v = [] {
-    const char *e = getenv("THG_BATCH_LANE");
-    return e && atoi(e) == 1;
-  }();
-  return v;
 }
 
 // Fails with THG_E_INVALID unless every triangle's vertex indices lie in its own mesh's vertices
@@ -466,11 +455,16 @@ static double time_plan_kernel(const Bvh &b, const float *q, int64_t n, int chil
   d.scale = b.scale;
   d.nelem = (int32_t)b.n;
   d.child_order = child_order;
+  d.lanes_log2 = use_queue(n, b.n, 0) ? queue_lanes_log2(n) : 0;
   THG_HIP(hipMemcpyAsync(dseg.p, &d, sizeof(SegDesc), hipMemcpyHostToDevice, s));
-  const uint64_t waves = (uint64_t)((n + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES);
-  launch_closest_multi(dseg.as<SegDesc>(), 1, waves, false, s, false, block_waves, spill);
+  const uint64_t waves = (uint64_t)(((n << d.lanes_log2) + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES);
+  auto launch = [&] {
+    if (d.lanes_log2) launch_closest_queue_multi(dseg.as<SegDesc>(), 1, waves, s);
+    else launch_closest_multi(dseg.as<SegDesc>(), 1, waves, false, s, false, block_waves, spill);
+  };
+  launch();
   THG_HIP(hipEventRecord(e0, s));
-  for (int r = 0; r < reps; ++r) launch_closest_multi(dseg.as<SegDesc>(), 1, waves, false, s, false, block_waves, spill);
+  for (int r = 0; r < reps; ++r) launch();
   THG_HIP(hipEventRecord(e1, s));
   THG_HIP(hipEventSynchronize(e1));
   float ms = 0;
@@ -516,6 +510,9 @@ int thg_batch_plan_create(thg_ctx ctx, int32_t nm, const int64_t *nv, const int6
     P->info.resize(nm);
     int64_t vo = 0, to = 0, qo = 0, io = 0;
     uint64_t waves = 0, lwaves = 0;
+    int64_t queue_n = 0;  // queries of the meshes whose queries take the work-queue kernel
+    for (int m = 0; m < nm; ++m)
+      if (nq[m] > 0 && nt[m] > 0 && use_queue(nq[m], nt[m], 0)) queue_n += nq[m];
     for (int m = 0; m < nm; ++m) {
       require(nv[m] >= 0 && nt[m] >= 0 && nq[m] >= 0, "negative count");
       int leaf = leaf_sizes ? leaf_sizes[m] : 4;
@@ -524,10 +521,7 @@ int thg_batch_plan_create(thg_ctx ctx, int32_t nm, const int64_t *nv, const int6
       x.voff = vo; x.toff = to; x.qoff = qo; x.ioff = io;
       x.nt = nt[m]; x.nq = nq[m]; x.nv = nv[m]; x.leaf = leaf;
       x.small_slot = (nt[m] >= 1 && nt[m] <= leaf) ? P->nsmall++ : -1;
-      // The single-call rule (use_wave_traversal): wave-cooperative when there is at least one query
-      // per 8 leaves; a collapsed LBVH has about 1.5 * triangles / leaf_size leaves.
-      const int64_t leaves = (3 * nt[m]) / (2 * leaf) + 1;
-      x.lane = batch_lane_split() && 8 * nq[m] < leaves ? group_lanes_log2(nq[m], 0) : 0;
+      x.lane = use_queue(nq[m], nt[m], 0) ? queue_lanes_log2(queue_n) : 0;
       const uint64_t w =
           nt[m] > 0 ? (uint64_t)(((nq[m] << x.lane) + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES) : 0;
       if (x.lane) { x.wave_begin = lwaves; lwaves += w; }

@@ -812,6 +812,317 @@ __global__ void __launch_bounds__(WPB * WAVE, WAVES) k_closest_multi(const SegDe
 }
 
 //--------------------------------------------------------------------------------------------------
+// Closest triangle, sparse batches: a wave's work queue
+//
+// A wave owns Q = 64 >> lg queries (1..32) and keeps (query, node) pairs on a stack in LDS. Each step
+// its 64 lanes pop up to 64 pairs, whatever query they belong to, test both children of each against
+// that query's own best, and push the admitted ones, the farther child below the nearer. Admitted
+// leaves go to a second LDS list; 64 of them at a time are screened as in the compacted walk above
+// (leaf bound, then plane-and-disc bound per triangle), and the surviving (query, triangle) pairs are
+// evaluated 64 at a time by cmp_flush. So a query far inside a closed surface, which meets a large
+// part of the tree, uses all 64 lanes, and one that ends after a few nodes leaves its lanes to the
+// wave's other queries; a walk of its own per lane would last as long as its slowest query.
+// The stack is LIFO, so it holds about 64 paths; a step pops at most an eighth of the entries left
+// free, and one pair near the stack's end (a plain depth-first walk, which adds at most one entry per
+// level), so it never overflows in trees of at most 63 levels. The batched plan learns its depths
+// only afterwards: deeper trees drop entries there and the plan fails.
+// A query's walk begins when a step would otherwise not be full, so easy queries share the steps and
+// a hard one does not fill the stack beside 31 others.
+//
+// Bound by the latency of the per-lane node and record loads (a step is one dependent load): 16 waves
+// per CU (10 KB of LDS each) hide it. Against the kernels it replaced, on a 1,048,576-triangle torus
+// (leaf size 4): 61 queries 667 -> 41 us, 3,001 1,614 -> 84 us, 32,768 3,974 -> 360 us (lanes of a
+// group walking disjoint subtrees of the tree, without the screening bounds); on the 20,480-triangle
+// sphere 100,000 queries 1,341 -> 390 us and on the torus 1,000,000 queries uniform in the box 4,737 ->
+// 3,694 us, near the surface 2,359 -> 766 us (the compacted wave walk, whose 64 queries share one walk
+// and one critical path).
+// Results are the canonical minima whatever the order: a pair is dropped only when its bound exceeds
+// its query's best.
+//--------------------------------------------------------------------------------------------------
+constexpr int WQ_QUERIES = 32;  // most queries per wave
+constexpr int WQ_STACK = 1024;
+constexpr int WQ_LEAVES = 3 * WAVE;
+constexpr int WQ_FLUSH_LG = 3;  // up to 8 queries per wave: evaluate after every leaf step
+
+struct QueueWave {
+  float4 qp[WQ_QUERIES];                // query point; w = excluded triangle id as int bits
+  unsigned long long key[WQ_QUERIES];   // its best (d^2 bits << 32 | id)
+  int32_t slot[WQ_QUERIES];             // the best's triangle record
+  int32_t ref[WQ_STACK];                // stack: node, lower bound it was admitted with, owner
+  int32_t leaf[WQ_LEAVES];              // admitted leaves: first record, lower bound, count, owner
+  int32_t qe[2 * WAVE];                 // queued pairs: triangle record, owner
+  uint16_t lb[WQ_STACK], llb[WQ_LEAVES];
+  uint8_t own[WQ_STACK], lcnt[WQ_LEAVES], lown[WQ_LEAVES], qo[2 * WAVE];
+};
+static_assert(sizeof(QueueWave) == 10240, "16 waves per CU (160 KB of LDS)");
+
+// A bound (>= 0) kept in 16 bits, cut towards zero: still a lower bound.
+__device__ __forceinline__ uint16_t lb_pack(float lb) { return (uint16_t)(__float_as_uint(lb) >> 16); }
+__device__ __forceinline__ float lb_unpack(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
+
+__device__ __forceinline__ float query_slack(float4 qp, float scale) {
+  return fmaxf(scale, fmaxf(fabsf(qp.x), fmaxf(fabsf(qp.y), fabsf(qp.z)))) * SLACK_REL;
+}
+
+// Evaluates queued pairs [0, m), one per lane, then moves pairs [m, qn) to the front (cmp_flush's
+// rule: the (d^2, id) pair whose key survived leaves its record).
+__device__ __forceinline__ void queue_flush(QueueWave &W, const TriRec *__restrict__ tr, int lane, int m, int qn) {
+  if (lane < m) {
+    const int32_t e = W.qe[lane];
+    const int o = W.qo[lane];
+    const float4 po = W.qp[o];
+    const TriRec *tk = tr + e;
+    const float4 p0 = tk->p0, p1 = tk->p1, p2 = tk->p2, pl = tk->pl, e0 = tk->e0, e1 = tk->e1, e2 = tk->e2;
+    float3 cp;
+    const float d = tri_closest(p0, p1, p2, pl, e0, e1, e2, f3(po.x, po.y, po.z), cp);
+    const int32_t id = trirec_id(pl);
+    const unsigned long long k = cmp_key(d, id);
+    const bool ok = id != __float_as_int(po.w) && !isnan(d);
+    if (ok) atomicMin(&W.key[o], k);
+    __builtin_amdgcn_wave_barrier();
+    if (ok && W.key[o] == k) W.slot[o] = e;
+  }
+  __builtin_amdgcn_wave_barrier();
+  const int rest = qn - m;
+  int32_t e = 0;
+  uint8_t o = 0;
+  if (lane < rest) { e = W.qe[m + lane]; o = W.qo[m + lane]; }
+  __builtin_amdgcn_wave_barrier();
+  if (lane < rest) { W.qe[lane] = e; W.qo[lane] = o; }
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ void closest_queue_body(QueueWave &W, const BNode *__restrict__ nodes,
+                                                   const TriRec *__restrict__ tr, const ScreenRec *__restrict__ scr,
+                                                   const LeafBound *__restrict__ lbnd, const float *__restrict__ q,
+                                                   const uint32_t *__restrict__ order, int64_t n, int64_t wave, int lg,
+                                                   float best_init, float scale, int exclude_self,
+                                                   int32_t *__restrict__ out_idx, float *__restrict__ out_cp,
+                                                   float *__restrict__ out_dist, float *__restrict__ out_d2,
+                                                   int32_t root) {
+  const int lane = lane_id();
+  const int Q = WAVE >> lg;
+  const int64_t t = wave * Q + lane;
+  const bool inrange = lane < Q && t < n;
+  int64_t qi = 0;
+  float3 p = f3(0, 0, 0);
+  bool active = inrange;
+  if (inrange) {
+    qi = order ? (int64_t)order[t] : t;
+    p = load_q(q, qi);
+    active = !(isnan(p.x) || isnan(p.y) || isnan(p.z));
+  }
+  if (lane < Q) {
+    W.qp[lane] = make_float4(p.x, p.y, p.z, __int_as_float(exclude_self ? (int32_t)qi : -1));
+    W.key[lane] = cmp_key(active ? best_init : 0.0f, 0x7fffffff);
+  }
+  const uint64_t amask = ballot(active && best_init >= 0.0f);
+  int sp = 0, ln = __popcll(amask), qn = 0;  // entries on the stack, in the leaf list, queued pairs
+  uint64_t todo = amask;                     // queries whose walk has not begun
+  // Each query's nearest leaf (a greedy descent) is evaluated first, so the walk starts with a bound:
+  // without one it would open 64 paths of every level below the sixth.
+  if ((amask >> lane) & 1) {
+    const float sl = query_slack(make_float4(p.x, p.y, p.z, 0.0f), scale);
+    int32_t f, cnt;
+    seed_leaf(nodes, root, f3(p.x - sl, p.y - sl, p.z - sl), f3(p.x + sl, p.y + sl, p.z + sl), f, cnt);
+    const int pos = __popcll(amask & lanemask_lt());
+    W.leaf[pos] = f;
+    W.llb[pos] = 0;
+    W.lcnt[pos] = (uint8_t)cnt;
+    W.lown[pos] = (uint8_t)lane;
+  }
+  bool seed = ln > 0;
+  __builtin_amdgcn_wave_barrier();
+  while (true) {
+    if (!seed && sp < WAVE && todo != 0) {
+      // begin further queries' walks while the steps would not be full
+      const int rank = __popcll(todo & lanemask_lt());
+      const bool take = ((todo >> lane) & 1) && sp + rank < WAVE;
+      if (take) {
+        W.ref[sp + rank] = root;
+        W.lb[sp + rank] = 0;
+        W.own[sp + rank] = (uint8_t)lane;
+      }
+      const uint64_t tm = ballot(take);
+      todo &= ~tm;
+      sp += __popcll(tm);
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (seed || ln >= WAVE || (sp == 0 && ln > 0)) {
+      // screen up to 64 leaves, one per lane
+      const int k = ln < WAVE ? ln : WAVE;
+      ln -= k;
+      bool act = lane < k;
+      int32_t f = 0;
+      int cnt = 0, o = 0;
+      float4 qp = make_float4(0, 0, 0, 0);
+      float sl = 0, rej2 = 0;
+      if (act) {
+        const int e = ln + lane;
+        f = W.leaf[e];
+        cnt = W.lcnt[e];
+        o = W.lown[e];
+        qp = W.qp[o];
+        const float best = cmp_key_d(W.key[o]);
+        sl = query_slack(qp, scale);
+        rej2 = rej_sq(best, sl);
+        act = lb_unpack(W.llb[e]) <= best;
+      }
+      if (act && lbnd) {
+        const LeafBound L = lbnd[f];
+        const float dx = qp.x - L.a.x, dy = qp.y - L.a.y, dz = qp.z - L.a.z;
+        const float dc2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+        const float sd = fmaf(dx, L.b.x, fmaf(dy, L.b.y, dz * L.b.z));
+        act = !(leaf_lb2(dc2, sd, L.b.w, L.a.w, sl) > rej2);
+      }
+      if (!act) cnt = 0;
+      for (int j = 0; ballot(j < cnt) != 0; ++j) {
+        bool need = false;
+        if (j < cnt) {
+          const ScreenRec sk = scr[f + j];
+          const float dx = qp.x - sk.c.x, dy = qp.y - sk.c.y, dz = qp.z - sk.c.z;
+          const float dc2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+          const float sd = fmaf(dx, sk.n.x, fmaf(dy, sk.n.y, dz * sk.n.z));
+          need = !(tri_lb2(dc2, sd, sk.c.w, sl) > rej2);
+        }
+        const uint64_t nb = ballot(need);
+        if (nb == 0) continue;
+        if (need) {
+          const int pos = qn + __popcll(nb & lanemask_lt());
+          W.qe[pos] = f + j;
+          W.qo[pos] = (uint8_t)o;
+        }
+        qn += __popcll(nb);
+        if (qn >= WAVE) {
+          __builtin_amdgcn_wave_barrier();
+          queue_flush(W, tr, lane, WAVE, qn);
+          qn -= WAVE;
+          rej2 = rej_sq(cmp_key_d(W.key[o]), sl);
+        }
+      }
+      if (qn > 0 && (seed || lg >= WQ_FLUSH_LG)) {
+        __builtin_amdgcn_wave_barrier();
+        queue_flush(W, tr, lane, qn, qn);
+        qn = 0;
+      }
+      seed = false;
+    } else if (sp > 0) {
+      // test the children of up to 64 nodes, one per lane
+      const int room = (WQ_STACK - WAVE - sp) >> 3;
+      int k = sp < WAVE ? sp : WAVE;
+      k = k < room ? k : (room > 1 ? room : 1);
+      bool act = lane < k;
+      int o = 0;
+      float best = 0, la = 0, lb = 0;
+      int32_t ra = 0, rb = 0, ca = 0, cb = 0;
+      if (act) {
+        const int e = sp - 1 - lane;
+        o = W.own[e];
+        best = cmp_key_d(W.key[o]);
+        act = lb_unpack(W.lb[e]) <= best;
+        if (act) {
+          const BNode nd = nodes[W.ref[e]];
+          const float4 qp = W.qp[o];
+          const float sl = query_slack(qp, scale);
+          const float3 qlo = f3(qp.x - sl, qp.y - sl, qp.z - sl), qhi = f3(qp.x + sl, qp.y + sl, qp.z + sl);
+          la = box_lb(qlo, qhi, nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y);
+          lb = box_lb(qlo, qhi, nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w);
+          ra = nd.d.x, rb = nd.d.y, ca = nd.d.z, cb = nd.d.w;
+          if (lb < la) {
+            const float tl = la; la = lb; lb = tl;
+            const int32_t tr_ = ra; ra = rb; rb = tr_;
+            const int32_t tc = ca; ca = cb; cb = tc;
+          }
+        }
+      }
+      sp -= k;
+      __builtin_amdgcn_wave_barrier();
+      // b is the farther child: pushed first, so the nearer ones are popped next
+      const bool in_a = act && la <= best, in_b = act && lb <= best;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const bool in = c == 0 ? in_b : in_a;
+        const int32_t r = c == 0 ? rb : ra;
+        const int32_t cnt = c == 0 ? cb : ca;
+        const float l = c == 0 ? lb : la;
+        const uint64_t mi = ballot(in && r >= 0), ml = ballot(in && r < 0 && cnt > 0);
+        if (in && r >= 0) {
+          const int pos = sp + __popcll(mi & lanemask_lt());
+          if (pos < WQ_STACK) {  // always, in trees of at most 63 levels
+            W.ref[pos] = r;
+            W.lb[pos] = lb_pack(l);
+            W.own[pos] = (uint8_t)o;
+          }
+        }
+        if (in && r < 0 && cnt > 0) {
+          const int pos = ln + __popcll(ml & lanemask_lt());
+          W.leaf[pos] = ~r;
+          W.llb[pos] = lb_pack(l);
+          W.lcnt[pos] = (uint8_t)cnt;
+          W.lown[pos] = (uint8_t)o;
+        }
+        sp += __popcll(mi);
+        if (sp > WQ_STACK) sp = WQ_STACK;
+        ln += __popcll(ml);
+      }
+    } else if (qn > 0) {
+      queue_flush(W, tr, lane, qn, qn);
+      qn = 0;
+    } else {
+      break;
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (!inrange) return;
+  const unsigned long long key = W.key[lane];
+  const int32_t bidx = (int32_t)(uint32_t)(key & 0xffffffffull);
+  const float own = cmp_key_d(key);
+  const bool hit = active && bidx != 0x7fffffff;
+  out_idx[qi] = hit ? bidx : -1;
+  if (out_cp) {
+    float3 c = f3(0, 0, 0);  // the winner's arithmetic again: one record per query instead of 16 bytes of LDS
+    if (hit) {
+      const TriRec *tk = tr + W.slot[lane];
+      tri_closest(tk->p0, tk->p1, tk->p2, tk->pl, tk->e0, tk->e1, tk->e2, p, c);
+    }
+    out_cp[3 * qi] = hit ? c.x : 0.0f;
+    out_cp[3 * qi + 1] = hit ? c.y : 0.0f;
+    out_cp[3 * qi + 2] = hit ? c.z : 0.0f;
+  }
+  if (out_dist) out_dist[qi] = hit ? sqrtf(own) : -1.0f;
+  if (out_d2) out_d2[qi] = hit ? own : -1.0f;
+}
+
+__global__ void __launch_bounds__(WAVE) k_closest_queue(const BNode *__restrict__ nodes, const TriRec *__restrict__ tr,
+                                                        const ScreenRec *__restrict__ scr,
+                                                        const LeafBound *__restrict__ lbnd,
+                                                        const float *__restrict__ q, const uint32_t *__restrict__ order,
+                                                        int64_t n, int lg, uint32_t nb_real, float best_init,
+                                                        float scale, int exclude_self, int32_t *__restrict__ out_idx,
+                                                        float *__restrict__ out_cp, float *__restrict__ out_dist,
+                                                        float *__restrict__ out_d2) {
+  __shared__ QueueWave s_w;
+  const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
+  if (lb_blk >= nb_real) return;
+  closest_queue_body(s_w, nodes, tr, scr, lbnd, q, order, n, (int64_t)lb_blk, lg, best_init, scale, exclude_self,
+                     out_idx, out_cp, out_dist, out_d2, 0);
+}
+
+// Many batches in one launch; the waves of a segment take 64 >> lanes_log2 queries each.
+__global__ void __launch_bounds__(WAVE) k_closest_queue_multi(const SegDesc *__restrict__ seg, int nseg,
+                                                              uint64_t total_waves, uint32_t nb_real) {
+  __shared__ QueueWave s_w;
+  const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
+  if (lb_blk >= nb_real || (uint64_t)lb_blk >= total_waves) return;
+  const int si = uni(find_segment(seg, nseg, (int64_t)lb_blk));
+  const SegDesc &d = seg[si];
+  closest_queue_body(s_w, readonly_ptr<BNode>(d.nodes), readonly_ptr<TriRec>(d.elems),
+                     readonly_ptr<ScreenRec>(d.screen), readonly_ptr<LeafBound>(d.lbounds), readonly_ptr<float>(d.q),
+                     readonly_ptr<uint32_t>(d.order), d.n, (int64_t)lb_blk - (int64_t)d.wave_begin, d.lanes_log2,
+                     d.best_init, d.scale, d.exclude_self, d.idx, d.cp, d.dist, d.d2, d.root);
+}
+
+//--------------------------------------------------------------------------------------------------
 // k nearest (sorted list of K (d^2, id) pairs per lane in registers)
 //--------------------------------------------------------------------------------------------------
 template <int STACK, bool POINTS, int K>
@@ -967,7 +1278,7 @@ __global__ void __launch_bounds__(Q_BLOCK) k_knn_lane_multi(const SegDesc *__res
 }
 
 //--------------------------------------------------------------------------------------------------
-// Sparse batches on a large tree, G lanes per query
+// Sparse batches on a large tree, G lanes per query (k-NN, and closest points of point BVHs)
 //
 // A lane walk costs its query's whole search: a query far inside a closed surface meets nearly
 // every leaf, and a launch of a few thousand such queries lasts as long as its slowest one. Here G
@@ -1034,7 +1345,7 @@ __device__ __forceinline__ int32_t group_route(const BNode *__restrict__ nodes, 
   return -1;
 }
 
-template <int STACK, bool POINTS>
+template <int STACK>
 __device__ __forceinline__ void closest_group_body(int32_t *__restrict__ s_ref, float *__restrict__ s_lb,
                                                    const BNode *__restrict__ nodes, const void *__restrict__ elems,
                                                    const float *__restrict__ q, int64_t qi, bool live, int lg,
@@ -1052,23 +1363,13 @@ __device__ __forceinline__ void closest_group_body(int32_t *__restrict__ s_ref, 
   int32_t bidx = 0x7fffffff;
   float3 bcp = f3(0, 0, 0);
   const int32_t self = exclude_self ? (int32_t)qi : -1;
-  const TriRec *__restrict__ tr = (const TriRec *)elems;
   const PointRec *__restrict__ pr = (const PointRec *)elems;
   auto eval = [&](int32_t f, int32_t cnt) {
     for (int32_t k = f; k < f + cnt; ++k) {
-      float d;
-      float3 cp;
-      int32_t id;
-      if (POINTS) {
-        float4 e = pr[k].p;
-        id = __float_as_int(e.w);
-        cp = f3(e.x, e.y, e.z);
-        d = sqn3(sub3(cp, p));
-      } else {
-        const TriRec *t = tr + k;
-        id = trirec_id(t->pl);
-        d = tri_closest(t->p0, t->p1, t->p2, t->pl, t->e0, t->e1, t->e2, p, cp);
-      }
+      const float4 e = pr[k].p;
+      const int32_t id = __float_as_int(e.w);
+      const float3 cp = f3(e.x, e.y, e.z);
+      const float d = sqn3(sub3(cp, p));
       if (id != self && better(d, id, best, bidx)) {
         best = d;
         bidx = id;
@@ -1268,7 +1569,7 @@ __device__ __forceinline__ void knn_group_body(int32_t *__restrict__ s_ref, floa
 // n * G within GRP_LANES lanes (about four waves per SIMD), as log2.
 constexpr int64_t GRP_LANES = (int64_t)1 << 18;
 
-template <int STACK, bool POINTS>
+template <int STACK>
 __global__ void __launch_bounds__(Q_BLOCK, STACK <= 32 ? 5 : 1) k_closest_group(const BNode *__restrict__ nodes,
                                                            const void *__restrict__ elems, const float *__restrict__ q,
                                                            const uint32_t *__restrict__ order, int64_t n, int lg,
@@ -1283,7 +1584,7 @@ __global__ void __launch_bounds__(Q_BLOCK, STACK <= 32 ? 5 : 1) k_closest_group(
   const int64_t s = ((int64_t)lb_blk * Q_BLOCK + threadIdx.x) >> lg;
   const bool live = s < n;
   const int64_t qi = live ? (order ? (int64_t)order[s] : s) : 0;
-  closest_group_body<STACK, POINTS>(s_ref, s_lb, nodes, elems, q, qi, live, lg, best_init, scale, exclude_self,
+  closest_group_body<STACK>(s_ref, s_lb, nodes, elems, q, qi, live, lg, best_init, scale, exclude_self,
                                     out_idx, out_cp, out_dist, out_d2, 0);
 }
 
@@ -1306,24 +1607,6 @@ __global__ void __launch_bounds__(Q_BLOCK) k_knn_group(const BNode *__restrict__
 
 // Server form: one 64-lane block per wave of a segment; a segment of n queries at 2^lg lanes each
 // spans ceil(n 2^lg / 64) waves (SegDesc::lanes_log2).
-template <int STACK, bool POINTS>
-__global__ void __launch_bounds__(Q_BLOCK, STACK <= 32 ? 5 : 1) k_closest_group_multi(const SegDesc *__restrict__ seg, int nseg,
-                                                                 uint64_t total_waves, uint32_t nb_real) {
-  __shared__ int32_t s_ref[lane_lds_entries<STACK, CL_REG>() * Q_BLOCK];
-  __shared__ float s_lb[CL_LB ? lane_lds_entries<STACK, CL_REG>() * Q_BLOCK : 1];
-  const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
-  if (lb_blk >= nb_real || (uint64_t)lb_blk >= total_waves) return;
-  const int si = uni(find_segment(seg, nseg, (int64_t)lb_blk));
-  const SegDesc &d = seg[si];
-  const int lg = d.lanes_log2;
-  const int64_t s = (((int64_t)lb_blk - (int64_t)d.wave_begin) * Q_BLOCK + threadIdx.x) >> lg;
-  const bool live = s < d.n;
-  const int64_t qi = live ? (d.order ? (int64_t)d.order[s] : s) : 0;
-  closest_group_body<STACK, POINTS>(s_ref, s_lb, readonly_ptr<BNode>(d.nodes), readonly_ptr<float>(d.elems),
-                                    readonly_ptr<float>(d.q), qi, live, lg, d.best_init,
-                                    d.scale, d.exclude_self, d.idx, d.cp, d.dist, d.d2, d.root);
-}
-
 template <int STACK, bool POINTS, int K>
 __global__ void __launch_bounds__(Q_BLOCK) k_knn_group_multi(const SegDesc *__restrict__ seg, int nseg,
                                                              uint64_t total_waves, uint32_t nb_real) {
@@ -2395,6 +2678,32 @@ bool use_wave_traversal(const Bvh &b, int64_t n) {
   return n >= ORDER_MIN_QUERIES && n >= b.num_leaves / 8;
 }
 
+// Closest triangles: the work-queue kernel or the compacted wave walk. One walk for 64 queries needs
+// the fewest loads where its queries are close together, from about 1.25 queries per triangle on;
+// below that, and below 3 2^18 queries on any mesh (where the longest walk bounds the launch), the
+// queue is faster. Torus of 1,048,576 triangles, queries uniform in the box, queue against wave:
+// 500,000 2.1 / 4.1 ms, 1,000,000 3.7 / 4.7 ms, 10,000,000 21.8 / 13.2 ms; of 100,000 triangles:
+// 500,000 0.84 / 1.31 ms, 1,000,000 1.45 / 1.54 ms. THG_TRAVERSAL=queue or =wave forces one; trees
+// deeper than 63 levels take one query per lane.
+bool use_queue(int64_t n, int64_t triangles, int max_depth) {
+  static const char *env = getenv("THG_TRAVERSAL");
+  if (max_depth + 1 > W_STACK || (env && std::string(env) == "lane")) return false;
+  if (env && std::string(env) == "wave") return n < ORDER_MIN_QUERIES;
+  if (env && std::string(env) == "queue") return true;
+  return n <= std::max<int64_t>(triangles + triangles / 4, (int64_t)3 << 18);
+}
+bool use_queue_traversal(const Bvh &b, int64_t n) { return !b.points && use_queue(n, b.n, b.max_depth); }
+
+// log2 of the lanes per query of the work-queue kernel (64 >> lg queries per wave) for n queries:
+// about 6,400 waves (256 CUs hold 4,096) until a wave has 16 queries, 32 from 2^19 queries on. Few
+// queries per wave shorten the longest wave, many share its steps better (queries near the surface,
+// 100,000 of them: 220, 199, 242, 346 us at 32, 16, 8, 4 per wave; in the box 1,209, 786, 670, 640).
+int queue_lanes_log2(int64_t n) {
+  int lg = n < ((int64_t)1 << 19) ? 2 : 1;
+  while (lg < 6 && n * ((int64_t)2 << lg) <= 6400 * WAVE) ++lg;
+  return lg;
+}
+
 // Lanes per query and per-element prefilter of the wave kernel (THG_WAVE_G, THG_PREFILTER override).
 struct WaveConfig {
   int g;
@@ -2428,6 +2737,17 @@ void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, 
   uint32_t nb = ceil_div(n, Q_BLOCK);
   uint32_t grid = round_up8(nb);
   float best = bound_to_best(dist_bound);
+  if (use_queue_traversal(b, n)) {
+    const int lg = queue_lanes_log2(n);
+    const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE);
+    KernelTimer kt(ws.timer_ctx(b.ctx), s, "closest");
+    hipLaunchKernelGGL(k_closest_queue, dim3(round_up8(qnb)), dim3(WAVE), 0, s, b.nodes.as<BNode>(),
+                       b.elems.as<TriRec>(), b.screen.as<ScreenRec>(), b.lbounds.as<LeafBound>(), q, ws.order, n, lg,
+                       qnb, best, b.scale, exclude_self, idx, cp, dist, d2);
+    launch_check("k_closest_queue");
+    kt.stop();
+    return;
+  }
   if (use_wave_traversal(b, n)) {
     const WaveConfig wc = wave_config(b);
     uint32_t wnb = ceil_div(n, (uint64_t)W_WAVES * (WAVE / wc.g));
@@ -2482,15 +2802,13 @@ void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, 
     kt.stop();
     return;
   }
-  if (const int lg = group_lanes_log2(n, b.max_depth)) {
+  if (const int lg = b.points ? group_lanes_log2(n, b.max_depth) : 0) {
     const uint32_t gnb = (uint32_t)ceil_div(n << lg, Q_BLOCK);
-    const bool deep = b.max_depth + 1 > 32;
     KernelTimer kt(ws.timer_ctx(b.ctx), s, "closest");
-#define THG_CG(S, P)                                                                                                  \
-  hipLaunchKernelGGL((k_closest_group<S, P>), dim3(round_up8(gnb)), dim3(Q_BLOCK), 0, s, b.nodes.as<BNode>(), b.elems.p, \
+#define THG_CG(S)                                                                                                    \
+  hipLaunchKernelGGL((k_closest_group<S>), dim3(round_up8(gnb)), dim3(Q_BLOCK), 0, s, b.nodes.as<BNode>(), b.elems.p, \
                      q, ws.order, n, lg, gnb, best, b.scale, exclude_self, idx, cp, dist, d2)
-    if (b.points) { if (deep) THG_CG(64, true); else THG_CG(32, true); }
-    else { if (deep) THG_CG(64, false); else THG_CG(32, false); }
+    if (b.max_depth + 1 > 32) THG_CG(64); else THG_CG(32);
 #undef THG_CG
     launch_check("k_closest_group");
     kt.stop();
@@ -2611,17 +2929,11 @@ void launch_knn_lane_multi(const SegDesc *seg_dev, int nseg, uint64_t total_wave
   launch_check("k_knn_lane_multi");
 }
 
-void launch_closest_group_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, bool points, int stack,
-                                hipStream_t s) {
+void launch_closest_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s) {
   if (nseg <= 0 || total_waves == 0) return;
   const uint32_t nb = (uint32_t)total_waves;
-  const uint32_t grid = round_up8(nb);
-#define THG_CGM(S, P) hipLaunchKernelGGL((k_closest_group_multi<S, P>), dim3(grid), dim3(Q_BLOCK), 0, s, seg_dev, nseg, \
-                                         total_waves, nb)
-  if (points) { if (stack <= 32) THG_CGM(32, true); else THG_CGM(64, true); }
-  else { if (stack <= 32) THG_CGM(32, false); else THG_CGM(64, false); }
-#undef THG_CGM
-  launch_check("k_closest_group_multi");
+  hipLaunchKernelGGL(k_closest_queue_multi, dim3(round_up8(nb)), dim3(WAVE), 0, s, seg_dev, nseg, total_waves, nb);
+  launch_check("k_closest_queue_multi");
 }
 
 void launch_knn_group_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int k, bool points, int stack,

@@ -25,6 +25,7 @@ struct SegDesc {
   const float *q2;       // ray directions
   const uint32_t *order; // optional spatial order of the batch
   const void *screen;    // ScreenRec records (mesh closest-point segments)
+  const void *lbounds;   // LeafBound records (mesh closest-point segments; optional)
   int32_t *idx;
   float *cp;             // closest points (closest) / normals (rays)
   float *dist;           // distances (closest, k-NN) / hit times (rays)
@@ -39,7 +40,7 @@ struct SegDesc {
   int32_t points;
   int32_t root;          // node the traversal starts from
   int32_t nelem;         // elements of the segment's tree (k-NN seed window)
-  int32_t lanes_log2;    // lanes per query (log2) of the grouped sparse kernels
+  int32_t lanes_log2;    // lanes per query (log2) of the work-queue and grouped kernels
   int32_t child_order;   // visiting order of the compacted closest-point kernel (0: majority)
 };
 
@@ -114,10 +115,13 @@ void launch_knn_lane_multi(const SegDesc *seg_dev, int nseg, uint64_t total_wave
                            hipStream_t s);
 // 2^lanes_log2 lanes per query over a segment table (SegDesc::lanes_log2 per segment, each
 // segment spanning ceil(n 2^lanes_log2 / 64) waves); stack >= the deepest tree plus 1, at most 64.
-void launch_closest_group_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, bool points, int stack,
-                                hipStream_t s);
 void launch_knn_group_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int k, bool points, int stack,
                             hipStream_t s);
+// Closest triangles by work queue: each segment spans ceil(n 2^lanes_log2 / 64) waves.
+void launch_closest_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s);
+bool use_queue(int64_t n, int64_t triangles, int max_depth);
+bool use_queue_traversal(const Bvh &b, int64_t n);
+int queue_lanes_log2(int64_t n);
 // log2 of the lanes per query the sparse kernels give a batch of n queries on a tree of this depth.
 int group_lanes_log2(int64_t n, int depth);
 bool use_wave_traversal(const Bvh &b, int64_t n);

@@ -146,19 +146,22 @@ static void worker_loop(Server *S, int wi) {
         for (int64_t id : batch) {
           SrvRequest &r = S->reqs[id];
           int kk = r.r.type == THG_REQ_KNN ? (r.r.k <= 4 ? 4 : r.r.k <= 8 ? 8 : r.r.k <= 16 ? 16 : 32) : 0;
-          int lane = r.r.type != THG_REQ_RAY && !use_wave_traversal(*r.bvh, r.r.n) ? 1 : 0;
+          // closest points: work queue (2), k-NN and the rest: wave-cooperative (0) or per query (1)
+          int lane = r.r.type == THG_REQ_CLOSEST && use_queue_traversal(*r.bvh, r.r.n) ? 2
+                     : r.r.type != THG_REQ_RAY && !use_wave_traversal(*r.bvh, r.r.n)  ? 1
+                                                                                      : 0;
           groups[{r.r.type, lane, kk}].push_back(&r);
         }
       }
       int region = 0;
       for (auto &kv : groups) {
         const int type = std::get<0>(kv.first);
-        const bool lane = std::get<1>(kv.first) != 0;
+        const bool lane = std::get<1>(kv.first) == 1, queue = std::get<1>(kv.first) == 2;
         int depth1 = 0;
         for (SrvRequest *r : kv.second) depth1 = std::max(depth1, r->bvh->max_depth + 1);
         // sparse requests share each query among several lanes (group kernels)
         bool grouped = false;
-        if (lane)
+        if (lane && type == THG_REQ_KNN)
           for (SrvRequest *r : kv.second)
             grouped = grouped || group_lanes_log2(r->r.n, r->bvh->max_depth) > 0;
         const int stack = std::max(32, depth1);
@@ -173,6 +176,8 @@ static void worker_loop(Server *S, int wi) {
           ++region;
           uint64_t waves = 0;
           int nseg = 0;
+          int64_t total = 0;
+          for (SrvRequest *r : list) total += r->r.n;
           for (SrvRequest *r : list) {
             const thg_request &q = r->r;
             const Bvh &b = *r->bvh;
@@ -182,6 +187,7 @@ static void worker_loop(Server *S, int wi) {
             d.rays = b.rays.p;
             d.qnodes = b.qnodes.p;
             d.screen = b.screen.p;
+            d.lbounds = b.lbounds.p;
             d.q = q.q;
             d.q2 = q.dirs;
             d.idx = q.idx;
@@ -206,14 +212,14 @@ static void worker_loop(Server *S, int wi) {
               else order_queries(b, q.q, q.n, *scratch.back(), s);
               d.order = scratch.back()->order;
             }
-            d.lanes_log2 = grouped ? group_lanes_log2(q.n, b.max_depth) : 0;
+            d.lanes_log2 = queue ? queue_lanes_log2(total) : grouped ? group_lanes_log2(q.n, b.max_depth) : 0;
             d.wave_begin = waves;
             waves += (uint64_t)(((q.n << d.lanes_log2) + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES);
             hd[nseg++] = d;
           }
           THG_HIP(hipMemcpyAsync(dd, hd, sizeof(SegDesc) * nseg, hipMemcpyHostToDevice, s));
           if (type == THG_REQ_CLOSEST) {
-            if (grouped) launch_closest_group_multi(dd, nseg, waves, false, stack, s);
+            if (queue) launch_closest_queue_multi(dd, nseg, waves, s);
             else if (lane) launch_closest_lane_multi(dd, nseg, waves, false, stack, s);
             else launch_closest_multi(dd, nseg, waves, false, s, /*concurrent=*/true);
           } else if (type == THG_REQ_KNN) {
