@@ -1,0 +1,90 @@
+"""The work-queue k-NN kernel (and closest points of point BVHs) against the wave walk and the oracle.
+
+A batch of more than max(4 queries per triangle, 2^18) on a mesh, or max(1 per 2 points, 2^17) on
+points, takes the wave walk up to k = 16; smaller ones, and every k above 16, take the queue. Both
+must give the canonical lists. Sizes are the edges of its waves (1 to 32 queries each, by k), k the
+edges of its list widths, and trees of fewer elements than k leave slots empty.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _equal(a, b, label):
+    for x, y in zip(a, b):
+        assert np.array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32)), label
+
+
+@pytest.fixture(scope="module")
+def mesh_case():
+    import thea_amd
+    from thea_amd import workloads as W
+    v, t = W.torus(40, 20)
+    g = np.random.default_rng(11)
+    lo, hi = W.inflated_box(v, 1.2)
+    q = g.uniform(lo, hi, size=((1 << 18) + 1, 3)).astype(np.float32)
+    q[3] = np.nan
+    return thea_amd.MeshBvh(thea_amd.Mesh(v, t)), q
+
+
+@pytest.mark.parametrize("k", [1, 2, 5, 8, 9, 16])
+def test_mesh_lists_equal_wave_walk(mesh_case, k):
+    b, q = mesh_case
+    ref = b.kClosestElements(q, k, want_d2=True)
+    refb = b.kClosestElements(q, k, dist_bound=0.15, want_d2=True)
+    for n in (1, 7, 33, 4_097, 12_801, 51_201, 1 << 18):
+        _equal(b.kClosestElements(q[:n], k, want_d2=True), [x[:n] for x in ref], f"k={k} n={n}")
+    _equal(b.kClosestElements(q[:900], k, dist_bound=0.15, want_d2=True), [x[:900] for x in refb], f"k={k} bound")
+
+
+@pytest.mark.parametrize("k", [1, 4, 16, 17, 32])
+@pytest.mark.parametrize("n", [1, 130, 9_000])
+def test_mesh_lists_equal_oracle(oracle, k, n):
+    import thea_amd
+    from thea_amd import workloads as W
+    v, t = W.geodesic_sphere(3)
+    v, t = np.concatenate([v, v * np.float32(0.5)]), np.concatenate([t, t + len(v), t[:50]])  # 50 duplicates
+    g = np.random.default_rng(n)
+    q = g.uniform(-1.5, 1.5, size=(n, 3)).astype(np.float32)
+    idx, _, d2 = thea_amd.MeshBvh(thea_amd.Mesh(v, t), leaf_size=2).kClosestElements(q, k, want_d2=True)
+    m = min(n, 400)
+    ridx, rd2, _ = oracle.KdTree(v, t).knn(q[:m], k, mode=0)
+    _equal((idx[:m], d2[:m]), (ridx, rd2), f"k={k} n={n}")
+
+
+@pytest.mark.parametrize("count", [1, 2, 3, 5, 31, 70])
+@pytest.mark.parametrize("exclude", [False, True])
+def test_small_point_sets(oracle, count, exclude):
+    import thea_amd
+    g = np.random.default_rng(count)
+    p = g.normal(size=(count, 3)).astype(np.float32)
+    p[count // 2] = p[0]  # an exact duplicate
+    b = thea_amd.PointBvh(p, leaf_size=2)
+    d2all = ((p[:, None] - p[None]) ** 2)
+    d2all = d2all[..., 0] + (d2all[..., 1] + d2all[..., 2])
+    for k in (1, 3, 8, 32):
+        idx, _, d2 = b.kClosestElements(p, k, exclude_self=exclude, want_d2=True)
+        for i in range(count):
+            order = sorted((d2all[i, j], j) for j in range(count) if not (exclude and j == i))[:k]
+            want = [j for _, j in order] + [-1] * (k - len(order))
+            assert idx[i].tolist() == want, (count, k, i)
+            assert np.array_equal(d2[i][:len(order)], np.array([d for d, _ in order], np.float32))
+
+
+@pytest.mark.parametrize("leaf", [1, 4, 16])
+def test_points_equal_wave_walk(leaf):
+    import thea_amd
+    g = np.random.default_rng(leaf)
+    p = g.normal(size=(30_000, 3)).astype(np.float32)
+    p[20_000:20_100] = p[:100]
+    b = thea_amd.PointBvh(p, leaf_size=leaf)
+    q = (g.normal(size=((1 << 17) + 1, 3)) * 1.2).astype(np.float32)
+    q[:500] = p[:500]
+    q[9] = np.inf
+    ref = b.closest(q, want_d2=True)
+    refk = b.kClosestElements(q, 6, want_d2=True)
+    for n in (1, 40, 4_097, 1 << 17):
+        _equal(b.closest(q[:n], want_d2=True), [x[:n] for x in ref], f"closest n={n}")
+        _equal(b.kClosestElements(q[:n], 6, want_d2=True), [x[:n] for x in refk], f"k-NN n={n}")
+    assert (b.closest(q[:50], dist_bound=0.0)[0] == -1).all()

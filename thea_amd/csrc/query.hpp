@@ -40,7 +40,7 @@ struct SegDesc {
   int32_t points;
   int32_t root;          // node the traversal starts from
   int32_t nelem;         // elements of the segment's tree (k-NN seed window)
-  int32_t lanes_log2;    // lanes per query (log2) of the work-queue and grouped kernels
+  int32_t lanes_log2;    // lanes per query (log2) of the work-queue kernels
   int32_t child_order;   // visiting order of the compacted closest-point kernel (0: majority)
 };
 
@@ -107,23 +107,22 @@ void scan_excl_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *tmp, 
 // block_waves: waves per workgroup (1, 2, 4, 8); spill_build: the 8-resident-wave build.
 void launch_closest_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, bool points, hipStream_t s,
                           bool concurrent = false, int block_waves = 4, bool spill_build = true);
+// k <= 16 (longer lists take the work queue).
 void launch_knn_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int k, bool points, hipStream_t s);
 // One query per lane over a segment table (stack >= the deepest tree of the segments, at most 64).
 void launch_closest_lane_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, bool points, int stack,
                                hipStream_t s);
 void launch_knn_lane_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int k, bool points, int stack,
                            hipStream_t s);
-// 2^lanes_log2 lanes per query over a segment table (SegDesc::lanes_log2 per segment, each
-// segment spanning ceil(n 2^lanes_log2 / 64) waves); stack >= the deepest tree plus 1, at most 64.
-void launch_knn_group_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int k, bool points, int stack,
-                            hipStream_t s);
 // Closest triangles by work queue: each segment spans ceil(n 2^lanes_log2 / 64) waves.
 void launch_closest_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s);
 bool use_queue(int64_t n, int64_t triangles, int max_depth);
 bool use_queue_traversal(const Bvh &b, int64_t n);
 int queue_lanes_log2(int64_t n);
-// log2 of the lanes per query the sparse kernels give a batch of n queries on a tree of this depth.
-int group_lanes_log2(int64_t n, int depth);
+// k nearest by work queue on mesh BVHs, segments as above.
+void launch_knn_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s);
+bool use_knn_queue(const Bvh &b, int64_t n, int k);
+int knn_queue_lanes_log2(int64_t n, int k, bool points);
 bool use_wave_traversal(const Bvh &b, int64_t n);
 // stack: the deepest tree among the segments plus one (32 or 64 entries). q_stack > 0 traverses
 // the segments' QNode4 trees instead; it must be at least q4_stack() of every segment's BVH.

@@ -138,18 +138,18 @@ static void worker_loop(Server *S, int wi) {
     std::string err;
     std::vector<std::unique_ptr<QueryScratch>> scratch;
     try {
-      // group by type, traversal (wave-cooperative for dense requests, one query per lane for
-      // sparse ones, as the single-call entry points choose) and, for k-NN, k
+      // group by type, traversal (as the single-call entry points choose) and, for k-NN, k
       std::map<std::tuple<int, int, int>, std::vector<SrvRequest *>> groups;
       {
         std::lock_guard<std::mutex> g(S->mu);
         for (int64_t id : batch) {
           SrvRequest &r = S->reqs[id];
           int kk = r.r.type == THG_REQ_KNN ? (r.r.k <= 4 ? 4 : r.r.k <= 8 ? 8 : r.r.k <= 16 ? 16 : 32) : 0;
-          // closest points: work queue (2), k-NN and the rest: wave-cooperative (0) or per query (1)
-          int lane = r.r.type == THG_REQ_CLOSEST && use_queue_traversal(*r.bvh, r.r.n) ? 2
-                     : r.r.type != THG_REQ_RAY && !use_wave_traversal(*r.bvh, r.r.n)  ? 1
-                                                                                      : 0;
+          // work queue (2), wave-cooperative (0) or one query per lane (1), as single calls choose
+          const bool queue = r.r.type == THG_REQ_CLOSEST ? use_queue_traversal(*r.bvh, r.r.n)
+                             : r.r.type == THG_REQ_KNN   ? use_knn_queue(*r.bvh, r.r.n, r.r.k)
+                                                         : false;
+          int lane = queue ? 2 : r.r.type != THG_REQ_RAY && !use_wave_traversal(*r.bvh, r.r.n) ? 1 : 0;
           groups[{r.r.type, lane, kk}].push_back(&r);
         }
       }
@@ -159,11 +159,6 @@ static void worker_loop(Server *S, int wi) {
         const bool lane = std::get<1>(kv.first) == 1, queue = std::get<1>(kv.first) == 2;
         int depth1 = 0;
         for (SrvRequest *r : kv.second) depth1 = std::max(depth1, r->bvh->max_depth + 1);
-        // sparse requests share each query among several lanes (group kernels)
-        bool grouped = false;
-        if (lane && type == THG_REQ_KNN)
-          for (SrvRequest *r : kv.second)
-            grouped = grouped || group_lanes_log2(r->r.n, r->bvh->max_depth) > 0;
         const int stack = std::max(32, depth1);
         // k-NN segments of one launch share k; split by exact k
         std::map<int, std::vector<SrvRequest *>> byk;
@@ -212,7 +207,9 @@ static void worker_loop(Server *S, int wi) {
               else order_queries(b, q.q, q.n, *scratch.back(), s);
               d.order = scratch.back()->order;
             }
-            d.lanes_log2 = queue ? queue_lanes_log2(total) : grouped ? group_lanes_log2(q.n, b.max_depth) : 0;
+            d.lanes_log2 = !queue                    ? 0
+                           : type == THG_REQ_CLOSEST ? queue_lanes_log2(total)
+                                                     : knn_queue_lanes_log2(total, kk.first, false);
             d.wave_begin = waves;
             waves += (uint64_t)(((q.n << d.lanes_log2) + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES);
             hd[nseg++] = d;
@@ -223,7 +220,7 @@ static void worker_loop(Server *S, int wi) {
             else if (lane) launch_closest_lane_multi(dd, nseg, waves, false, stack, s);
             else launch_closest_multi(dd, nseg, waves, false, s, /*concurrent=*/true);
           } else if (type == THG_REQ_KNN) {
-            if (grouped) launch_knn_group_multi(dd, nseg, waves, kk.first, false, stack, s);
+            if (queue) launch_knn_queue_multi(dd, nseg, waves, s);
             else if (lane) launch_knn_lane_multi(dd, nseg, waves, kk.first, false, stack, s);
             else launch_knn_multi(dd, nseg, waves, kk.first, false, s);
           } else {
