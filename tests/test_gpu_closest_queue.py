@@ -32,7 +32,7 @@ def torus(request):
     return b, q, b.closest(q, want_d2=True), b.closest(q, dist_bound=0.1, want_d2=True)
 
 
-@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 64, 4_095, 4_097, 6_400, 6_401, 12_801, 51_201, 102_401, 204_801,
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 64, 4_095, 4_097, 6_400, 6_401, 12_801, 51_201, 102_401, 131_072, 131_073, 204_801, 262_143, 262_144,
                                524_287, 524_288, WAVE_N - 1])
 def test_queue_equals_wave_walk(torus, n):
     b, q, ref, ref_bound = torus

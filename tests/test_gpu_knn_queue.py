@@ -33,7 +33,7 @@ def test_mesh_lists_equal_wave_walk(mesh_case, k):
     b, q = mesh_case
     ref = b.kClosestElements(q, k, want_d2=True)
     refb = b.kClosestElements(q, k, dist_bound=0.15, want_d2=True)
-    for n in (1, 7, 33, 4_097, 12_801, 51_201, 1 << 18):
+    for n in (1, 7, 33, 4_097, 12_801, 51_201, 131_073, (1 << 18) - 1, 1 << 18):
         _equal(b.kClosestElements(q[:n], k, want_d2=True), [x[:n] for x in ref], f"k={k} n={n}")
     _equal(b.kClosestElements(q[:900], k, dist_bound=0.15, want_d2=True), [x[:900] for x in refb], f"k={k} bound")
 

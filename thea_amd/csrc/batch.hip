@@ -10,8 +10,9 @@
 //      which groups the elements by mesh in input order
 //   -> Karras radix trees, each over its mesh's key range (global positions and node ids)
 //   -> one bottom-up refit, per-mesh leaf sizes, one compaction, one emit, records with local ids
-//   -> queries sorted by (mesh, Morton) the same way
-//   -> one multi-segment closest-point launch: segment m walks mesh m's tree from its root.
+//   -> queries sorted by (mesh, Morton) the same way where some mesh's kernel needs it
+//   -> multi-segment closest-point launches (work queue, wave walk): segment m walks mesh m's tree from
+//      its root.
 // Small meshes (no more elements than their leaf size) get a single-leaf root node each.
 #include <algorithm>
 #include <chrono>
@@ -49,6 +50,7 @@ struct BatchPlan {
   int32_t nsmall = 0;
   uint64_t total_waves = 0, lane_waves = 0;
   int32_t nwave_meshes = 0;
+  bool sort_queries = false;  // some mesh's queries need their spatial order
   std::vector<int4> tchunks, qchunks;
   DevBuf verts, tris, queries;
   DevBuf d_info, d_tchunks, d_qchunks, mbounds;
@@ -311,10 +313,10 @@ __global__ void k_bsegs(const MeshInfo *__restrict__ mi, int nm, const int *__re
   d.nodes = nodes;
   d.elems = recs;
   d.screen = scr;
-  d.q = q;
-  d.order = qorder + x.qoff;
-  d.idx = out_idx;
-  d.dist = out_dist;
+  d.q = qorder ? q : q + 3 * x.qoff;  // the order holds positions in the whole batch
+  d.order = qorder ? qorder + x.qoff : nullptr;
+  d.idx = qorder ? out_idx : out_idx + x.qoff;
+  d.dist = qorder ? out_dist : out_dist + x.qoff;
   d.n = x.nt > 0 ? x.nq : 0;
   d.wave_begin = x.wave_begin;
   d.best_init = INFINITY;
@@ -387,12 +389,15 @@ static void plan_pipeline(BatchPlan &P, hipStream_t s, hipEvent_t mid = nullptr)
   }
   if (mid) THG_HIP(hipEventRecord(mid, s));
   if (P.NQ > 0) {
-    // queries: reuse the key/value buffers (the element order is no longer needed after the records)
-    hipLaunchKernelGGL(k_bqkeys, dim3(ceil_div(P.NQ, BB)), dim3(BB), 0, s, P.queries.as<float>(), mi, nm, mb, P.mesh_bits,
-                       P.NQ, P.keys.as<uint32_t>());
-    launch_check("k_bqkeys");
-    const uint32_t *qorder = radix_sort_order(P.keys.as<uint32_t>(), P.vals.as<uint32_t>(), P.tk.as<uint32_t>(),
-                                              P.tv.as<uint32_t>(), P.hist.as<uint32_t>(), P.NQ, 0, 32, false, s);
+    const uint32_t *qorder = nullptr;
+    if (P.sort_queries) {
+      // reuses the key/value buffers (the element order is no longer needed after the records)
+      hipLaunchKernelGGL(k_bqkeys, dim3(ceil_div(P.NQ, BB)), dim3(BB), 0, s, P.queries.as<float>(), mi, nm, mb,
+                         P.mesh_bits, P.NQ, P.keys.as<uint32_t>());
+      launch_check("k_bqkeys");
+      qorder = radix_sort_order(P.keys.as<uint32_t>(), P.vals.as<uint32_t>(), P.tk.as<uint32_t>(), P.tv.as<uint32_t>(),
+                                P.hist.as<uint32_t>(), P.NQ, 0, 32, false, s);
+    }
     hipLaunchKernelGGL(k_bsegs, dim3(ceil_div(nm, BB)), dim3(BB), 0, s, mi, nm, mb, P.fidx.as<uint32_t>(), P.nsmall,
                        P.nodes.as<BNode>(), P.recs.as<TriRec>(), P.screen.as<ScreenRec>(), P.queries.as<float>(),
                        qorder, P.out_idx.as<int32_t>(), P.out_dist.as<float>(), P.seg.as<SegDesc>());
@@ -440,7 +445,8 @@ static double time_plan_kernel(const Bvh &b, const float *q, int64_t n, int chil
                                int reps, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
   QueryScratch ws;
   ws.timed = false;
-  order_queries(b, q, n, ws, s);
+  const bool queue = use_queue(n, b.n, 0);
+  if (!queue || n > QUEUE_UNSORTED_MAX) order_queries(b, q, n, ws, s);
   AsyncBuf oi(n * 4, s), od(n * 4, s), dseg(sizeof(SegDesc), s);
   SegDesc d{};
   d.nodes = b.nodes.p;
@@ -455,7 +461,7 @@ static double time_plan_kernel(const Bvh &b, const float *q, int64_t n, int chil
   d.scale = b.scale;
   d.nelem = (int32_t)b.n;
   d.child_order = child_order;
-  d.lanes_log2 = use_queue(n, b.n, 0) ? queue_lanes_log2(n) : 0;
+  d.lanes_log2 = queue ? queue_lanes_log2(n) : 0;
   THG_HIP(hipMemcpyAsync(dseg.p, &d, sizeof(SegDesc), hipMemcpyHostToDevice, s));
   const uint64_t waves = (uint64_t)(((n << d.lanes_log2) + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES);
   auto launch = [&] {
@@ -522,6 +528,7 @@ int thg_batch_plan_create(thg_ctx ctx, int32_t nm, const int64_t *nv, const int6
       x.nt = nt[m]; x.nq = nq[m]; x.nv = nv[m]; x.leaf = leaf;
       x.small_slot = (nt[m] >= 1 && nt[m] <= leaf) ? P->nsmall++ : -1;
       x.lane = use_queue(nq[m], nt[m], 0) ? queue_lanes_log2(queue_n) : 0;
+      P->sort_queries = P->sort_queries || !x.lane || nq[m] > QUEUE_UNSORTED_MAX;
       const uint64_t w =
           nt[m] > 0 ? (uint64_t)(((nq[m] << x.lane) + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES) : 0;
       if (x.lane) { x.wave_begin = lwaves; lwaves += w; }

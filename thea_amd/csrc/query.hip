@@ -1035,6 +1035,18 @@ __device__ __forceinline__ void queue_screen(W_ &W, int lane, const ScreenRec *_
   }
 }
 
+// Position in the batch of a lane's query. In a sorted batch below WQ_SPREAD_N queries, groups of
+// WQ_SPREAD waves deal their queries out like cards, so a cluster of hard queries falls on many waves
+// (150,000 queries in the box, torus of 1,048,576 triangles 958 -> 745 us; near the surface 230 ->
+// 238 us). From 500,000 on there are waves enough, and dealing only costs locality.
+constexpr int64_t WQ_SPREAD = 16, WQ_SPREAD_N = (int64_t)1 << 18;
+__device__ __forceinline__ int64_t queue_slot(int64_t wave, int lane, int Q, int64_t n, bool sorted) {
+  if (!sorted || n >= WQ_SPREAD_N) return wave * Q + lane;
+  const int64_t waves = (n + Q - 1) / Q, base = wave / WQ_SPREAD * WQ_SPREAD;
+  const int64_t c = waves - base < WQ_SPREAD ? waves - base : WQ_SPREAD;
+  return base * Q + lane * c + (wave - base);
+}
+
 __device__ __forceinline__ void closest_queue_body(QueueWave &W, const BNode *__restrict__ nodes,
                                                    const TriRec *__restrict__ tr, const ScreenRec *__restrict__ scr,
                                                    const LeafBound *__restrict__ lbnd, const float *__restrict__ q,
@@ -1045,7 +1057,7 @@ __device__ __forceinline__ void closest_queue_body(QueueWave &W, const BNode *__
                                                    int32_t root) {
   const int lane = lane_id();
   const int Q = WAVE >> lg;
-  const int64_t t = wave * Q + lane;
+  const int64_t t = queue_slot(wave, lane, Q, n, order != nullptr);
   const bool inrange = lane < Q && t < n;
   int64_t qi = 0;
   float3 p = f3(0, 0, 0);
@@ -1233,7 +1245,7 @@ __device__ __forceinline__ void knn_queue_body(KnnWave &W, const BNode *__restri
                                                int32_t nelem, int32_t root) {
   const int lane = lane_id();
   const int Q = WAVE >> lg;
-  const int64_t t = wave * Q + lane;
+  const int64_t t = queue_slot(wave, lane, Q, n, order != nullptr);
   const bool inrange = lane < Q && t < n;
   uint32_t qi = 0;
   float3 p = f3(0, 0, 0);
@@ -2671,11 +2683,12 @@ float bound_to_best(double dist_bound) {
 void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, int exclude_self, int32_t *idx,
                     float *cp, float *dist, float *d2, QueryScratch &ws, hipStream_t s) {
   if (n <= 0) return;
-  order_queries(b, q, n, ws, s);
+  const bool queue = b.points ? use_knn_queue(b, n, 1) : use_queue_traversal(b, n);
+  if (!queue || n > QUEUE_UNSORTED_MAX) order_queries(b, q, n, ws, s);
   uint32_t nb = ceil_div(n, Q_BLOCK);
   uint32_t grid = round_up8(nb);
   float best = bound_to_best(dist_bound);
-  if (use_queue_traversal(b, n)) {
+  if (queue && !b.points) {
     const int lg = queue_lanes_log2(n);
     const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE);
     KernelTimer kt(ws.timer_ctx(b.ctx), s, "closest");
@@ -2686,7 +2699,7 @@ void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, 
     kt.stop();
     return;
   }
-  if (b.points && use_knn_queue(b, n, 1)) {
+  if (queue) {
     const int lg = knn_queue_lanes_log2(n, 1, true);
     const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE);
     KernelTimer kt(ws.timer_ctx(b.ctx), s, "closest");
@@ -2936,11 +2949,12 @@ void knn_wave_stats(const Bvh &b, const float *q, int64_t n, int exclude_self, i
 void launch_knn(const Bvh &b, const float *q, int64_t n, int k, double dist_bound, int exclude_self, int32_t *idx,
                 float *dist, float *d2, QueryScratch &ws, hipStream_t s) {
   if (n <= 0) return;
-  order_queries(b, q, n, ws, s);
+  const bool queue = use_knn_queue(b, n, k);
+  if (!queue || n > QUEUE_UNSORTED_MAX) order_queries(b, q, n, ws, s);
   uint32_t nb = ceil_div(n, Q_BLOCK);
   uint32_t grid = round_up8(nb);
   float best = bound_to_best(dist_bound);
-  if (use_knn_queue(b, n, k)) {
+  if (queue) {
     const int lg = knn_queue_lanes_log2(n, k, b.points);
     const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE);
     KernelTimer kt(b.ctx, s, "knn");

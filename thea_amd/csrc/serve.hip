@@ -201,7 +201,7 @@ static void worker_loop(Server *S, int wi) {
               d.cp = q.cp;
               d.best_init = bound_to_best(q.bound);
             }
-            if (q.n >= ORDER_MIN_QUERIES) {
+            if (q.n >= ORDER_MIN_QUERIES && (!queue || q.n > QUEUE_UNSORTED_MAX)) {
               scratch.emplace_back(new QueryScratch());
               if (type == THG_REQ_RAY) order_rays(b, q.q, q.dirs, q.n, *scratch.back(), s);
               else order_queries(b, q.q, q.n, *scratch.back(), s);
