@@ -9,7 +9,7 @@
 //   -> keys (mesh id << b) | Morton code (32 - b bits) and one stable radix sort over all meshes,
 //      which groups the elements by mesh in input order
 //   -> Karras radix trees, each over its mesh's key range (global positions and node ids)
-//   -> one bottom-up refit, per-mesh leaf sizes, one compaction, one emit, records with local ids
+//   -> records with local ids and the box pyramid, per-mesh leaf sizes, one compaction, one emit
 //   -> queries sorted by (mesh, Morton) the same way where some mesh's kernel needs it
 //   -> multi-segment closest-point launches (work queue, wave walk): segment m walks mesh m's tree from
 //      its root.
@@ -22,6 +22,7 @@
 
 #include "common.hpp"
 #include "kernels_common.hpp"
+#include "build_device.hpp"
 #include "query.hpp"
 #include "tri_math.hpp"
 
@@ -54,9 +55,9 @@ struct BatchPlan {
   std::vector<int4> tchunks, qchunks;
   DevBuf verts, tris, queries;
   DevBuf d_info, d_tchunks, d_qchunks, mbounds;
-  DevBuf center, blo, bhi, keys, vals, tk, tv, hist;
-  DevBuf left, right, rfirst, rlast, nparent, lparent, flags, nbox, keep, fidx, stmp;
-  DevBuf nodes, recs, screen, seg, out_idx, out_dist, counters, rent, rcount, rlist, bad;
+  DevBuf center, boxes, keys, vals, tk, tv, hist;
+  DevBuf split, rfirst, rlast, parent, keep, fidx, stmp;
+  DevBuf nodes, recs, screen, seg, out_idx, out_dist, counters, bad;
   int block_waves = 4;     // workgroup shape of the query launch (waves per workgroup)
   bool spill_build = true;  // the 8-resident-wave build of the query kernel
   hipGraphExec_t exec = nullptr;
@@ -113,8 +114,7 @@ __global__ void k_init_mbounds(int *mb, int nm) {
 // Element boxes/centres and per-mesh bounds; chunk = (mesh, first element, count), one mesh each.
 __global__ void __launch_bounds__(BB) k_bprep(const float *__restrict__ verts, const int32_t *__restrict__ tris,
                                               const MeshInfo *__restrict__ mi, const int4 *__restrict__ chunks,
-                                              float4 *__restrict__ center, float4 *__restrict__ blo,
-                                              float4 *__restrict__ bhi, int *__restrict__ mb) {
+                                              float4 *__restrict__ center, int *__restrict__ mb) {
   const int4 ch = chunks[blockIdx.x];
   const int m = ch.x;
   const int64_t voff = mi[m].voff, toff = mi[m].toff;
@@ -136,8 +136,6 @@ __global__ void __launch_bounds__(BB) k_bprep(const float *__restrict__ verts, c
     float3 s = add3(add3(v[0], v[1]), v[2]);
     float3 c = f3(s.x / 3.0f, s.y / 3.0f, s.z / 3.0f);
     center[e] = make_float4(c.x, c.y, c.z, 0.0f);
-    blo[e] = make_float4(lo.x, lo.y, lo.z, 0.0f);
-    bhi[e] = make_float4(hi.x, hi.y, hi.z, 0.0f);
     mn[0] = fminf(mn[0], lo.x); mn[1] = fminf(mn[1], lo.y); mn[2] = fminf(mn[2], lo.z);
     mx[0] = fmaxf(mx[0], hi.x); mx[1] = fmaxf(mx[1], hi.y); mx[2] = fmaxf(mx[2], hi.z);
     mn[3] = fminf(mn[3], c.x); mn[4] = fminf(mn[4], c.y); mn[5] = fminf(mn[5], c.z);
@@ -216,9 +214,8 @@ __device__ __forceinline__ int bdelta(const uint32_t *__restrict__ k, int64_t a,
 }
 
 __global__ void __launch_bounds__(BB) k_bkarras(const uint32_t *__restrict__ k, const MeshInfo *__restrict__ mi, int nm,
-                                                int64_t NT, int32_t *__restrict__ left, int32_t *__restrict__ right,
-                                                int32_t *__restrict__ rfirst, int32_t *__restrict__ rlast,
-                                                int32_t *__restrict__ nparent, int32_t *__restrict__ lparent) {
+                                                int64_t NT, int32_t *__restrict__ rfirst, int32_t *__restrict__ rlast,
+                                                uint32_t *__restrict__ split, uint32_t *__restrict__ keep) {
   int64_t pos = (int64_t)blockIdx.x * BB + threadIdx.x;
   if (pos >= NT) return;
   int m = mesh_of(mi, nm, pos, false, false);
@@ -244,42 +241,33 @@ __global__ void __launch_bounds__(BB) k_bkarras(const uint32_t *__restrict__ k, 
   int64_t g = i + s * d + (d < 0 ? -1 : 0);
   int64_t first = i < j ? i : j, last = i < j ? j : i;
   const int64_t node = ibase + i;
-  int32_t lc, rc;
-  if (first == g) { lc = (int32_t)(g | 0x80000000u); lparent[g] = (int32_t)node; }
-  else { lc = (int32_t)(ibase + g); nparent[ibase + g] = (int32_t)node; }
-  if (last == g + 1) { rc = (int32_t)((g + 1) | 0x80000000u); lparent[g + 1] = (int32_t)node; }
-  else { rc = (int32_t)(ibase + g + 1); nparent[ibase + g + 1] = (int32_t)node; }
-  left[node] = lc;
-  right[node] = rc;
   rfirst[node] = (int32_t)first;
   rlast[node] = (int32_t)last;
-  if (i == a) nparent[node] = -1;
-}
-
-__global__ void __launch_bounds__(BB) k_bkeep(const int32_t *__restrict__ rfirst, const int32_t *__restrict__ rlast,
-                                              const MeshInfo *__restrict__ mi, int nm, int64_t NI,
-                                              uint32_t *__restrict__ keep) {
-  int64_t g = (int64_t)blockIdx.x * BB + threadIdx.x;
-  if (g >= NI) return;
-  int m = mesh_of(mi, nm, rfirst[g], false, false);
-  keep[g] = (rlast[g] - rfirst[g] + 1) > mi[m].leaf ? 1u : 0u;
+  split[node] = (uint32_t)g | (d < 0 ? 0x80000000u : 0u);
+  keep[node] = last - first + 1 > mi[m].leaf ? 1u : 0u;
 }
 
 __global__ void __launch_bounds__(BB) k_brecords(const float *__restrict__ verts, const int32_t *__restrict__ tris,
                                                  const uint32_t *__restrict__ sorted, const MeshInfo *__restrict__ mi,
-                                                 int nm, int64_t NT, TriRec *__restrict__ out) {
-  int64_t pos = (int64_t)blockIdx.x * BB + threadIdx.x;
-  if (pos >= NT) return;
-  const int64_t e = sorted[pos];
-  const int m = mesh_of(mi, nm, e, false, false);
-  const int64_t voff = mi[m].voff;
-  float3 v[3];
+                                                 int nm, int64_t NT, TriRec *__restrict__ out,
+                                                 ScreenRec *__restrict__ scr, BoxLevels P) {
+  const int64_t pos = (int64_t)blockIdx.x * BB + threadIdx.x;
+  float3 lo = f3(INFINITY, INFINITY, INFINITY), hi = f3(-INFINITY, -INFINITY, -INFINITY);
+  if (pos < NT) {
+    const int64_t e = sorted[pos];
+    const int m = mesh_of(mi, nm, e, false, false);
+    const int64_t voff = mi[m].voff;
+    float3 v[3];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const int64_t vi = voff + tris[3 * e + c];
-    v[c] = f3(verts[3 * vi], verts[3 * vi + 1], verts[3 * vi + 2]);
+    for (int c = 0; c < 3; ++c) {
+      const int64_t vi = voff + tris[3 * e + c];
+      v[c] = f3(verts[3 * vi], verts[3 * vi + 1], verts[3 * vi + 2]);
+    }
+    lo = min3(v[0], min3(v[1], v[2]));
+    hi = max3(v[0], max3(v[1], v[2]));
+    put_triangle(pos, v[0], v[1], v[2], (int32_t)(e - mi[m].toff), out, nullptr, scr);
   }
-  out[pos] = make_trirec(v[0], v[1], v[2], (int32_t)(e - mi[m].toff));
+  pyramid_block(P, 0, true, lo, hi);
 }
 
 // Single-leaf roots of small meshes and the segment table of the query launch.
@@ -348,44 +336,35 @@ static void plan_pipeline(BatchPlan &P, hipStream_t s, hipEvent_t mid = nullptr)
   const MeshInfo *mi = P.d_info.as<MeshInfo>();
   int *mb = P.mbounds.as<int>();
   hipLaunchKernelGGL(k_init_mbounds, dim3(ceil_div((uint64_t)nm * 12, BB)), dim3(BB), 0, s, mb, nm);
-  hipLaunchKernelGGL(k_fill_i32, dim3(ceil_div(std::max<int64_t>(P.NT, 1), BB)), dim3(BB), 0, s, P.lparent.as<int32_t>(),
-                     P.NT, -1);
-  if (P.NI > 0)
-    hipLaunchKernelGGL(k_fill_i32, dim3(ceil_div(P.NI, BB)), dim3(BB), 0, s, (int32_t *)P.flags.as<uint32_t>(), P.NI, 0);
+  if (P.NI > 0)  // roots keep -1
+    hipLaunchKernelGGL(k_fill_i32, dim3(ceil_div(P.NI + P.nsmall, BB)), dim3(BB), 0, s, P.parent.as<int32_t>(),
+                       P.NI + P.nsmall, -1);
   hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(BB), 0, s, P.counters.as<int32_t>(), (int64_t)4, 0);
   launch_check("batch fill");
   if (P.NT > 0) {
     hipLaunchKernelGGL(k_bprep, dim3((uint32_t)P.tchunks.size()), dim3(BB), 0, s, P.verts.as<float>(), P.tris.as<int32_t>(),
-                       mi, P.d_tchunks.as<int4>(), P.center.as<float4>(), P.blo.as<float4>(), P.bhi.as<float4>(), mb);
+                       mi, P.d_tchunks.as<int4>(), P.center.as<float4>(), mb);
     launch_check("k_bprep");
     hipLaunchKernelGGL(k_bkeys, dim3(ceil_div(P.NT, BB)), dim3(BB), 0, s, P.center.as<float4>(), mi, nm, mb, P.mesh_bits,
                        P.NT, P.keys.as<uint32_t>());
     launch_check("k_bkeys");
     radix_sort_iota(P.keys.as<uint32_t>(), P.vals.as<uint32_t>(), P.tk.as<uint32_t>(), P.tv.as<uint32_t>(),
-                    P.hist.as<uint32_t>(), P.NT, 0, 32, s);
+                    P.hist.as<uint32_t>(), P.NT, 0, 32, false, s);
     hipLaunchKernelGGL(k_bkarras, dim3(ceil_div(P.NT, BB)), dim3(BB), 0, s, P.keys.as<uint32_t>(), mi, nm, P.NT,
-                       P.left.as<int32_t>(), P.right.as<int32_t>(), P.rfirst.as<int32_t>(), P.rlast.as<int32_t>(),
-                       P.nparent.as<int32_t>(), P.lparent.as<int32_t>());
+                       P.rfirst.as<int32_t>(), P.rlast.as<int32_t>(), P.split.as<uint32_t>(), P.keep.as<uint32_t>());
     launch_check("k_bkarras");
-    launch_refit(P.NT, P.vals.as<uint32_t>(), P.blo.as<float4>(), P.bhi.as<float4>(), P.left.as<int32_t>(),
-                 P.right.as<int32_t>(), P.rfirst.as<int32_t>(), P.rlast.as<int32_t>(), P.nparent.as<int32_t>(),
-                 P.lparent.as<int32_t>(), P.flags.as<uint32_t>(), P.nbox.as<float>(), P.rent.as<int32_t>(),
-                 P.rcount.as<uint32_t>(), P.rlist.as<int32_t>(), s);
-    if (P.NI > 0) {
-      hipLaunchKernelGGL(k_bkeep, dim3(ceil_div(P.NI, BB)), dim3(BB), 0, s, P.rfirst.as<int32_t>(), P.rlast.as<int32_t>(),
-                         mi, nm, P.NI, P.keep.as<uint32_t>());
-      launch_check("k_bkeep");
-      scan_excl_u32(P.keep.as<uint32_t>(), P.fidx.as<uint32_t>(), P.NI, P.stmp.as<uint32_t>(), s);
-      launch_emit(P.NI, P.nsmall, P.keep.as<uint32_t>(), P.fidx.as<uint32_t>(), P.left.as<int32_t>(), P.right.as<int32_t>(),
-                  P.rfirst.as<int32_t>(), P.rlast.as<int32_t>(), P.vals.as<uint32_t>(), P.blo.as<float4>(),
-                  P.bhi.as<float4>(), P.nbox.as<float>(), P.nodes.as<BNode>(), nullptr, s);
-      launch_depth(P.NT, P.lparent.as<int32_t>(), P.nparent.as<int32_t>(), P.keep.as<uint32_t>(),
-                   P.rfirst.as<int32_t>(), P.counters.as<int32_t>() + 1, s);
-    }
+    const BoxLevels L = box_levels(P.NT, P.boxes.as<float4>());
     hipLaunchKernelGGL(k_brecords, dim3(ceil_div(P.NT, BB)), dim3(BB), 0, s, P.verts.as<float>(), P.tris.as<int32_t>(),
-                       P.vals.as<uint32_t>(), mi, nm, P.NT, P.recs.as<TriRec>());
+                       P.vals.as<uint32_t>(), mi, nm, P.NT, P.recs.as<TriRec>(), P.screen.as<ScreenRec>(), L);
     launch_check("k_brecords");
-    launch_screen_records(P.recs.as<TriRec>(), P.NT, P.screen.as<ScreenRec>(), s);
+    if (P.NI > 0) {
+      launch_pyramid_top(L, s);
+      scan_excl_u32(P.keep.as<uint32_t>(), P.fidx.as<uint32_t>(), P.NI, P.stmp.as<uint32_t>(), s);
+      launch_emit(P.NI, P.nsmall, P.keep.as<uint32_t>(), P.fidx.as<uint32_t>(), P.rfirst.as<int32_t>(),
+                  P.rlast.as<int32_t>(), P.split.as<uint32_t>(), L, P.nodes.as<BNode>(), P.parent.as<int32_t>(), s);
+      launch_node_depth(P.NI, P.nsmall, P.fidx.as<uint32_t>() + P.NI, P.parent.as<int32_t>(),
+                        P.counters.as<int32_t>() + 1, nullptr, s);
+    }
   }
   if (mid) THG_HIP(hipEventRecord(mid, s));
   if (P.NQ > 0) {
@@ -551,11 +530,11 @@ int thg_batch_plan_create(thg_ctx ctx, int32_t nm, const int64_t *nv, const int6
       THG_HIP(hipMemcpy(P->d_tchunks.p, P->tchunks.data(), sizeof(int4) * P->tchunks.size(), hipMemcpyHostToDevice));
     P->mbounds.alloc(sizeof(int) * 12 * nm);
     const int64_t T1 = std::max<int64_t>(to, 1), I1 = std::max<int64_t>(io, 1);
-    P->center.alloc(T1 * 16); P->blo.alloc(T1 * 16); P->bhi.alloc(T1 * 16);
+    P->center.alloc(T1 * 16); P->boxes.alloc((size_t)box_level_entries(T1) * 32);
     P->keys.alloc(K * 4); P->vals.alloc(K * 4); P->tk.alloc(K * 4); P->tv.alloc(K * 4);
     P->hist.alloc(radix_hist_words(K) * 4);
-    P->left.alloc(I1 * 4); P->right.alloc(I1 * 4); P->rfirst.alloc(I1 * 4); P->rlast.alloc(I1 * 4);
-    P->nparent.alloc(I1 * 4); P->lparent.alloc(T1 * 4); P->flags.alloc(I1 * 4); P->nbox.alloc(I1 * 24);
+    P->split.alloc(I1 * 4); P->rfirst.alloc(I1 * 4); P->rlast.alloc(I1 * 4);
+    P->parent.alloc((size_t)(P->nsmall + io + 1) * 4);
     P->keep.alloc(I1 * 4); P->fidx.alloc((I1 + 1) * 4); P->stmp.alloc(scan_tmp_words(I1) * 4);
     P->nodes.alloc(sizeof(BNode) * (size_t)(P->nsmall + io + 1));
     P->recs.alloc(sizeof(TriRec) * T1);
@@ -564,9 +543,6 @@ int thg_batch_plan_create(thg_ctx ctx, int32_t nm, const int64_t *nv, const int6
     P->out_idx.alloc(std::max<int64_t>(qo, 1) * 4);
     P->out_dist.alloc(std::max<int64_t>(qo, 1) * 4);
     P->counters.alloc(16);
-    P->rent.alloc(T1 * 4);
-    P->rcount.alloc(refit_count_words(T1) * 4);
-    P->rlist.alloc(refit_needs_list(T1) ? T1 * 4 : 4);
     P->bad.alloc(4);
     THG_HIP(hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking));
     *out = reinterpret_cast<thg_batch_plan>(P.release());

@@ -7,14 +7,18 @@
 //  3. radix sort      (code, element) pairs, stable, so equal codes keep element order.
 //  4. k_karras        binary radix tree over the sorted codes (Karras, "Maximizing Parallelism in
 //                     the Construction of BVHs, Octrees, and k-d Trees", HPG 2012), duplicate codes
-//                     disambiguated by position.
-//  5. k_refit         bottom-up boxes; the second child to arrive at a node (atomic counter) merges.
-//  6. k_collapse/emit subtrees of <= leaf_size elements become leaves; remaining nodes are
-//                     compacted into 64-byte BNodes holding both children's boxes.
-//  7. k_records       element records in leaf order (TriRec with Thea's per-triangle constants).
+//                     disambiguated by position; nodes of more than leaf_size elements are kept.
+//  5. k_records       element records in leaf order (TriRec with Thea's per-triangle constants,
+//                     RayTri, ScreenRec) and the box pyramid: the boxes of every aligned run of 2^L
+//                     sorted elements, a block's 256 at a time from registers.
+//  6. k_emit          kept nodes compacted into 64-byte BNodes holding both children's boxes. A
+//                     node is a range of sorted elements, so its box is the union of the at most
+//                     2 log2(range) pyramid runs that tile it.
+//  7. k_node_depth    levels of the compacted tree.
 // Boxes are exact float min/max of element coordinates; the query kernels add their own rounding
 // slack, so no padding is applied here.
 #include "kernels_common.hpp"
+#include "build_device.hpp"
 #include "query.hpp"
 #include "tri_math.hpp"
 
@@ -32,7 +36,6 @@ __device__ __forceinline__ float3 ld_vert(const float *__restrict__ verts, int64
 
 __global__ void __launch_bounds__(B_BLOCK) k_elem_prep(const float *__restrict__ verts, const int32_t *__restrict__ tris,
                                                        int64_t n, int points, float4 *__restrict__ center,
-                                                       float4 *__restrict__ blo, float4 *__restrict__ bhi,
                                                        int *__restrict__ part) {
   float mn[6] = {INFINITY, INFINITY, INFINITY, INFINITY, INFINITY, INFINITY};
   float mx[6] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -50,8 +53,6 @@ __global__ void __launch_bounds__(B_BLOCK) k_elem_prep(const float *__restrict__
       c = f3(s.x / 3.0f, s.y / 3.0f, s.z / 3.0f);
     }
     center[i] = make_float4(c.x, c.y, c.z, 0.0f);
-    blo[i] = make_float4(lo.x, lo.y, lo.z, 0.0f);
-    bhi[i] = make_float4(hi.x, hi.y, hi.z, 0.0f);
     mn[0] = fminf(mn[0], lo.x); mn[1] = fminf(mn[1], lo.y); mn[2] = fminf(mn[2], lo.z);
     mx[0] = fmaxf(mx[0], hi.x); mx[1] = fmaxf(mx[1], hi.y); mx[2] = fmaxf(mx[2], hi.z);
     mn[3] = fminf(mn[3], c.x); mn[4] = fminf(mn[4], c.y); mn[5] = fminf(mn[5], c.z);
@@ -79,9 +80,16 @@ __global__ void __launch_bounds__(B_BLOCK) k_elem_prep(const float *__restrict__
 }
 
 // One wave per slot: the min (lo slots) or max (hi slots) of the block partials.
+// Also clears the depth, sets the node count of a single-leaf tree and marks node 0 as the root.
 __global__ void __launch_bounds__(12 * WAVE) k_bounds_reduce(const int *__restrict__ part, int nb,
-                                                             BoundsAcc *__restrict__ acc) {
+                                                             BoundsAcc *__restrict__ acc, int32_t *__restrict__ depth,
+                                                             uint32_t *__restrict__ one, int32_t *__restrict__ parent) {
   const int k = threadIdx.x / WAVE, lane = lane_id();
+  if (threadIdx.x == 0) {
+    *depth = 0;
+    *one = 1;
+    parent[0] = -1;
+  }
   const bool lo_slot = k < 3 || (k >= 6 && k < 9);
   int v = lo_slot ? float_to_ord(INFINITY) : float_to_ord(-INFINITY);
   for (int b = lane; b < nb; b += WAVE) {
@@ -112,12 +120,32 @@ __device__ __forceinline__ uint32_t morton30(float3 c, float3 lo, float3 inv) {
   return (spread10(ix) << 2) | (spread10(iy) << 1) | spread10(iz);
 }
 
-__global__ void __launch_bounds__(B_BLOCK) k_morton(const float4 *__restrict__ center, int64_t n, float3 lo, float3 inv,
-                                                    uint32_t *__restrict__ keys) {
-  int64_t i = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  if (i >= n) return;
-  float4 c = center[i];
-  keys[i] = morton30(f3(c.x, c.y, c.z), lo, inv);
+// Morton codes in the centre bounds (acc) and the histograms of their first sorted digit, one sort
+// tile per block.
+template <int ITEMS>
+__global__ void __launch_bounds__(RS_BLOCK) k_morton(const float4 *__restrict__ center, int64_t n,
+                                                     const BoundsAcc *__restrict__ acc, uint32_t tiles,
+                                                     uint32_t *__restrict__ keys, uint32_t *__restrict__ hist) {
+  __shared__ RadixHist h;
+  h.clear();
+  float f[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) f[k] = ord_to_float(acc->v[6 + k]);
+  const float3 lo = f3(f[0], f[1], f[2]), ext = f3(f[3] - f[0], f[4] - f[1], f[5] - f[2]);
+  const float3 inv = f3(ext.x > 0 ? 1.0f / ext.x : 0.0f, ext.y > 0 ? 1.0f / ext.y : 0.0f,
+                        ext.z > 0 ? 1.0f / ext.z : 0.0f);
+  const int64_t base = (int64_t)blockIdx.x * (RS_BLOCK * ITEMS);
+#pragma unroll 4
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t i = base + (int64_t)r * RS_BLOCK + threadIdx.x;
+    if (i < n) {
+      const float4 c = center[i];
+      const uint32_t key = morton30(f3(c.x, c.y, c.z), lo, inv);
+      keys[i] = key;
+      h.count(key, 0);
+    }
+  }
+  h.store(hist, tiles);
 }
 
 // Common prefix length of sorted (code, position) keys i and j; -1 outside [0, n).
@@ -128,11 +156,12 @@ __device__ __forceinline__ int delta(const uint32_t *__restrict__ k, int64_t n, 
   return __clz(a ^ b);
 }
 
-// Internal node i of n - 1: children (leaf if flag bit 31 set), range, parent links.
-__global__ void __launch_bounds__(B_BLOCK) k_karras(const uint32_t *__restrict__ k, int64_t n, int32_t *__restrict__ left,
-                                                    int32_t *__restrict__ right, int32_t *__restrict__ rfirst,
-                                                    int32_t *__restrict__ rlast, int32_t *__restrict__ node_parent,
-                                                    int32_t *__restrict__ leaf_parent) {
+// Internal node i of n - 1: its range [first, last], its split g (left child [first, g], right child
+// [g + 1, last]; bit 31 set if i is the range's end) and whether it is kept. Its children, where they
+// are internal, are the nodes g and g + 1.
+__global__ void __launch_bounds__(B_BLOCK) k_karras(const uint32_t *__restrict__ k, int64_t n, int leaf_size,
+                                                    int32_t *__restrict__ rfirst, int32_t *__restrict__ rlast,
+                                                    uint32_t *__restrict__ split, uint32_t *__restrict__ keep) {
   int64_t i = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
   if (i >= n - 1) return;
   int d = (delta(k, n, i, i + 1) - delta(k, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -154,346 +183,124 @@ __global__ void __launch_bounds__(B_BLOCK) k_karras(const uint32_t *__restrict__
   } while (t > 1);
   int64_t g = i + s * d + (d < 0 ? -1 : 0);
   int64_t first = i < j ? i : j, last = i < j ? j : i;
-  int32_t lc, rc;
-  if (first == g) { lc = (int32_t)(g | 0x80000000u); leaf_parent[g] = (int32_t)i; }
-  else { lc = (int32_t)g; node_parent[g] = (int32_t)i; }
-  if (last == g + 1) { rc = (int32_t)((g + 1) | 0x80000000u); leaf_parent[g + 1] = (int32_t)i; }
-  else { rc = (int32_t)(g + 1); node_parent[g + 1] = (int32_t)i; }
-  left[i] = lc;
-  right[i] = rc;
   rfirst[i] = (int32_t)first;
   rlast[i] = (int32_t)last;
-  if (i == 0) node_parent[0] = -1;
+  split[i] = (uint32_t)g | (d < 0 ? 0x80000000u : 0u);
+  keep[i] = last - first + 1 > leaf_size ? 1u : 0u;
 }
 
-__device__ __forceinline__ float ld_coherent(const float *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_coherent(float *p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Levels base + 1 .. base + 8 from level base.
+__global__ void __launch_bounds__(B_BLOCK) k_pyramid(BoxLevels P, int base) {
+  const int64_t i = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
+  float3 lo = f3(INFINITY, INFINITY, INFINITY), hi = f3(-INFINITY, -INFINITY, -INFINITY);
+  if (i < P.count(base)) {
+    const float4 a = P.box[2 * (P.off[base] + i)], b = P.box[2 * (P.off[base] + i) + 1];
+    lo = f3(a.x, a.y, a.z);
+    hi = f3(b.x, b.y, b.z);
+  }
+  pyramid_block(P, base, false, lo, hi);
 }
 
-// Bottom-up refit over the Karras tree. Node boxes: nbox[6 i + 0..5] = lo xyz, hi xyz.
-// `sorted` maps sorted position -> element; element boxes come from blo/bhi.
-__global__ void __launch_bounds__(B_BLOCK) k_refit(int64_t n, const uint32_t *__restrict__ sorted,
-                                                   const float4 *__restrict__ blo, const float4 *__restrict__ bhi,
-                                                   const int32_t *__restrict__ left, const int32_t *__restrict__ right,
-                                                   const int32_t *__restrict__ node_parent,
-                                                   const int32_t *__restrict__ leaf_parent, uint32_t *__restrict__ flags,
-                                                   float *nbox) {
-  int64_t k = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  if (k >= n) return;
-  int32_t cur = leaf_parent[k];
-  while (cur >= 0) {
-    __threadfence();
-    uint32_t old = atomicAdd(&flags[cur], 1u);
-    if (old == 0) return;  // first child to arrive; the sibling's thread continues
-    __threadfence();
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    int32_t ch[2] = {left[cur], right[cur]};
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      if (ch[c] < 0) {
-        uint32_t e = sorted[ch[c] & 0x7fffffff];
-        float4 a = blo[e], b = bhi[e];
-        lo[0] = fminf(lo[0], a.x); lo[1] = fminf(lo[1], a.y); lo[2] = fminf(lo[2], a.z);
-        hi[0] = fmaxf(hi[0], b.x); hi[1] = fmaxf(hi[1], b.y); hi[2] = fmaxf(hi[2], b.z);
-      } else {
-        const float *q = nbox + 6 * (int64_t)ch[c];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          lo[a] = fminf(lo[a], ld_coherent(q + a));
-          hi[a] = fmaxf(hi[a], ld_coherent(q + 3 + a));
-        }
-      }
+BoxLevels box_levels(int64_t n, float4 *box) {
+  BoxLevels P{};
+  P.n = n;
+  P.box = box;
+  while (((int64_t)2 << P.top) <= n) ++P.top;
+  for (int L = 0; L < P.top; ++L) P.off[L + 1] = P.off[L] + P.count(L);
+  return P;
+}
+int64_t box_level_entries(int64_t n) {
+  const BoxLevels P = box_levels(n, nullptr);
+  return P.off[P.top] + P.count(P.top);
+}
+
+void launch_pyramid_top(const BoxLevels &P, hipStream_t s) {
+  for (int base = 8; base < P.top; base += 8) {
+    hipLaunchKernelGGL(k_pyramid, dim3(ceil_div(P.count(base), B_BLOCK)), dim3(B_BLOCK), 0, s, P, base);
+    launch_check("k_pyramid");
+  }
+}
+
+// Union of the element boxes of sorted positions [first, last].
+__device__ __forceinline__ void range_box(const BoxLevels &P, int64_t first, int64_t last, float3 &lo, float3 &hi) {
+  lo = f3(INFINITY, INFINITY, INFINITY);
+  hi = f3(-INFINITY, -INFINITY, -INFINITY);
+  int64_t l = first, r = last + 1;
+  for (int L = 0; l < r; ++L, l >>= 1, r >>= 1) {
+    const float4 *b = P.box + 2 * P.off[L];
+    if (l & 1) {
+      const float4 x = b[2 * l], y = b[2 * l + 1];
+      lo = min3(lo, f3(x.x, x.y, x.z));
+      hi = max3(hi, f3(y.x, y.y, y.z));
+      ++l;
     }
-    float *o = nbox + 6 * (int64_t)cur;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) { st_coherent(o + a, lo[a]); st_coherent(o + 3 + a, hi[a]); }
-    cur = node_parent[cur];
-  }
-}
-
-// Two-pass refit. Pass 1 (k_refit_span): a block owns REFIT_SPAN consecutive sorted positions and
-// computes every internal node whose element range lies inside them. A node's split position g
-// (left child = [first, g], right child = [g + 1, last]) is unique, so LDS slot g - span start
-// holds the node's arrival counter and one box per side; the second child to arrive merges, with
-// workgroup-scope ordering only. Node boxes go to global memory as they are computed. A child whose
-// parent straddles the span appends the parent to the span's own list, entries[span start ...]
-// with an LDS counter, and the block stores the list's length in nentries[span]. (One device-wide
-// counter for all spans serialised the pass: a few hundred thousand appends on one address.) The
-// maximal subtrees inside a span have disjoint ranges in it, so a list never outgrows the span.
-// Pass 2 (k_refit_top) finishes the straddling nodes with the device-wide arrival protocol of
-// k_refit; there are O(depth) of them per span boundary, so the costly device-scope fences run for
-// a small fraction of the nodes.
-constexpr int REFIT_SPAN = 1024;
-constexpr int REFIT_THREADS = 256;
-constexpr int REFIT_TOP_LANES = 16;
-
-__device__ __forceinline__ void elem_box(const uint32_t *__restrict__ sorted, const float4 *__restrict__ blo,
-                                         const float4 *__restrict__ bhi, int64_t pos, float b[6]) {
-  const uint32_t e = sorted[pos];
-  const float4 a = blo[e], c = bhi[e];
-  b[0] = a.x; b[1] = a.y; b[2] = a.z; b[3] = c.x; b[4] = c.y; b[5] = c.z;
-}
-
-__global__ void __launch_bounds__(REFIT_THREADS) k_refit_span(int64_t n, const uint32_t *__restrict__ sorted,
-                                                              const float4 *__restrict__ blo,
-                                                              const float4 *__restrict__ bhi,
-                                                              const int32_t *__restrict__ rfirst,
-                                                              const int32_t *__restrict__ rlast,
-                                                              const int32_t *__restrict__ node_parent,
-                                                              const int32_t *__restrict__ leaf_parent, float *nbox,
-                                                              int32_t *__restrict__ entries,
-                                                              uint32_t *__restrict__ nentries) {
-  __shared__ float s_l[REFIT_SPAN * 6], s_r[REFIT_SPAN * 6];
-  __shared__ uint32_t s_flag[REFIT_SPAN];
-  __shared__ uint32_t s_nent;
-  const int64_t lo = (int64_t)blockIdx.x * REFIT_SPAN;
-  const int64_t hi = lo + REFIT_SPAN < n ? lo + REFIT_SPAN : n;
-  for (int i = threadIdx.x; i < REFIT_SPAN; i += REFIT_THREADS) s_flag[i] = 0;
-  if (threadIdx.x == 0) s_nent = 0;
-  __syncthreads();
-  for (int64_t k = lo + threadIdx.x; k < hi; k += REFIT_THREADS) {
-    float b[6];
-    elem_box(sorted, blo, bhi, k, b);
-    int64_t cf = k, cl = k;  // element range of the completed child
-    int32_t p = leaf_parent[k];
-    while (p >= 0) {
-      const int64_t fp = rfirst[p], lp = rlast[p];
-      if (fp < lo || lp >= hi) {
-        entries[lo + atomicAdd(&s_nent, 1u)] = p;
-        break;
-      }
-      const bool is_left = cf == fp;
-      const int slot = (int)((is_left ? cl : cf - 1) - lo);
-      float *mine = (is_left ? s_l : s_r) + 6 * slot;
-#pragma unroll
-      for (int a = 0; a < 6; ++a) mine[a] = b[a];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-      if (atomicAdd(&s_flag[slot], 1u) == 0) break;  // the sibling's thread continues
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-      const float *other = (is_left ? s_r : s_l) + 6 * slot;
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        b[a] = fminf(b[a], other[a]);
-        b[3 + a] = fmaxf(b[3 + a], other[3 + a]);
-      }
-      float *o = nbox + 6 * (int64_t)p;
-#pragma unroll
-      for (int a = 0; a < 6; ++a) o[a] = b[a];
-      cf = fp;
-      cl = lp;
-      p = node_parent[p];
+    if (r & 1) {
+      --r;
+      const float4 x = b[2 * r], y = b[2 * r + 1];
+      lo = min3(lo, f3(x.x, x.y, x.z));
+      hi = max3(hi, f3(y.x, y.y, y.z));
     }
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) nentries[blockIdx.x] = s_nent;
-}
-
-// Box of internal node `cur` from its two children: element boxes, or node boxes written before
-// (read at L2 with agent-scope atomics, so a concurrent writer's box is never a stale L1 copy).
-__device__ __forceinline__ void refit_node(int32_t cur, const uint32_t *__restrict__ sorted,
-                                           const float4 *__restrict__ blo, const float4 *__restrict__ bhi,
-                                           const int32_t *__restrict__ left, const int32_t *__restrict__ right,
-                                           float *nbox) {
-  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  const int32_t ch[2] = {left[cur], right[cur]};
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    float b[6];
-    if (ch[c] < 0) {
-      elem_box(sorted, blo, bhi, ch[c] & 0x7fffffff, b);
-    } else {
-      const float *q = nbox + 6 * (int64_t)ch[c];
-#pragma unroll
-      for (int a = 0; a < 6; ++a) b[a] = ld_coherent(q + a);
-    }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      lo[a] = fminf(lo[a], b[a]);
-      hi[a] = fmaxf(hi[a], b[3 + a]);
-    }
-  }
-  float *o = nbox + 6 * (int64_t)cur;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) { st_coherent(o + a, lo[a]); st_coherent(o + 3 + a, hi[a]); }
-}
-
-// Fenced walk from `cur` to the root with the device-wide arrival protocol of k_refit.
-__device__ __forceinline__ void refit_walk(int32_t cur, const uint32_t *__restrict__ sorted,
-                                           const float4 *__restrict__ blo, const float4 *__restrict__ bhi,
-                                           const int32_t *__restrict__ left, const int32_t *__restrict__ right,
-                                           const int32_t *__restrict__ node_parent, uint32_t *flags, float *nbox) {
-  while (cur >= 0) {
-    __threadfence();
-    if (atomicAdd(&flags[cur], 1u) == 0) break;  // first arrival; the other child's thread continues
-    __threadfence();
-    refit_node(cur, sorted, blo, bhi, left, right, nbox);
-    cur = node_parent[cur];
-  }
-}
-
-// Pass 2 for small trees: REFIT_TOP_LANES threads per span list walk up with fences.
-__global__ void __launch_bounds__(B_BLOCK) k_refit_top(const uint32_t *__restrict__ sorted,
-                                                       const float4 *__restrict__ blo, const float4 *__restrict__ bhi,
-                                                       const int32_t *__restrict__ left,
-                                                       const int32_t *__restrict__ right,
-                                                       const int32_t *__restrict__ node_parent,
-                                                       const int32_t *__restrict__ entries,
-                                                       const uint32_t *__restrict__ nentries, uint32_t spans,
-                                                       uint32_t *flags, float *nbox) {
-  const uint64_t t = (uint64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  const uint32_t sp = (uint32_t)(t / REFIT_TOP_LANES);
-  if (sp >= spans) return;
-  const uint32_t count = nentries[sp];
-  for (uint32_t e = (uint32_t)(t % REFIT_TOP_LANES); e < count; e += REFIT_TOP_LANES)
-    refit_walk(entries[(int64_t)sp * REFIT_SPAN + e], sorted, blo, bhi, left, right, node_parent, flags, nbox);
-}
-
-// Pass 2 for large trees, level by level. A device-scope fence writes back the issuing XCD's L2 on
-// this GPU, and the fenced walk pays two per node: 5-7 ms on the 512-mesh batched build, where
-// the top tree above 41.7k spans has some 10^5 nodes. Instead, k_refit_arrive counts one arrival
-// per span-list entry, and a node's second arrival queues it as ready (both children's boxes are
-// written); each k_refit_level launch then writes the boxes of the ready nodes and counts one
-// arrival at each parent, queueing the parents that became ready for the next launch. Kernel
-// boundaries order every box write before its reads, so no fence is needed. After REFIT_LEVELS
-// launches (more than a tree's usual height), the last one finishes any remaining nodes with the
-// fenced walk, so the result never depends on the height.
-constexpr int REFIT_LEVELS = 64;
-constexpr uint32_t REFIT_LEVEL_MIN_SPANS = 4096;
-constexpr uint32_t REFIT_LEVEL_GRID = 512;
-
-__global__ void k_zero_words(uint32_t *p, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
-}
-
-__global__ void __launch_bounds__(B_BLOCK) k_refit_arrive(const int32_t *__restrict__ entries,
-                                                          const uint32_t *__restrict__ nentries, uint32_t spans,
-                                                          uint32_t *flags, int32_t *__restrict__ out,
-                                                          uint32_t *out_cnt) {
-  const uint64_t t = (uint64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  const uint32_t sp = (uint32_t)(t / REFIT_TOP_LANES);
-  if (sp >= spans) return;
-  const uint32_t count = nentries[sp];
-  for (uint32_t e = (uint32_t)(t % REFIT_TOP_LANES); e < count; e += REFIT_TOP_LANES) {
-    const int32_t p = entries[(int64_t)sp * REFIT_SPAN + e];
-    if (atomicAdd(&flags[p], 1u) == 1u) out[wave_append(out_cnt)] = p;
-  }
-}
-
-__global__ void __launch_bounds__(B_BLOCK) k_refit_level(const uint32_t *__restrict__ sorted,
-                                                         const float4 *__restrict__ blo,
-                                                         const float4 *__restrict__ bhi,
-                                                         const int32_t *__restrict__ left,
-                                                         const int32_t *__restrict__ right,
-                                                         const int32_t *__restrict__ node_parent,
-                                                         const int32_t *__restrict__ in,
-                                                         const uint32_t *__restrict__ in_cnt,
-                                                         int32_t *__restrict__ out, uint32_t *out_cnt,
-                                                         uint32_t *flags, float *nbox, int last) {
-  const uint32_t count = *in_cnt;
-  for (uint32_t i = blockIdx.x * B_BLOCK + threadIdx.x; i < count; i += gridDim.x * B_BLOCK) {
-    const int32_t p = in[i];
-    refit_node(p, sorted, blo, bhi, left, right, nbox);
-    const int32_t q = node_parent[p];
-    if (last) {
-      refit_walk(q, sorted, blo, bhi, left, right, node_parent, flags, nbox);
-    } else if (q >= 0 && atomicAdd(&flags[q], 1u) == 1u) {
-      out[wave_append(out_cnt)] = q;
-    }
-  }
-}
-
-// keep[i] = 1 if internal node i stays an internal node of the collapsed tree (range > leaf_size).
-__global__ void __launch_bounds__(B_BLOCK) k_keep(int64_t n, const int32_t *__restrict__ rfirst,
-                                                  const int32_t *__restrict__ rlast, int leaf_size,
-                                                  uint32_t *__restrict__ keep) {
-  int64_t i = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  if (i >= n - 1) return;
-  keep[i] = (rlast[i] - rfirst[i] + 1) > leaf_size ? 1u : 0u;
-}
-
-__device__ __forceinline__ void child_box(int32_t c, const uint32_t *sorted, const float4 *blo, const float4 *bhi,
-                                          const float *nbox, float lo[3], float hi[3]) {
-  if (c < 0) {
-    uint32_t e = sorted[c & 0x7fffffff];
-    float4 a = blo[e], b = bhi[e];
-    lo[0] = a.x; lo[1] = a.y; lo[2] = a.z; hi[0] = b.x; hi[1] = b.y; hi[2] = b.z;
-  } else {
-    const float *q = nbox + 6 * (int64_t)c;
-    lo[0] = q[0]; lo[1] = q[1]; lo[2] = q[2]; hi[0] = q[3]; hi[1] = q[4]; hi[2] = q[5];
   }
 }
 
 // Emit the collapsed tree. `fidx` = exclusive prefix of keep (final node index of kept nodes, plus
-// `base`); a child that is not kept becomes a leaf over its whole element range. `leaf_count`, when
-// given, receives the number of leaves (a diagnostic: a full binary tree with `kept` internal nodes
-// has kept + 1 leaves, which the builders use instead, since one counter that every wave adds to
-// serialises the launch: 7.6 ms of the 512-mesh batched build).
-__global__ void __launch_bounds__(B_BLOCK) k_emit(int64_t n, int32_t base, const uint32_t *__restrict__ keep,
-                                                  const uint32_t *__restrict__ fidx, const int32_t *__restrict__ left,
-                                                  const int32_t *__restrict__ right, const int32_t *__restrict__ rfirst,
-                                                  const int32_t *__restrict__ rlast, const uint32_t *__restrict__ sorted,
-                                                  const float4 *__restrict__ blo, const float4 *__restrict__ bhi,
-                                                  const float *__restrict__ nbox, BNode *__restrict__ out,
-                                                  uint32_t *__restrict__ leaf_count) {
-  int64_t i = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  uint32_t leaves = 0;
-  if (i < n - 1 && keep[i]) {
-    int32_t ch[2] = {left[i], right[i]};
-    float lo[2][3], hi[2][3];
-    int32_t ref[2], cnt[2];
+// `base`); a child that is not kept becomes a leaf over its whole element range. parent[node] = the
+// parent's final index, for every kept node but the roots.
+//
+// Each box is read from the pyramid (a handful of 32-byte runs, most ranges being short) instead of
+// being merged bottom-up: the walks of a refit, one element per thread to the next unfinished ancestor
+// and fenced above 1,024 elements, took 285 us of a 1M-triangle build, where this kernel takes 41 us
+// (17 us without boxes) and the pyramid's upper levels 10 us, and needed parent links, arrival counters
+// and a box per internal node (96-mesh plan: 502 -> 117 us).
+__global__ void __launch_bounds__(B_BLOCK) k_emit(int64_t ni, int32_t base, const uint32_t *__restrict__ keep,
+                                                  const uint32_t *__restrict__ fidx, const int32_t *__restrict__ rfirst,
+                                                  const int32_t *__restrict__ rlast,
+                                                  const uint32_t *__restrict__ split, BoxLevels P,
+                                                  BNode *__restrict__ out, int32_t *__restrict__ parent) {
+  const int64_t i = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
+  if (i >= ni || !keep[i]) return;
+  const uint32_t sp = split[i];
+  const int64_t first = rfirst[i], last = rlast[i], g = sp & 0x7fffffffu;
+  const int64_t shift = i - ((sp >> 31) ? last : first);  // node index less sorted position (batched trees)
+  float3 lo[2], hi[2];
+  int32_t ref[2], cnt[2];
+  const int32_t me = base + (int32_t)fidx[i];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      child_box(ch[c], sorted, blo, bhi, nbox, lo[c], hi[c]);
-      if (ch[c] < 0) {
-        ref[c] = ~(ch[c] & 0x7fffffff);
-        cnt[c] = 1;
-        ++leaves;
-      } else if (!keep[ch[c]]) {
-        ref[c] = ~rfirst[ch[c]];
-        cnt[c] = rlast[ch[c]] - rfirst[ch[c]] + 1;
-        ++leaves;
-      } else {
-        ref[c] = base + (int32_t)fidx[ch[c]];
-        cnt[c] = 0;
-      }
+  for (int c = 0; c < 2; ++c) {
+    const int64_t a = c == 0 ? first : g + 1, b = c == 0 ? g : last;
+    const int64_t node = g + c + shift;
+    range_box(P, a, b, lo[c], hi[c]);
+    if (a == b || !keep[node]) {
+      ref[c] = ~(int32_t)a;
+      cnt[c] = (int32_t)(b - a + 1);
+    } else {
+      ref[c] = base + (int32_t)fidx[node];
+      cnt[c] = 0;
+      parent[ref[c]] = me;
     }
-    BNode nd;
-    nd.a = make_float4(lo[0][0], lo[0][1], lo[0][2], hi[0][0]);
-    nd.b = make_float4(hi[0][1], hi[0][2], lo[1][0], lo[1][1]);
-    nd.c = make_float4(lo[1][2], hi[1][0], hi[1][1], hi[1][2]);
-    nd.d = make_int4(ref[0], ref[1], cnt[0], cnt[1]);
-    out[base + fidx[i]] = nd;
   }
-  if (leaf_count) {
-    // one atomic per wave on the shared counter (every lane of the wave takes part in the sum)
-    leaves = wave_sum(leaves);
-    if (lane_id() == 0 && leaves) atomicAdd(leaf_count, leaves);
-  }
+  BNode nd;
+  nd.a = make_float4(lo[0].x, lo[0].y, lo[0].z, hi[0].x);
+  nd.b = make_float4(hi[0].y, hi[0].z, lo[1].x, lo[1].y);
+  nd.c = make_float4(lo[1].z, hi[1].x, hi[1].y, hi[1].z);
+  nd.d = make_int4(ref[0], ref[1], cnt[0], cnt[1]);
+  out[me] = nd;
 }
 
-// Maximum leaf depth of the collapsed tree (number of kept ancestors), via atomicMax. The elements
-// of one collapsed leaf share their kept ancestors, so only the leaf's first element walks to the
-// root; the others stop after the non-kept nodes above them (all inside that leaf). Ancestors of a
-// kept node are kept (their ranges are larger).
-__global__ void __launch_bounds__(B_BLOCK) k_depth(int64_t n, const int32_t *__restrict__ leaf_parent,
-                                                   const int32_t *__restrict__ node_parent,
-                                                   const uint32_t *__restrict__ keep,
-                                                   const int32_t *__restrict__ rfirst, int32_t *__restrict__ max_depth) {
-  int64_t k = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
+// Levels of the compacted tree (nodes [first, first + *count)): *max_depth becomes the largest number
+// of nodes on a path, which is the depth of the deepest leaf; even[i] (optional) = 1 for nodes at even
+// depth.
+__global__ void __launch_bounds__(B_BLOCK) k_node_depth(int64_t first, const uint32_t *__restrict__ count,
+                                                        const int32_t *__restrict__ parent,
+                                                        int32_t *__restrict__ max_depth, uint32_t *__restrict__ even) {
+  const int64_t k = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
   int d = 0;
-  if (k < n) {
-    int32_t cur = leaf_parent[k], top = -1;
-    while (cur >= 0 && !keep[cur]) {
-      top = cur;
-      cur = node_parent[cur];
-    }
-    if (top < 0 || rfirst[top] == k)
-      for (; cur >= 0; cur = node_parent[cur]) ++d;
+  if (k < (int64_t)*count) {
+    d = 1;
+    for (int32_t p = parent[first + k]; p >= 0; p = parent[p]) ++d;
+    if (even) even[k] = d & 1;
   }
-  int m = (int)wave_max((float)d);  // every lane of the wave takes part in the reduction
+  const int m = (int)wave_max((float)d);  // every lane of the wave takes part in the reduction
   // one atomic per wave, and none once the maximum is known to be at least this wave's
   if (lane_id() == 0 && m > __hip_atomic_load(max_depth, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
     atomicMax(max_depth, m);
@@ -501,55 +308,33 @@ __global__ void __launch_bounds__(B_BLOCK) k_depth(int64_t n, const int32_t *__r
 
 __global__ void __launch_bounds__(B_BLOCK) k_tri_records(const float *__restrict__ verts, const int32_t *__restrict__ tris,
                                                          const uint32_t *__restrict__ sorted, int64_t n,
-                                                         TriRec *__restrict__ out) {
-  int64_t k = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  if (k >= n) return;
-  uint32_t e = sorted[k];
-  float3 v0 = ld_vert(verts, tris[3 * (int64_t)e]), v1 = ld_vert(verts, tris[3 * (int64_t)e + 1]),
-         v2 = ld_vert(verts, tris[3 * (int64_t)e + 2]);
-  out[k] = make_trirec(v0, v1, v2, (int32_t)e);
+                                                         TriRec *__restrict__ rec, RayTri *__restrict__ ray,
+                                                         ScreenRec *__restrict__ scr, BoxLevels P) {
+  const int64_t k = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
+  float3 lo = f3(INFINITY, INFINITY, INFINITY), hi = f3(-INFINITY, -INFINITY, -INFINITY);
+  if (k < n) {
+    const int64_t e = sorted[k];
+    const float3 v0 = ld_vert(verts, tris[3 * e]), v1 = ld_vert(verts, tris[3 * e + 1]),
+                 v2 = ld_vert(verts, tris[3 * e + 2]);
+    lo = min3(v0, min3(v1, v2));
+    hi = max3(v0, max3(v1, v2));
+    put_triangle(k, v0, v1, v2, (int32_t)e, rec, ray, scr);
+  }
+  pyramid_block(P, 0, true, lo, hi);
 }
 
 __global__ void __launch_bounds__(B_BLOCK) k_point_records(const float *__restrict__ xyz, const uint32_t *__restrict__ sorted,
-                                                           int64_t n, PointRec *__restrict__ out) {
-  int64_t k = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  if (k >= n) return;
-  uint32_t e = sorted[k];
-  PointRec r;
-  r.p = make_float4(xyz[3 * (int64_t)e], xyz[3 * (int64_t)e + 1], xyz[3 * (int64_t)e + 2], __int_as_float((int)e));
-  out[k] = r;
-}
-
-// Screening records from the triangle records, in the same (leaf) order.
-__global__ void __launch_bounds__(B_BLOCK) k_screen_records(const TriRec *__restrict__ tr, int64_t n,
-                                                            ScreenRec *__restrict__ out) {
+                                                           int64_t n, PointRec *__restrict__ out, BoxLevels P) {
   const int64_t k = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  if (k >= n) return;
-  ScreenRec r;
-  r.c = tr[k].sb;
-  r.n = make_float4(tr[k].p0.w, tr[k].p1.w, tr[k].p2.w, 0.0f);
-  out[k] = r;
-}
-
-void launch_screen_records(const TriRec *tr, int64_t n, ScreenRec *out, hipStream_t s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_screen_records, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, tr, n, out);
-  launch_check("k_screen_records");
-}
-
-// Ray records from the triangle records, in the same (leaf) order.
-__global__ void __launch_bounds__(B_BLOCK) k_ray_records(const TriRec *__restrict__ tr, int64_t n,
-                                                         RayTri *__restrict__ out) {
-  const int64_t k = (int64_t)blockIdx.x * B_BLOCK + threadIdx.x;
-  if (k >= n) return;
-  const TriRec &r = tr[k];
-  const float3 v0 = f3(r.p0.x, r.p0.y, r.p0.z);
-  const float3 e01 = sub3(f3(r.p1.x, r.p1.y, r.p1.z), v0), e02 = sub3(f3(r.p2.x, r.p2.y, r.p2.z), v0);
-  RayTri o;
-  o.a = make_float4(v0.x, v0.y, v0.z, r.pl.w);
-  o.b = make_float4(e01.x, e01.y, e01.z, 0.0f);
-  o.c = make_float4(e02.x, e02.y, e02.z, 0.0f);
-  out[k] = o;
+  float3 lo = f3(INFINITY, INFINITY, INFINITY), hi = f3(-INFINITY, -INFINITY, -INFINITY);
+  if (k < n) {
+    const uint32_t e = sorted[k];
+    lo = hi = ld_vert(xyz, e);
+    PointRec r;
+    r.p = make_float4(lo.x, lo.y, lo.z, __int_as_float((int)e));
+    out[k] = r;
+  }
+  pyramid_block(P, 0, true, lo, hi);
 }
 
 // Flags the last ray record of every non-empty leaf (RayTri::b.w int bits = 1), so ray traversal can
@@ -706,77 +491,25 @@ void scan_excl_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *tmp, 
 
 // Entry points for the batched many-mesh pipeline (batch.hip), which reuses these kernels over
 // concatenated meshes with global element positions and node indices.
-static bool refit_atomic_only() {
-  static const bool v = [] {
-    const char *e = getenv("THG_REFIT");
-    return e && atoi(e) == 1;
-  }();
-  return v;
-}
-
-size_t refit_count_words(int64_t n) {
-  return (size_t)std::max<int64_t>(ceil_div(n, (int64_t)REFIT_SPAN), 1) + REFIT_LEVELS + 2;
-}
-bool refit_needs_list(int64_t n) { return ceil_div(n, (int64_t)REFIT_SPAN) >= REFIT_LEVEL_MIN_SPANS; }
-
-// `flags` (one per internal node) must be zero; `entries` holds n int32, `nentries`
-// refit_count_words(n) uint32, and `list` n int32 when refit_needs_list(n) (else it may be null).
-void launch_refit(int64_t n, const uint32_t *sorted, const float4 *blo, const float4 *bhi, const int32_t *left,
-                  const int32_t *right, const int32_t *rfirst, const int32_t *rlast, const int32_t *nparent,
-                  const int32_t *lparent, uint32_t *flags, float *nbox, int32_t *entries, uint32_t *nentries,
-                  int32_t *list, hipStream_t s) {
-  if (n <= 0) return;
-  if (refit_atomic_only()) {
-    hipLaunchKernelGGL(k_refit, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, n, sorted, blo, bhi, left, right,
-                       nparent, lparent, flags, nbox);
-    launch_check("k_refit");
-    return;
-  }
-  const uint32_t spans = ceil_div(n, (int64_t)REFIT_SPAN);
-  hipLaunchKernelGGL(k_refit_span, dim3(spans), dim3(REFIT_THREADS), 0, s, n, sorted, blo, bhi, rfirst, rlast, nparent,
-                     lparent, nbox, entries, nentries);
-  launch_check("k_refit_span");
-  const uint32_t grid = (uint32_t)ceil_div((int64_t)spans * REFIT_TOP_LANES, (int64_t)B_BLOCK);
-  if (!refit_needs_list(n)) {
-    hipLaunchKernelGGL(k_refit_top, dim3(grid), dim3(B_BLOCK), 0, s, sorted, blo, bhi, left, right, nparent, entries,
-                       nentries, spans, flags, nbox);
-    launch_check("k_refit_top");
-    return;
-  }
-  require(list != nullptr, "refit: level list missing");
-  uint32_t *cnt = nentries + spans;  // REFIT_LEVELS + 1 list lengths
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(128), 0, s, cnt, REFIT_LEVELS + 1);
-  launch_check("k_zero_words");
-  hipLaunchKernelGGL(k_refit_arrive, dim3(grid), dim3(B_BLOCK), 0, s, entries, nentries, spans, flags, list, cnt);
-  launch_check("k_refit_arrive");
-  // level L reads list L (even: `list`, odd: `entries`, whose span lists are consumed) and writes L + 1
-  for (int L = 0; L < REFIT_LEVELS; ++L) {
-    int32_t *in = (L & 1) ? entries : list, *out = (L & 1) ? list : entries;
-    hipLaunchKernelGGL(k_refit_level, dim3(REFIT_LEVEL_GRID), dim3(B_BLOCK), 0, s, sorted, blo, bhi, left, right,
-                       nparent, in, cnt + L, out, cnt + L + 1, flags, nbox, L == REFIT_LEVELS - 1 ? 1 : 0);
-    launch_check("k_refit_level");
-  }
-}
-
-void launch_emit(int64_t ni, int32_t base, const uint32_t *keep, const uint32_t *fidx, const int32_t *left,
-                 const int32_t *right, const int32_t *rfirst, const int32_t *rlast, const uint32_t *sorted,
-                 const float4 *blo, const float4 *bhi, const float *nbox, BNode *out, uint32_t *leaf_count,
+void launch_emit(int64_t ni, int32_t base, const uint32_t *keep, const uint32_t *fidx, const int32_t *rfirst,
+                 const int32_t *rlast, const uint32_t *split, const BoxLevels &P, BNode *out, int32_t *parent,
                  hipStream_t s) {
   if (ni <= 0) return;
-  hipLaunchKernelGGL(k_emit, dim3(ceil_div(ni, B_BLOCK)), dim3(B_BLOCK), 0, s, ni + 1, base, keep, fidx, left, right,
-                     rfirst, rlast, sorted, blo, bhi, nbox, out, leaf_count);
+  hipLaunchKernelGGL(k_emit, dim3(ceil_div(ni, B_BLOCK)), dim3(B_BLOCK), 0, s, ni, base, keep, fidx, rfirst, rlast,
+                     split, P, out, parent);
   launch_check("k_emit");
 }
 
-void launch_depth(int64_t n, const int32_t *lparent, const int32_t *nparent, const uint32_t *keep, const int32_t *rfirst,
-                  int32_t *max_depth, hipStream_t s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_depth, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, n, lparent, nparent, keep, rfirst,
-                     max_depth);
-  launch_check("k_depth");
+void launch_node_depth(int64_t max_nodes, int64_t first, const uint32_t *count, const int32_t *parent,
+                       int32_t *max_depth, uint32_t *even, hipStream_t s) {
+  if (max_nodes <= 0) return;
+  hipLaunchKernelGGL(k_node_depth, dim3(ceil_div(max_nodes, B_BLOCK)), dim3(B_BLOCK), 0, s, first, count, parent,
+                     max_depth, even);
+  launch_check("k_node_depth");
 }
 
-// Host driver shared by mesh and point builds.
+// Host driver shared by mesh and point builds. Two waits: for the bounds and the kept node count, which
+// size the nodes, and for the depth and the ray tree's node count, which sizes that.
 void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool points, int leaf_size, hipStream_t s) {
   b.points = points;
   b.n = n;
@@ -787,16 +520,80 @@ void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool 
     b.max_depth = 0;
     return;
   }
-  uint32_t grid = std::min<uint32_t>(ceil_div(n, B_BLOCK), 4096);
-  DevBuf center(n * sizeof(float4)), blo(n * sizeof(float4)), bhi(n * sizeof(float4)), acc(sizeof(BoundsAcc)),
-      part((size_t)grid * 12 * sizeof(int));
-  hipLaunchKernelGGL(k_elem_prep, dim3(grid), dim3(B_BLOCK), 0, s, verts, tris, n, points ? 1 : 0,
-                     center.as<float4>(), blo.as<float4>(), bhi.as<float4>(), part.as<int>());
+  // arrays over the elements that the BVH keeps, in one allocation
+  {
+    const size_t eb = (size_t)n * (points ? sizeof(PointRec) : sizeof(TriRec));
+    Layout lay;
+    const size_t oe = lay.add(eb), orr = lay.add(points ? 0 : n * sizeof(RayTri)),
+                 os = lay.add(points ? 0 : n * sizeof(ScreenRec)), ol = lay.add(points ? 0 : n * sizeof(LeafBound));
+    b.store.alloc(lay.total);
+    char *base = b.store.as<char>();
+    b.elems.view(base + oe, eb);
+    b.rays.view(base + orr, points ? 0 : n * sizeof(RayTri));
+    b.screen.view(base + os, points ? 0 : n * sizeof(ScreenRec));
+    b.lbounds.view(base + ol, points ? 0 : n * sizeof(LeafBound));
+  }
+  const int64_t ni = std::max<int64_t>(n - 1, 1);
+  const uint32_t grid = std::min<uint32_t>(ceil_div(n, B_BLOCK), 1024);
+  struct Counts {  // device words read by the host
+    BoundsAcc bounds;
+    int32_t depth;
+    uint32_t one;
+  };
+  Layout lay;
+  const size_t o_cnt = lay.add(sizeof(Counts)), o_part = lay.add((size_t)grid * 12 * sizeof(int)),
+               o_keys = lay.add(n * 4), o_vals = lay.add(n * 4), o_tk = lay.add(n * 4), o_tv = lay.add(n * 4),
+               o_hist = lay.add(radix_hist_words(n) * 4), o_first = lay.add(ni * 4), o_last = lay.add(ni * 4),
+               o_split = lay.add(ni * 4), o_keep = lay.add(ni * 4), o_fidx = lay.add((ni + 1) * 4),
+               o_parent = lay.add(ni * 4), o_stmp = lay.add(scan_tmp_words(ni) * 4),
+               // the centres are read before the pyramid is written, the flags of the ray tree written after
+               // the pyramid's last use
+               o_box = lay.add(std::max<size_t>((size_t)box_level_entries(n) * 32, n * sizeof(float4)));
+  Workspace ws;
+  ws.alloc(lay.total, s);
+  Counts *cnt = ws.at<Counts>(o_cnt);
+  float4 *center = ws.at<float4>(o_box);
+  uint32_t *keys = ws.at<uint32_t>(o_keys), *vals = ws.at<uint32_t>(o_vals), *hist = ws.at<uint32_t>(o_hist);
+  uint32_t *keep = ws.at<uint32_t>(o_keep), *fidx = ws.at<uint32_t>(o_fidx), *stmp = ws.at<uint32_t>(o_stmp);
+  int32_t *parent = ws.at<int32_t>(o_parent);
+
+  hipLaunchKernelGGL(k_elem_prep, dim3(grid), dim3(B_BLOCK), 0, s, verts, tris, n, points ? 1 : 0, center,
+                     ws.at<int>(o_part));
   launch_check("k_elem_prep");
-  hipLaunchKernelGGL(k_bounds_reduce, dim3(1), dim3(12 * WAVE), 0, s, part.as<int>(), (int)grid, acc.as<BoundsAcc>());
+  hipLaunchKernelGGL(k_bounds_reduce, dim3(1), dim3(12 * WAVE), 0, s, ws.at<int>(o_part), (int)grid, &cnt->bounds,
+                     &cnt->depth, &cnt->one, parent);
   launch_check("k_bounds_reduce");
+  const uint32_t tiles = radix_tiles(n);
+  if (radix_items(n) == RS_ITEMS_SMALL)
+    hipLaunchKernelGGL(k_morton<RS_ITEMS_SMALL>, dim3(tiles), dim3(RS_BLOCK), 0, s, center, n, &cnt->bounds, tiles,
+                       keys, hist);
+  else
+    hipLaunchKernelGGL(k_morton<RS_ITEMS_LARGE>, dim3(tiles), dim3(RS_BLOCK), 0, s, center, n, &cnt->bounds, tiles,
+                       keys, hist);
+  launch_check("k_morton");
+  radix_sort_iota(keys, vals, ws.at<uint32_t>(o_tk), ws.at<uint32_t>(o_tv), hist, n, 0, 32, true, s);
+
+  const BoxLevels P = box_levels(n, ws.at<float4>(o_box));
+  if (points)
+    hipLaunchKernelGGL(k_point_records, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, verts, vals, n,
+                       b.elems.as<PointRec>(), P);
+  else
+    hipLaunchKernelGGL(k_tri_records, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, verts, tris, vals, n,
+                       b.elems.as<TriRec>(), b.rays.as<RayTri>(), b.screen.as<ScreenRec>(), P);
+  launch_check("k_records");
+
+  const bool single = n <= leaf_size;
+  uint32_t kept = 1;
+  if (!single) {
+    hipLaunchKernelGGL(k_karras, dim3(ceil_div(ni, B_BLOCK)), dim3(B_BLOCK), 0, s, keys, n, leaf_size,
+                       ws.at<int32_t>(o_first), ws.at<int32_t>(o_last), ws.at<uint32_t>(o_split), keep);
+    launch_check("k_karras");
+    scan_excl_u32(keep, fidx, ni, stmp, s);
+    launch_pyramid_top(P, s);
+    THG_HIP(hipMemcpyAsync(&kept, fidx + ni, 4, hipMemcpyDeviceToHost, s));
+  }
   BoundsAcc h;
-  THG_HIP(hipMemcpyAsync(&h, acc.p, sizeof(h), hipMemcpyDeviceToHost, s));
+  THG_HIP(hipMemcpyAsync(&h, &cnt->bounds, sizeof(h), hipMemcpyDeviceToHost, s));
   THG_HIP(hipStreamSynchronize(s));
   float f[12];
   for (int k = 0; k < 12; ++k) f[k] = ord_to_float(h.v[k]);
@@ -805,102 +602,37 @@ void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool 
   b.scale = 0;
   for (int k = 0; k < 6; ++k) b.scale = std::max(b.scale, std::fabs(f[k]));
   require(std::isfinite(b.scale), "element coordinates must be finite");
-
-  size_t rec_bytes = points ? sizeof(PointRec) : sizeof(TriRec);
-  b.elems.alloc(n * rec_bytes);
-
-  DevBuf keys(n * 4), vals(n * 4), tk(n * 4), tv(n * 4), hist(radix_hist_words(n) * 4);
-  float3 clo = f3(f[6], f[7], f[8]);
-  float3 cext = f3(f[9] - f[6], f[10] - f[7], f[11] - f[8]);
-  float3 inv = f3(cext.x > 0 ? 1.0f / cext.x : 0.0f, cext.y > 0 ? 1.0f / cext.y : 0.0f, cext.z > 0 ? 1.0f / cext.z : 0.0f);
-  hipLaunchKernelGGL(k_morton, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, center.as<float4>(), n, clo, inv,
-                     keys.as<uint32_t>());
-  launch_check("k_morton");
-  radix_sort_iota(keys.as<uint32_t>(), vals.as<uint32_t>(), tk.as<uint32_t>(), tv.as<uint32_t>(), hist.as<uint32_t>(), n,
-                   0, 32, s);
-  const uint32_t *sorted = vals.as<uint32_t>();
-
-  if (points)
-    hipLaunchKernelGGL(k_point_records, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, verts, sorted, n,
-                       b.elems.as<PointRec>());
-  else
-    hipLaunchKernelGGL(k_tri_records, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, verts, tris, sorted, n,
-                       b.elems.as<TriRec>());
-  launch_check("k_records");
-  if (!points) {
-    b.rays.alloc(n * sizeof(RayTri));
-    hipLaunchKernelGGL(k_ray_records, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, b.elems.as<TriRec>(), n,
-                       b.rays.as<RayTri>());
-    launch_check("k_ray_records");
-    b.screen.alloc(n * sizeof(ScreenRec));
-    launch_screen_records(b.elems.as<TriRec>(), n, b.screen.as<ScreenRec>(), s);
-  }
-
-  if (n <= leaf_size) {
-    b.nodes.alloc(sizeof(BNode));
+  b.nodes.alloc((size_t)kept * sizeof(BNode));
+  b.num_nodes = kept;
+  b.num_leaves = single ? 1 : (int64_t)kept + 1;  // a full binary tree
+  const uint32_t *count = single ? &cnt->one : fidx + ni;
+  if (single) {
     hipLaunchKernelGGL(k_single_leaf, dim3(1), dim3(1), 0, s, n, b.lo, b.hi, b.nodes.as<BNode>());
     launch_check("k_single_leaf");
-    if (!points) {
-      hipLaunchKernelGGL(k_leaf_ends, dim3(1), dim3(B_BLOCK), 0, s, b.nodes.as<BNode>(), (int64_t)1,
-                         b.rays.as<RayTri>());
-      launch_check("k_leaf_ends");
-      b.lbounds.alloc(n * sizeof(LeafBound));
-      launch_leaf_bounds(b.nodes.as<BNode>(), 1, nullptr, 1, b.elems.as<TriRec>(), b.lbounds.as<LeafBound>(), s);
-    }
-    b.num_nodes = 1;
-    b.num_leaves = 1;
-    b.max_depth = 1;
-    if (!points) build_qbvh4(b, s);
-    THG_HIP(hipStreamSynchronize(s));
-    return;
+  } else {
+    launch_emit(ni, 0, keep, fidx, ws.at<int32_t>(o_first), ws.at<int32_t>(o_last), ws.at<uint32_t>(o_split), P,
+                b.nodes.as<BNode>(), parent, s);
   }
-
-  int64_t ni = n - 1;
-  DevBuf left(ni * 4), right(ni * 4), rfirst(ni * 4), rlast(ni * 4), nparent(ni * 4), lparent(n * 4);
-  DevBuf flags(ni * 4), nbox(ni * 6 * sizeof(float)), keep(ni * 4), fidx((ni + 1) * 4), counters(16);
-  DevBuf entries(n * 4), nentries(refit_count_words(n) * 4), rlist(refit_needs_list(n) ? n * 4 : 4);
-  THG_HIP(hipMemsetAsync(flags.p, 0, ni * 4, s));
-  THG_HIP(hipMemsetAsync(counters.p, 0, 16, s));
-  hipLaunchKernelGGL(k_karras, dim3(ceil_div(ni, B_BLOCK)), dim3(B_BLOCK), 0, s, keys.as<uint32_t>(), n,
-                     left.as<int32_t>(), right.as<int32_t>(), rfirst.as<int32_t>(), rlast.as<int32_t>(),
-                     nparent.as<int32_t>(), lparent.as<int32_t>());
-  launch_check("k_karras");
-  launch_refit(n, sorted, blo.as<float4>(), bhi.as<float4>(), left.as<int32_t>(), right.as<int32_t>(),
-               rfirst.as<int32_t>(), rlast.as<int32_t>(), nparent.as<int32_t>(), lparent.as<int32_t>(),
-               flags.as<uint32_t>(), nbox.as<float>(), entries.as<int32_t>(), nentries.as<uint32_t>(), rlist.as<int32_t>(), s);
-  hipLaunchKernelGGL(k_keep, dim3(ceil_div(ni, B_BLOCK)), dim3(B_BLOCK), 0, s, n, rfirst.as<int32_t>(),
-                     rlast.as<int32_t>(), leaf_size, keep.as<uint32_t>());
-  launch_check("k_keep");
-  DevBuf stmp(scan_tmp_words(ni) * 4);
-  scan_excl_u32(keep.as<uint32_t>(), fidx.as<uint32_t>(), ni, stmp.as<uint32_t>(), s);
-  uint32_t kept = 0;
-  THG_HIP(hipMemcpyAsync(&kept, fidx.as<uint32_t>() + ni, 4, hipMemcpyDeviceToHost, s));
-  THG_HIP(hipStreamSynchronize(s));
-  b.nodes.alloc((size_t)kept * sizeof(BNode));
-  int32_t *maxd = reinterpret_cast<int32_t *>(counters.as<uint32_t>() + 1);
-  hipLaunchKernelGGL(k_emit, dim3(ceil_div(ni, B_BLOCK)), dim3(B_BLOCK), 0, s, n, 0, keep.as<uint32_t>(),
-                     fidx.as<uint32_t>(), left.as<int32_t>(), right.as<int32_t>(), rfirst.as<int32_t>(),
-                     rlast.as<int32_t>(), sorted, blo.as<float4>(), bhi.as<float4>(), nbox.as<float>(),
-                     b.nodes.as<BNode>(), nullptr);
-  launch_check("k_emit");
-  hipLaunchKernelGGL(k_depth, dim3(ceil_div(n, B_BLOCK)), dim3(B_BLOCK), 0, s, n, lparent.as<int32_t>(),
-                     nparent.as<int32_t>(), keep.as<uint32_t>(), rfirst.as<int32_t>(), maxd);
-  launch_check("k_depth");
-  uint32_t cnt[2];
-  THG_HIP(hipMemcpyAsync(cnt, counters.p, 8, hipMemcpyDeviceToHost, s));
-  THG_HIP(hipStreamSynchronize(s));
-  b.num_nodes = kept;
-  b.num_leaves = (int64_t)kept + 1;  // a full binary tree
-  b.max_depth = (int32_t)cnt[1];
+  // even-depth flags of the nodes and their scan, for the ray tree (in the pyramid's place)
+  uint32_t *even = points ? nullptr : ws.at<uint32_t>(o_box), *qidx = keep;  // keep: ni >= kept words
+  launch_node_depth(kept, 0, count, parent, &cnt->depth, even, s);
+  uint32_t nq = 0;
   if (!points) {
+    qidx = ws.at<uint32_t>(o_first);  // the ranges are no longer needed; o_last follows for the total
+    scan_excl_u32(even, qidx, kept, stmp, s);
+    THG_HIP(hipMemcpyAsync(&nq, qidx + kept, 4, hipMemcpyDeviceToHost, s));
     hipLaunchKernelGGL(k_leaf_ends, dim3(ceil_div(kept, B_BLOCK)), dim3(B_BLOCK), 0, s, b.nodes.as<BNode>(),
                        (int64_t)kept, b.rays.as<RayTri>());
     launch_check("k_leaf_ends");
-    b.lbounds.alloc(n * sizeof(LeafBound));
     launch_leaf_bounds(b.nodes.as<BNode>(), (int64_t)kept, nullptr, (int64_t)kept, b.elems.as<TriRec>(),
                        b.lbounds.as<LeafBound>(), s);
-    build_qbvh4(b, s);
   }
+  int32_t depth = 0;
+  THG_HIP(hipMemcpyAsync(&depth, &cnt->depth, 4, hipMemcpyDeviceToHost, s));
+  THG_HIP(hipStreamSynchronize(s));
+  b.max_depth = depth;
+  if (!points) build_qbvh4(b, even, qidx, nq, s);
+  THG_HIP(hipStreamSynchronize(s));
 }
 
 }  // namespace thg

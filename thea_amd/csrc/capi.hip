@@ -50,6 +50,91 @@ __global__ void k_check_tris(const int32_t *__restrict__ tris, int64_t n3, int64
   }
 }
 
+namespace {
+struct DevBlock {
+  void *p;
+  size_t bytes;
+  int device;
+};
+std::mutex g_blocks_mu;
+std::vector<DevBlock> &kept_blocks() {  // oldest first; never destroyed (the driver is gone by then)
+  static auto *v = new std::vector<DevBlock>();
+  return *v;
+}
+}  // namespace
+
+hipError_t dev_alloc(void **p, size_t n, size_t *block, int *device) {
+  hipError_t e = hipGetDevice(device);
+  if (e != hipSuccess) return e;
+  {
+    std::lock_guard<std::mutex> g(g_blocks_mu);
+    auto &v = kept_blocks();
+    size_t best = v.size();
+    for (size_t i = 0; i < v.size(); ++i)
+      if (v[i].device == *device && v[i].bytes >= n && v[i].bytes - n <= n / 4 &&
+          (best == v.size() || v[i].bytes < v[best].bytes))
+        best = i;
+    if (best < v.size()) {
+      *p = v[best].p;
+      *block = v[best].bytes;
+      v.erase(v.begin() + best);
+      return hipSuccess;
+    }
+  }
+  e = hipMalloc(p, n);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    dev_cache_release(*device);
+    e = hipMalloc(p, n);
+  }
+  *block = n;
+  return e;
+}
+
+void dev_free(void *p, size_t block, int device) {
+  if (block > DEV_CACHE_BYTES) {
+    (void)hipFree(p);
+    return;
+  }
+  int cur = device;
+  (void)hipGetDevice(&cur);
+  if (cur != device) (void)hipSetDevice(device);
+  const bool idle = hipDeviceSynchronize() == hipSuccess;
+  if (cur != device) (void)hipSetDevice(cur);
+  std::vector<void *> out;
+  if (idle) {
+    std::lock_guard<std::mutex> g(g_blocks_mu);
+    auto &v = kept_blocks();
+    v.push_back({p, block, device});
+    size_t held = 0;
+    for (const auto &b : v) held += b.device == device ? b.bytes : 0;
+    for (size_t i = 0; i < v.size() && held > DEV_CACHE_BYTES;) {
+      if (v[i].device != device) { ++i; continue; }
+      held -= v[i].bytes;
+      out.push_back(v[i].p);
+      v.erase(v.begin() + i);
+    }
+  } else {
+    (void)hipGetLastError();
+    out.push_back(p);
+  }
+  for (void *q : out) (void)hipFree(q);
+}
+
+void dev_cache_release(int device) {
+  std::vector<void *> out;
+  {
+    std::lock_guard<std::mutex> g(g_blocks_mu);
+    auto &v = kept_blocks();
+    for (size_t i = 0; i < v.size();) {
+      if (v[i].device != device) { ++i; continue; }
+      out.push_back(v[i].p);
+      v.erase(v.begin() + i);
+    }
+  }
+  for (void *q : out) (void)hipFree(q);
+}
+
 // Fails with THG_E_INVALID unless every index of the nt triangles (device memory) is in [0, nv).
 void check_tri_indices(const int32_t *tris, int64_t nt, int64_t nv, hipStream_t s) {
   if (nt <= 0) return;
@@ -133,7 +218,13 @@ int thg_ctx_create(int32_t device, thg_ctx *out) {
 }
 
 int thg_ctx_destroy(thg_ctx ctx) {
-  return guarded([&] { delete reinterpret_cast<Ctx *>(ctx); });
+  return guarded([&] {
+    Ctx *c = reinterpret_cast<Ctx *>(ctx);
+    if (!c) return;
+    const int device = c->device;
+    delete c;
+    dev_cache_release(device);
+  });
 }
 
 int thg_ctx_set_timing(thg_ctx ctx, int32_t enable) {
@@ -189,8 +280,11 @@ int thg_mesh_create(thg_ctx ctx, const float *verts, int64_t nv, const int32_t *
     m->nv = nv;
     m->nt = nt;
     hipMemcpyKind kind = mem == THG_MEM_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-    m->verts.alloc(nv * 3 * sizeof(float));
-    m->tris.alloc(nt * 3 * sizeof(int32_t));
+    Layout lay;
+    const size_t o_v = lay.add(nv * 3 * sizeof(float)), o_t = lay.add(nt * 3 * sizeof(int32_t));
+    m->store.alloc(lay.total);
+    m->verts.view(m->store.as<char>() + o_v, nv * 3 * sizeof(float));
+    m->tris.view(m->store.as<char>() + o_t, nt * 3 * sizeof(int32_t));
     if (nv) THG_HIP(hipMemcpy(m->verts.p, verts, nv * 3 * sizeof(float), kind));
     if (nt) {
       THG_HIP(hipMemcpy(m->tris.p, tris, nt * 3 * sizeof(int32_t), kind));

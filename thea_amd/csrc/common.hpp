@@ -47,38 +47,70 @@ inline void require(bool ok, const std::string &msg) {
   if (!ok) fail(THG_E_INVALID, msg);
 }
 
-// Owning device allocation.
+// Device memory blocks of DevBuf. A freed block is kept for the next allocation of about its size (at
+// least its request, at most a quarter more), up to DEV_CACHE_BYTES per device, oldest given back first;
+// all of a device's blocks are given back when one of its contexts is destroyed and before an
+// allocation is reported as failed. Like hipFree, dev_free waits for the device first, so a kept block
+// is idle and any stream or thread may take it.
+// Mapping and unmapping hundreds of megabytes for every mesh of a changing scene took 35 us per
+// hipMalloc and 170 us per hipFree at best, and from run to run 8 ms per build (the driver's share, in
+// whichever call came next).
+constexpr size_t DEV_CACHE_BYTES = (size_t)1 << 30;
+hipError_t dev_alloc(void **p, size_t n, size_t *block, int *device);
+void dev_free(void *p, size_t block, int device);
+void dev_cache_release(int device);
+
+// Owning device allocation, or a view into another one (view()).
 struct DevBuf {
   void *p = nullptr;
   size_t bytes = 0;
+  size_t block = 0;  // size of the owned block, 0 for a view
+  int device = 0;
   DevBuf() = default;
   explicit DevBuf(size_t n) { alloc(n); }
   DevBuf(const DevBuf &) = delete;
   DevBuf &operator=(const DevBuf &) = delete;
-  DevBuf(DevBuf &&o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; o.bytes = 0; }
+  DevBuf(DevBuf &&o) noexcept { take(o); }
   DevBuf &operator=(DevBuf &&o) noexcept {
-    if (this != &o) { reset(); p = o.p; bytes = o.bytes; o.p = nullptr; o.bytes = 0; }
+    if (this != &o) { reset(); take(o); }
     return *this;
   }
   ~DevBuf() { reset(); }
   void alloc(size_t n) {
     reset();
     if (n == 0) return;
-    hipError_t e = hipMalloc(&p, n);
+    const hipError_t e = dev_alloc(&p, n, &block, &device);
     if (e != hipSuccess) {
       p = nullptr;
+      block = 0;
       (void)hipGetLastError();
       fail(THG_E_OOM, "hipMalloc(" + std::to_string(n) + " bytes) failed: " + hipGetErrorString(e));
     }
     bytes = n;
   }
   void ensure(size_t n) { if (n > bytes) alloc(n); }
+  // n bytes at q, which belong to an allocation that outlives this object.
+  void view(void *q, size_t n) {
+    reset();
+    p = n ? q : nullptr;
+    bytes = n;
+  }
   void reset() {
-    if (p) (void)hipFree(p);
+    if (p && block) dev_free(p, block, device);
     p = nullptr;
-    bytes = 0;
+    bytes = block = 0;
   }
   template <typename T> T *as() const { return static_cast<T *>(p); }
+
+ private:
+  void take(DevBuf &o) {
+    p = o.p;
+    bytes = o.bytes;
+    block = o.block;
+    device = o.device;
+    o.p = nullptr;
+    o.bytes = o.block = 0;
+  }
 };
 
 // Stream-ordered device allocation (hipMallocAsync): freed on its stream, so the memory is reused
@@ -111,6 +143,36 @@ struct AsyncBuf {
     bytes = 0;
   }
   template <typename T> T *as() const { return static_cast<T *>(p); }
+};
+
+// Sizes of several arrays laid out in one allocation (each 256-byte aligned): add() every array, then
+// allocate total bytes and take base + the offsets it returned.
+struct Layout {
+  size_t total = 0;
+  size_t add(size_t n) {
+    const size_t o = total;
+    total += (n + 255) / 256 * 256;
+    return o;
+  }
+};
+
+// One allocation for a build's some 15 temporary arrays: up to WORKSPACE_POOL bytes from the device's
+// stream-ordered pool, more, which would stay in the pool, as a block of their own.
+constexpr size_t WORKSPACE_POOL = (size_t)256 << 20;
+struct Workspace {
+  AsyncBuf pooled;
+  DevBuf large;
+  char *base = nullptr;
+  void alloc(size_t n, hipStream_t s) {
+    if (n <= WORKSPACE_POOL) {
+      pooled.ensure(n, s);
+      base = pooled.as<char>();
+    } else {
+      large.alloc(n);
+      base = large.as<char>();
+    }
+  }
+  template <typename T> T *at(size_t o) const { return reinterpret_cast<T *>(base + o); }
 };
 
 // Host-memory staging for one call: inputs copied to device buffers, outputs written to device
@@ -189,6 +251,7 @@ struct KernelTimer {
 struct Mesh {
   Ctx *ctx = nullptr;
   int64_t nv = 0, nt = 0;
+  DevBuf store;          // the allocation verts and tris are views of
   DevBuf verts;          // float[3 nv]
   DevBuf tris;           // int32[3 nt]
   DevBuf area;           // float[nt], Thea's per-triangle area (Triangle3.hpp:154)
@@ -213,6 +276,7 @@ struct Bvh {
   int32_t child_order = 0;  // child visiting order of the compacted kernel (0: majority of lanes)
   float scale = 0;       // max |coordinate| over the elements
   float3 lo{}, hi{};     // scene bounds (element boxes)
+  DevBuf store;          // the allocation of the arrays over elements (views below)
   DevBuf nodes;          // BNode[num_nodes]
   DevBuf elems;          // TriRec[n] or PointRec[n], leaf order
   DevBuf rays;           // RayTri[n] (mesh BVHs), leaf order

@@ -141,7 +141,7 @@ const uint32_t *radix_sort_order(uint32_t *keys, uint32_t *vals, uint32_t *tmp_k
                                  hipStream_t s);
 // The same order with the sorted keys in `keys` and the positions in `vals`.
 void radix_sort_iota(uint32_t *keys, uint32_t *vals, uint32_t *tmp_keys, uint32_t *tmp_vals, uint32_t *hist,
-                     int64_t n, int begin_bit, int end_bit, hipStream_t s);
+                     int64_t n, int begin_bit, int end_bit, bool first_hist, hipStream_t s);
 size_t radix_hist_words(int64_t n);
 
 }  // namespace thg

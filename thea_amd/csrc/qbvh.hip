@@ -12,26 +12,6 @@ namespace thg {
 
 constexpr int QB_BLOCK = 256;
 
-__global__ void __launch_bounds__(QB_BLOCK) k_q_parents(const BNode *__restrict__ nodes, int64_t nn,
-                                                        int32_t *__restrict__ parent) {
-  const int64_t i = (int64_t)blockIdx.x * QB_BLOCK + threadIdx.x;
-  if (i >= nn) return;
-  if (i == 0) parent[0] = -1;
-  const int4 d = nodes[i].d;
-  if (d.x >= 0) parent[d.x] = (int32_t)i;
-  if (d.y >= 0) parent[d.y] = (int32_t)i;
-}
-
-// flag[i] = 1 for binary nodes at even depth (walking the parents up to the root).
-__global__ void __launch_bounds__(QB_BLOCK) k_q_flags(const int32_t *__restrict__ parent, int64_t nn,
-                                                      uint32_t *__restrict__ flag) {
-  const int64_t i = (int64_t)blockIdx.x * QB_BLOCK + threadIdx.x;
-  if (i >= nn) return;
-  int depth = 0;
-  for (int32_t p = parent[i]; p >= 0; p = parent[p]) ++depth;
-  flag[i] = (depth & 1) == 0 ? 1u : 0u;
-}
-
 // Smallest power-of-two exponent e (within the normal range) with fmaf(255, 2^e, lo) >= hi.
 __device__ int q_exponent(float lo, float hi) {
   const double E = (double)hi - (double)lo;
@@ -140,26 +120,15 @@ __global__ void __launch_bounds__(QB_BLOCK) k_q_emit(const BNode *__restrict__ n
   out[qidx[i]] = q;
 }
 
-void build_qbvh4(Bvh &b, hipStream_t s) {
+void build_qbvh4(Bvh &b, const uint32_t *even, const uint32_t *qidx, int64_t nq, hipStream_t s) {
   const int64_t nn = b.num_nodes;
   if (nn <= 0) return;
   // Leaf counts are kept in 16 bits (leaves hold at most leaf_size elements).
   require(b.leaf_size <= 65535, "leaf size too large for the ray tree");
-  DevBuf parent(nn * 4), flag(nn * 4), qidx((nn + 1) * 4), tmp(scan_tmp_words(nn) * 4);
-  const uint32_t grid = ceil_div(nn, QB_BLOCK);
-  hipLaunchKernelGGL(k_q_parents, dim3(grid), dim3(QB_BLOCK), 0, s, b.nodes.as<BNode>(), nn, parent.as<int32_t>());
-  launch_check("k_q_parents");
-  hipLaunchKernelGGL(k_q_flags, dim3(grid), dim3(QB_BLOCK), 0, s, parent.as<int32_t>(), nn, flag.as<uint32_t>());
-  launch_check("k_q_flags");
-  scan_excl_u32(flag.as<uint32_t>(), qidx.as<uint32_t>(), nn, tmp.as<uint32_t>(), s);
-  uint32_t nq = 0;
-  THG_HIP(hipMemcpyAsync(&nq, qidx.as<uint32_t>() + nn, 4, hipMemcpyDeviceToHost, s));
-  THG_HIP(hipStreamSynchronize(s));
   b.qnodes.alloc((size_t)nq * sizeof(QNode4));
-  hipLaunchKernelGGL(k_q_emit, dim3(grid), dim3(QB_BLOCK), 0, s, b.nodes.as<BNode>(), nn, flag.as<uint32_t>(),
-                     qidx.as<uint32_t>(), b.qnodes.as<QNode4>());
+  hipLaunchKernelGGL(k_q_emit, dim3(ceil_div(nn, QB_BLOCK)), dim3(QB_BLOCK), 0, s, b.nodes.as<BNode>(), nn, even, qidx,
+                     b.qnodes.as<QNode4>());
   launch_check("k_q_emit");
-  THG_HIP(hipStreamSynchronize(s));
   b.num_qnodes = nq;
   // Binary internal levels d = 0 .. max_depth - 1 fold into levels 0, 2, 4, ...
   b.q_depth = b.max_depth / 2 + 1;

@@ -73,8 +73,9 @@ size_t sort_scratch_words(int64_t cap);
 // [0, nv); synchronises `s`.
 void check_tri_indices(const int32_t *tris, int64_t nt, int64_t nv, hipStream_t s);
 void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool points, int leaf_size, hipStream_t s);
-// The 4-wide quantized ray tree (Bvh::qnodes) of a built mesh BVH; synchronises `s`.
-void build_qbvh4(Bvh &b, hipStream_t s);
+// The 4-wide quantized ray tree (Bvh::qnodes) of a built mesh BVH: even[i] = 1 for the nodes at even
+// depth, which become its nq nodes, qidx its exclusive scan.
+void build_qbvh4(Bvh &b, const uint32_t *even, const uint32_t *qidx, int64_t nq, hipStream_t s);
 int order_bits_lo(int64_t n);
 void order_queries(const Bvh &b, const float *q, int64_t n, QueryScratch &ws, hipStream_t s);
 void order_rays(const Bvh &b, const float *o, const float *d, int64_t n, QueryScratch &ws, hipStream_t s);
@@ -84,23 +85,29 @@ void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, 
 // Build-pipeline pieces reused by the batched many-mesh plan (batch.hip).
 // Leaf bounds of a mesh BVH's leaves into out[first record of each leaf]: nodes [0, nsmall + *kept)
 // (kept null: none beyond nsmall), at most max_nodes.
-void launch_screen_records(const TriRec *tr, int64_t n, ScreenRec *out, hipStream_t s);
 void launch_leaf_bounds(const BNode *nodes, int64_t nsmall, const uint32_t *kept, int64_t max_nodes, const TriRec *tr,
                         LeafBound *out, hipStream_t s);
-// Words of the refit's per-span entry counts (and level-list lengths) for n elements, and whether
-// the refit of n elements needs its n-word level list.
-size_t refit_count_words(int64_t n);
-bool refit_needs_list(int64_t n);
-void launch_refit(int64_t n, const uint32_t *sorted, const float4 *blo, const float4 *bhi, const int32_t *left,
-                  const int32_t *right, const int32_t *rfirst, const int32_t *rlast, const int32_t *nparent,
-                  const int32_t *lparent, uint32_t *flags, float *nbox, int32_t *entries, uint32_t *nentries,
-                  int32_t *list, hipStream_t s);
-void launch_emit(int64_t ni, int32_t base, const uint32_t *keep, const uint32_t *fidx, const int32_t *left,
-                 const int32_t *right, const int32_t *rfirst, const int32_t *rlast, const uint32_t *sorted,
-                 const float4 *blo, const float4 *bhi, const float *nbox, BNode *out, uint32_t *leaf_count,
+// The boxes of every aligned run of 2^L sorted elements, L = 0 .. top: run i of level L at
+// box[2 (off[L] + i)] (low corner) and the next (high corner). Runs cut short by n are stored but are
+// never part of a range.
+struct BoxLevels {
+  float4 *box;
+  int64_t n;
+  int64_t off[33];
+  int top;
+  __host__ __device__ int64_t count(int L) const { return (n + ((int64_t)1 << L) - 1) >> L; }
+};
+BoxLevels box_levels(int64_t n, float4 *box);
+int64_t box_level_entries(int64_t n);
+// Levels 9 and up, from level 8 (the record kernels store levels 0 to 8).
+void launch_pyramid_top(const BoxLevels &P, hipStream_t s);
+// Compacted nodes of the kept internal nodes (k_emit); parent[] of every non-root compacted node.
+void launch_emit(int64_t ni, int32_t base, const uint32_t *keep, const uint32_t *fidx, const int32_t *rfirst,
+                 const int32_t *rlast, const uint32_t *split, const BoxLevels &P, BNode *out, int32_t *parent,
                  hipStream_t s);
-void launch_depth(int64_t n, const int32_t *lparent, const int32_t *nparent, const uint32_t *keep, const int32_t *rfirst,
-                  int32_t *max_depth, hipStream_t s);
+// *max_depth = max(*max_depth, levels) over nodes [first, first + *count); even: see k_node_depth.
+void launch_node_depth(int64_t max_nodes, int64_t first, const uint32_t *count, const int32_t *parent,
+                       int32_t *max_depth, uint32_t *even, hipStream_t s);
 // Exclusive scan of n words: out must hold n + 1 words (the total lands in out[n]) and tmp
 // scan_tmp_words(n) words.
 size_t scan_tmp_words(int64_t n);

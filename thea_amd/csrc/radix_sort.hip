@@ -198,9 +198,9 @@ const uint32_t *radix_sort_order(uint32_t *keys, uint32_t *vals, uint32_t *tmp_k
 }
 
 void radix_sort_iota(uint32_t *keys, uint32_t *vals, uint32_t *tmp_keys, uint32_t *tmp_vals, uint32_t *hist,
-                     int64_t n, int begin_bit, int end_bit, hipStream_t s) {
+                     int64_t n, int begin_bit, int end_bit, bool first_hist, hipStream_t s) {
   const RadixResult r =
-      radix_sort_passes(keys, vals, tmp_keys, tmp_vals, hist, n, begin_bit, end_bit, true, true, false, s);
+      radix_sort_passes(keys, vals, tmp_keys, tmp_vals, hist, n, begin_bit, end_bit, true, true, first_hist, s);
   if (r.vals != vals) {
     THG_HIP(hipMemcpyAsync(keys, r.keys, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     THG_HIP(hipMemcpyAsync(vals, r.vals, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
