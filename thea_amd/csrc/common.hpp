@@ -256,6 +256,8 @@ struct Mesh {
   DevBuf tris;           // int32[3 nt]
   DevBuf area;           // float[nt], Thea's per-triangle area (Triangle3.hpp:154)
   DevBuf cdf;            // double[nt], prefix sums of area in triangle order (lazy)
+  DevBuf guide;          // uint32[2^guide_bits + 1]: see k_guide (built with cdf)
+  int guide_bits = 0;
   bool cdf_ready = false;
   bool cdf_exact_scan = false;  // CDF built by the parallel exact scan (else sequentially)
   double total_area = 0;

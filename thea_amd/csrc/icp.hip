@@ -82,6 +82,16 @@ __global__ void __launch_bounds__(256) k_icp_pos(int64_t n, int A, const int32_t
   pos[3 * i + 2] = (T)z;
 }
 
+// q[prob[s] n + j] = tmp[s n + j]: the correspondences of a launch over part of the problems.
+template <typename T>
+__global__ void __launch_bounds__(256) k_icp_place(int64_t n, int A, const int32_t *__restrict__ prob,
+                                                   const T *__restrict__ tmp, T *__restrict__ q) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= 3 * n * A) return;
+  const int64_t s = i / (3 * n);
+  q[3 * n * prob[s] + (i - s * 3 * n)] = tmp[i];
+}
+
 // Sums over the points of each active problem, with q the correspondences by problem (q[k n + j]).
 // MODE 0: wt p (3), wt q (3), wt (1). MODE 1: the cross-covariance sum of (wr dp)(wr dq)^T with the
 // up component removed (9). MODE 2: wr^2 |L dp - dq|^2 (1). aux (12 per problem): up in [0..2] and
@@ -340,12 +350,14 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
   const int nb = (int)((n + ICP_CHUNK - 1) / ICP_CHUNK);
   AsyncBuf src(n * K * 24, s), cur(K * 96, s), aux(K * 96, s), sums7(K * 56, s), cov(K * 72, s), errs(K * 8, s);
   // qpts: the correspondences of problem k at [k n, (k + 1) n) (kept across iterations whatever the
-  // active set); qtmp: the nearest points of one launch, by slot
+  // active set); qtmp: the nearest points of one launch over part of the problems, by slot. While every
+  // problem is active the launch writes qpts itself (a copy per problem and launch took 0.6 ms of device
+  // time and as much of launches in a 24-problem search of 60,000 points).
   // A double point BVH (BvhN<Vector3d>, ShapeAlign.cpp:339) is searched in double with the positions
   // kept in double; a float BVH with the positions rounded to float.
   const bool f64 = to.f64;
   const int64_t pb = f64 ? 24 : 12;  // bytes per position / correspondence
-  AsyncBuf pos(n * K * pb, s), qpts(n * K * pb, s), qtmp(n * K * pb, s), idx(n * K * 4, s), prob(K * 4, s);
+  AsyncBuf pos(n * K * pb, s), qpts(n * K * pb, s), qtmp, idx(n * K * 4, s), prob(K * 4, s);
   AsyncBuf partial((size_t)K * nb * ICP_MAXC * 8, s);
   hipLaunchKernelGGL(k_icp_init, dim3(ceil_div(n * K, 256)), dim3(256), 0, s, n, K, from, init, src.as<double>());
   launch_check("k_icp_init");
@@ -366,24 +378,34 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
     if (!active.empty())
       THG_HIP(hipMemcpyAsync(prob.p, active.data(), 4 * active.size(), hipMemcpyHostToDevice, s));
   };
+  QueryScratch ws;  // sort memory of the nearest-point launches
   // nearest points of the active problems' current positions
   auto nearest = [&]() {
     const int A = (int)active.size();
-    QueryScratch ws;
+    const bool all = A == K;
+    if (!all) qtmp.ensure(n * K * pb, s);
+    void *out = all ? qpts.p : qtmp.p;
     if (f64) {
       hipLaunchKernelGGL(k_icp_pos<double>, dim3(ceil_div(n * A, 256)), dim3(256), 0, s, n, A, prob.as<int32_t>(),
                          src.as<double>(), cur.as<double>(), pos.as<double>());
       launch_check("k_icp_pos");
-      launch_closest64(to, pos.as<double>(), n * A, -1.0, idx.as<int32_t>(), qtmp.as<double>(), nullptr, nullptr, ws, s);
+      launch_closest64(to, pos.as<double>(), n * A, -1.0, idx.as<int32_t>(), (double *)out, nullptr, nullptr, ws, s);
     } else {
       hipLaunchKernelGGL(k_icp_pos<float>, dim3(ceil_div(n * A, 256)), dim3(256), 0, s, n, A, prob.as<int32_t>(),
                          src.as<double>(), cur.as<double>(), pos.as<float>());
       launch_check("k_icp_pos");
-      launch_closest(to, pos.as<float>(), n * A, -1.0, 0, idx.as<int32_t>(), qtmp.as<float>(), nullptr, nullptr, ws, s);
+      launch_closest(to, pos.as<float>(), n * A, -1.0, 0, idx.as<int32_t>(), (float *)out, nullptr, nullptr, ws, s);
     }
-    for (int sl = 0; sl < A; ++sl)
-      THG_HIP(hipMemcpyAsync((char *)qpts.p + pb * (int64_t)active[sl] * n, (char *)qtmp.p + pb * (int64_t)sl * n, n * pb,
-                             hipMemcpyDeviceToDevice, s));
+    if (!all) {
+      const dim3 g(ceil_div(3 * n * A, 256));
+      if (f64)
+        hipLaunchKernelGGL(k_icp_place<double>, g, dim3(256), 0, s, n, A, prob.as<int32_t>(), qtmp.as<double>(),
+                           qpts.as<double>());
+      else
+        hipLaunchKernelGGL(k_icp_place<float>, g, dim3(256), 0, s, n, A, prob.as<int32_t>(), qtmp.as<float>(),
+                           qpts.as<float>());
+      launch_check("k_icp_place");
+    }
   };
   auto sums = [&](int mode, double *dst, int stride) {
     const int A = (int)active.size();

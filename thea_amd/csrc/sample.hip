@@ -6,8 +6,11 @@
 //                every partial sum is exactly representable (all areas are multiples of the smallest
 //                area ulp 2^e and n * max area < 2^(e + 53)) any association gives the same bits,
 //                so a parallel scan is used; otherwise a single lane sums in order.
+//  k_guide       first CDF entry each of 2^b equal ranges of the 32-bit random word can reach, made
+//                with the CDF.
 //  k_sample      per sample: Philox4x32-10 words -> uniform01 (Random.hpp:126-131) -> lower_bound
-//                over the CDF, clamped to the last triangle -> reflected barycentric point.
+//                over the CDF between its range's two guide entries, clamped to the last triangle ->
+//                reflected barycentric point.
 #include "kernels_common.hpp"
 #include "philox.hpp"
 #include "query.hpp"
@@ -134,6 +137,30 @@ __global__ void k_dscan_seq(const float *__restrict__ a, int64_t n, double *__re
   for (; i < n; ++i) { c += (double)a[i]; cdf[i] = c; }
 }
 
+// std::lower_bound over cdf[first, first + count): the first c with !(cdf[c] < t).
+__device__ __forceinline__ int64_t cdf_lower(const double *__restrict__ cdf, int64_t first, int64_t count, double t) {
+  while (count > 0) {
+    const int64_t step = count >> 1, mid = first + step;
+    if (cdf[mid] < t) { first = mid + 1; count -= step + 1; }
+    else count = step;
+  }
+  return first;
+}
+
+// guide[j] = lower_bound of the target of word j << (32 - bits), guide[2^bits] = nt. The target
+// u01(word) * total never decreases with the word, so a word w of range j = w >> (32 - bits) finds its
+// lower_bound in [guide[j], guide[j + 1]]: the same triangle as a search of the whole CDF.
+__global__ void __launch_bounds__(S_BLOCK) k_guide(const double *__restrict__ cdf, int64_t nt, double total, int bits,
+                                                   uint32_t *__restrict__ guide) {
+  const int64_t j = (int64_t)blockIdx.x * S_BLOCK + threadIdx.x;
+  const int64_t n = (int64_t)1 << bits;
+  if (j > n) return;
+  guide[j] = j == n ? (uint32_t)nt : (uint32_t)cdf_lower(cdf, 0, nt, (double)u01((uint32_t)j << (32 - bits)) * total);
+}
+
+// About one range per triangle: a sample then reads two or three CDF entries instead of log2(nt).
+constexpr int GUIDE_MIN_BITS = 8, GUIDE_MAX_BITS = 22;
+
 void mesh_cdf(Mesh &m, hipStream_t s) {
   std::lock_guard<std::mutex> g(m.cdf_lock);
   if (m.cdf_ready) return;
@@ -176,12 +203,21 @@ void mesh_cdf(Mesh &m, hipStream_t s) {
   THG_HIP(hipMemcpyAsync(&total, m.cdf.as<double>() + (m.nt - 1), sizeof(double), hipMemcpyDeviceToHost, s));
   THG_HIP(hipStreamSynchronize(s));
   m.total_area = total;
+  m.guide_bits = GUIDE_MIN_BITS;
+  while (m.guide_bits < GUIDE_MAX_BITS && ((int64_t)1 << m.guide_bits) < m.nt) ++m.guide_bits;
+  m.guide.alloc((((size_t)1 << m.guide_bits) + 1) * 4);
+  hipLaunchKernelGGL(k_guide, dim3(ceil_div(((uint64_t)1 << m.guide_bits) + 1, S_BLOCK)), dim3(S_BLOCK), 0, s,
+                     m.cdf.as<double>(), m.nt, total, m.guide_bits, m.guide.as<uint32_t>());
+  launch_check("k_guide");
+  THG_HIP(hipStreamSynchronize(s));
   m.cdf_exact_scan = exact;
   m.cdf_ready = true;
 }
 
+// SAMPLE_NOTE
 __global__ void __launch_bounds__(S_BLOCK) k_sample(const float *__restrict__ verts, const int32_t *__restrict__ tris,
-                                                    const double *__restrict__ cdf, int64_t nt, double total, int64_t n,
+                                                    const double *__restrict__ cdf, const uint32_t *__restrict__ guide,
+                                                    int guide_bits, int64_t nt, double total, int64_t n,
                                                     uint32_t k0, uint32_t k1, uint32_t s0, uint32_t s1,
                                                     float *__restrict__ pos, float *__restrict__ nrm,
                                                     int32_t *__restrict__ tri_out) {
@@ -189,14 +225,9 @@ __global__ void __launch_bounds__(S_BLOCK) k_sample(const float *__restrict__ ve
   if (i >= n) return;
   uint32_t w[4];
   philox4x32_10((uint32_t)i, (uint32_t)((uint64_t)i >> 32), s0, s1, k0, k1, w);
-  double t = (double)u01(w[0]) * total;
-  // std::lower_bound: first c with !(cdf[c] < t)
-  int64_t first = 0, count = nt;
-  while (count > 0) {
-    int64_t step = count >> 1, mid = first + step;
-    if (cdf[mid] < t) { first = mid + 1; count -= step + 1; }
-    else count = step;
-  }
+  const uint32_t *g = guide + (w[0] >> (32 - guide_bits));
+  const int64_t lo = g[0], hi = g[1];
+  const int64_t first = cdf_lower(cdf, lo, hi - lo, (double)u01(w[0]) * total);
   int64_t ti = first < nt - 1 ? first : nt - 1;
   float3 v0 = vtx(verts, tris[3 * ti]), v1 = vtx(verts, tris[3 * ti + 1]), v2 = vtx(verts, tris[3 * ti + 2]);
   float3 e01 = sub3(v1, v0), e02 = sub3(v2, v0);
@@ -310,7 +341,7 @@ void launch_sample(Mesh &m, int64_t n, uint64_t seed, uint64_t stream_id, float 
   if (n <= 0 || m.nt <= 0 || !(m.total_area > 0)) return;
   KernelTimer kt(m.ctx, s, "sample");
   hipLaunchKernelGGL(k_sample, dim3(ceil_div(n, S_BLOCK)), dim3(S_BLOCK), 0, s, m.verts.as<float>(), m.tris.as<int32_t>(),
-                     m.cdf.as<double>(), m.nt, m.total_area, n, (uint32_t)seed, (uint32_t)(seed >> 32),
+                     m.cdf.as<double>(), m.guide.as<uint32_t>(), m.guide_bits, m.nt, m.total_area, n, (uint32_t)seed, (uint32_t)(seed >> 32),
                      (uint32_t)stream_id, (uint32_t)(stream_id >> 32), pos, nrm, tri);
   launch_check("k_sample");
   kt.stop();
