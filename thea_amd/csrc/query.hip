@@ -1,9 +1,10 @@
 // Query kernels: closest element / closest point, k nearest, ray first hit and any hit.
 //
-// One query per lane; each lane walks the BVH depth first with its own stack in LDS (node ref and
-// the lower bound it was pushed with), visiting the nearer child first. Queries are first put in
-// spatial (Morton) order so the 64 lanes of a wave walk nearby paths; blocks are remapped so each
-// XCD's L2 serves one contiguous spatial range. Results go to the caller's query index.
+// Rays, sparse and small batches take the work-queue kernels (a wave keeps the (query, node) pairs of
+// its queries on one LDS stack and steps through 64 of them at a time); dense batches of point queries,
+// put in spatial (Morton) order first, take one tree walk per wave; trees too deep for either take one
+// query per lane with a stack in LDS. Blocks are remapped so each XCD's L2 serves one contiguous range
+// of queries. Results go to the caller's query index.
 //
 // Results are defined canonically: the lexicographic minimum of (float d^2, element index) for
 // closest queries (and the k smallest such pairs for k-NN), (float t, element index) for rays,
@@ -2256,203 +2257,284 @@ __device__ __forceinline__ bool raytri_last(const float4 &b) { return __float_as
 // Node reference that ends a lane's traversal (~RAY_DONE would be leaf INT32_MAX: never a real one).
 constexpr int32_t RAY_DONE = INT32_MIN;
 
-// Rays over the 4-wide quantized tree (QNode4), one per lane, in while-while form (Aila and Laine,
-// "Understanding the efficiency of ray traversal on GPUs", HPG 2009): a lane walks inner nodes,
-// postponing the first leaf it meets, and the wave runs its leaf tests together once every lane
-// still walking holds one. Leaves are node references like inner nodes (on the stack too), and a
-// leaf's triangles run up to the record flagged as its last (RayTri::b.w). Results do not depend on
-// the visiting order: a ray's answer is the least (t, index) over the triangles it tests, and a box
-// is skipped only when it cannot hold that.
-// A node's four child boxes are decoded only on the ray's near and far planes per axis (the
-// direction's sign picks qlo or qhi). Fast form, when every direction component of the wave's rays
-// has |1/d| <= 2^40 and the scene is below 2^60: t = fmaf(q, 2^e / d, (origin - o') / d), whose
-// error is below 2^-19 of max(scale, |o|), inside the 2^-16 widening. Otherwise the wave decodes
-// each plane with the build's own fmaf and intersects it as k_ray does, so rays parallel to an axis
-// keep IEEE infinities. The traversal stack holds LST entries per lane in LDS and OVF more in
-// private memory; the host picks OVF so that LST + OVF covers three entries per QNode4 level.
 __device__ __forceinline__ float q_byte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xffu); }
 
 // Scenes at or beyond 2^60 take the decoding form (the fast form's terms could overflow).
 __host__ __device__ __forceinline__ int q4_exact_only(float scale) { return scale < 1.152921504606846976e18f ? 0 : 1; }
 
-template <bool ANY, int LST, int OVF, bool POST>
-__device__ __forceinline__ void ray_q4_body(int32_t *__restrict__ s_ref, const QNode4 *__restrict__ qn,
-                                            const RayTri *__restrict__ rt, const TriRec *__restrict__ tr,
-                                            const float *__restrict__ orig, const float *__restrict__ dirs,
-                                            int64_t ri, float best_init, float max_time, float scale,
-                                            int exact_only, int32_t *__restrict__ out_idx,
-                                            float *__restrict__ out_t, float *__restrict__ out_n,
-                                            uint8_t *__restrict__ out_any) {
-  int32_t ovf[OVF];
-  const int tid = threadIdx.x;
+//--------------------------------------------------------------------------------------------------
+// Rays over the 4-wide quantized tree (QNode4), by work queue
+//
+// A vector load costs the data path 16 cycles per instruction and wave whatever its active lanes, and
+// the longest ray of a wave of per-lane walks sets its time. So a wave keeps the (ray, node) pairs of its
+// 64 >> lg rays on one LDS stack: each step pops up to 64 pairs, whichever rays they belong to, loads
+// 64 nodes and pushes the children the rays enter, the nearest last; leaves (node references like inner
+// nodes, their triangles up to the record flagged as the last, RayTri::b.w) collect in a list and are
+// tested one per lane, 64 at a time. A ray begins when the stack holds less than a step's pairs. A pair
+// whose entry time (16 bits, rounded down) lies beyond its ray's best hit drops out when popped. 10 KB of
+// LDS per wave: 16 resident waves. Results do not depend on the order: a ray's answer is the least
+// (t, index) over the triangles it tests, and a box is skipped only when it cannot hold that.
+// Against one ray per lane of a sorted batch (us, first hit / any hit within 0.7; torus of 1,048,576
+// triangles, leaves of 2): 4,000,000 rays 1,526 -> 741 / 1,897 -> 1,058; 100,000 384 -> 48 / 521 -> 59; 100
+// 54 -> 23 / 102 -> 22; rough sphere of 1,000,000: 4,000,000 rays 3,590 -> 2,196, 100,000 796 -> 104.
+//
+// A node's four child boxes are decoded only on the ray's near and far planes per axis (the
+// direction's sign picks qlo or qhi). Fast form, when every direction component of the wave's rays
+// has |1/d| <= 2^40 and the scene is below 2^60: t = fmaf(q, 2^e / d, (origin - o') / d), whose
+// error is below 2^-19 of max(scale, |o|), inside the 2^-16 widening. Otherwise the wave decodes
+// each plane with the build's own fmaf and intersects it as k_ray does, so rays parallel to an axis
+// keep IEEE infinities.
+//--------------------------------------------------------------------------------------------------
+// The stack takes steps of 64 pairs while it has room for their children; nearer its end, fewer, down to
+// one pair, whose walk adds at most three entries per level (Q4_MAX_STACK).
+constexpr int RQ_STACK = 752;
+constexpr int RQ_LEAVES = 5 * WAVE;
+
+struct RayWave {
+  float4 ow[WAVE];               // origin, slack half-width
+  float4 iv[WAVE];               // 1 / direction, direction x
+  float2 dyz[WAVE];              // direction y, z
+  unsigned long long key[WAVE];  // best hit (t bits << 32 | id)
+  int32_t slot[WAVE];            // its RayTri
+  int32_t ref[RQ_STACK];         // stack: node, entry time, ray
+  int32_t leaf[RQ_LEAVES];       // met leaves, ray
+  uint16_t t[RQ_STACK];
+  uint8_t own[RQ_STACK], lown[RQ_LEAVES];
+};
+static_assert(sizeof(RayWave) <= 10240, "16 waves per CU (160 KB of LDS)");
+
+template <bool ANY>
+__device__ __forceinline__ void ray_queue_body(RayWave &W, const QNode4 *__restrict__ qn,
+                                               const RayTri *__restrict__ rt, const TriRec *__restrict__ tr,
+                                               const float *__restrict__ orig, const float *__restrict__ dirs,
+                                               const uint32_t *__restrict__ order, int64_t n, int64_t wave, int lg,
+                                               float best_init, float max_time, float scale, int exact_only,
+                                               int32_t *__restrict__ out_idx, float *__restrict__ out_t,
+                                               float *__restrict__ out_n, uint8_t *__restrict__ out_any) {
+  const int lane = lane_id();
   const float REL = 1.0f + 1.0f / 4096.0f;
-  RayLane L;
-  ray_lane_init(L, orig, dirs, ri, best_init, scale);
-  const bool px = L.inv.x >= 0.0f, py = L.inv.y >= 0.0f, pz = L.inv.z >= 0.0f;
-  const float3 on = f3(px ? L.olo.x : L.ohi.x, py ? L.olo.y : L.ohi.y, pz ? L.olo.z : L.ohi.z);
-  const float3 of = f3(px ? L.ohi.x : L.olo.x, py ? L.ohi.y : L.olo.y, pz ? L.ohi.z : L.olo.z);
   const float INV_MAX = 1099511627776.0f;  // 2^40
-  const bool lane_fast = fabsf(L.inv.x) <= INV_MAX && fabsf(L.inv.y) <= INV_MAX && fabsf(L.inv.z) <= INV_MAX;
-  const bool fast = !exact_only && __ballot(!lane_fast) == 0;
-  int sp = 0;
-  auto push = [&](int32_t v) {
-    if (sp < LST) s_ref[sp * Q_BLOCK + tid] = v;
-    else if (sp < LST + OVF) ovf[sp - LST] = v;
-    else return;  // never taken: LST + OVF covers the deepest path
-    ++sp;
-  };
-  auto pop = [&]() -> int32_t {
-    if (sp == 0) return RAY_DONE;
-    --sp;
-    return sp < LST ? s_ref[sp * Q_BLOCK + tid] : ovf[sp - LST];
-  };
-  // The triangles of leaf lf; true when an any-hit query has its answer.
-  auto run_leaf = [&](int32_t lf) -> bool {
-    int32_t k = ~lf;
-    bool last;
-    do {
-      const RayTri *t = rt + k;
-      const float4 a = t->a, b = t->b, c = t->c;
-      last = raytri_last(b);
-      const float th = tri_ray_e(f3(a.x, a.y, a.z), f3(b.x, b.y, b.z), f3(c.x, c.y, c.z), L.o, L.d, max_time);
-      if (th >= 0) {
-        const int32_t id = __float_as_int(a.w);
-        if (better(th, id, L.best, L.bidx)) {
-          L.best = th;
-          L.bidx = id;
-          L.bslot = k;
-          if (ANY) return true;
+  const int Q = WAVE >> lg;
+  const int64_t t = wave * Q + lane;
+  const bool inrange = lane < Q && t < n;
+  int64_t ri = 0;
+  float3 o = f3(0, 0, 0), d = f3(0, 0, 0);
+  if (inrange) {
+    ri = order ? (int64_t)order[t] : t;
+    o = load_q(orig, ri);
+    d = load_q(dirs, ri);
+  }
+  const float3 inv = f3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+  const float m = fmaxf(scale, fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))));
+  W.ow[lane] = make_float4(o.x, o.y, o.z, m * SLACK_REL);
+  W.iv[lane] = make_float4(inv.x, inv.y, inv.z, d.x);
+  W.dyz[lane] = make_float2(d.y, d.z);
+  W.key[lane] = cmp_key(best_init, 0x7fffffff);
+  const bool slow = !(fabsf(inv.x) <= INV_MAX && fabsf(inv.y) <= INV_MAX && fabsf(inv.z) <= INV_MAX);
+  const bool fast = !exact_only && ballot(inrange && slow) == 0;
+  uint64_t todo = ballot(inrange && best_init >= 0.0f);  // rays whose walk has not begun
+  int sp = 0, ln = 0;
+  __builtin_amdgcn_wave_barrier();
+  while (true) {
+    if (sp < WAVE && todo != 0) {
+      const int rank = __popcll(todo & lanemask_lt());
+      const bool take = ((todo >> lane) & 1) && sp + rank < WAVE;
+      if (take) {
+        W.ref[sp + rank] = 0;
+        W.t[sp + rank] = 0;
+        W.own[sp + rank] = (uint8_t)lane;
+      }
+      const uint64_t tm = ballot(take);
+      todo &= ~tm;
+      sp += __popcll(tm);
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (ln >= WAVE || (sp == 0 && ln > 0)) {
+      // the triangles of up to 64 leaves, one leaf per lane
+      const int k = ln < WAVE ? ln : WAVE;
+      ln -= k;
+      if (lane < k) {
+        const int r = W.lown[ln + lane];
+        const unsigned long long key0 = W.key[r];
+        if (!ANY || (key0 >> 63) == 0) {
+          int32_t e = ~W.leaf[ln + lane];
+          const float4 ow = W.ow[r];
+          const float2 dyz = W.dyz[r];
+          const float3 ro = f3(ow.x, ow.y, ow.z), rd = f3(W.iv[r].w, dyz.x, dyz.y);
+          unsigned long long best = key0;
+          int32_t bslot = -1;
+          bool last;
+          do {
+            const RayTri *tp = rt + e;
+            const float4 a = tp->a, b = tp->b, c = tp->c;
+            last = raytri_last(b);
+            const float th = tri_ray_e(f3(a.x, a.y, a.z), f3(b.x, b.y, b.z), f3(c.x, c.y, c.z), ro, rd, max_time);
+            if (th >= 0) {
+              const unsigned long long kk = cmp_key(th, __float_as_int(a.w));
+              if (kk < best) { best = kk; bslot = e; }
+            }
+            ++e;
+          } while (!last && !(ANY && bslot >= 0));
+          if (bslot >= 0) {
+            if (ANY) {
+              W.key[r] = ~0ull;  // negative bound: the ray's other pairs drop out
+            } else {
+              atomicMin(&W.key[r], best);
+              __builtin_amdgcn_wave_barrier();
+              if (W.key[r] == best) W.slot[r] = bslot;
+            }
+          }
         }
       }
-      ++k;
-    } while (!last);
-    return false;
-  };
-  int32_t node = 0;
-  int32_t leaf = 0;
-  while (node != RAY_DONE || leaf < 0) {
-    while (node >= 0) {
-      const QNode4 *np = qn + node;
-      const float4 na = np->a;
-      const uint4 nb4 = np->b;
-      const int4 nc4 = np->c;
-      const int2 nd2 = *reinterpret_cast<const int2 *>(&np->d);
-      const uint32_t meta = __float_as_uint(na.w);
-      const int nc = (int)(meta >> 24);
-      const float3 sc = f3(__uint_as_float((meta & 0xffu) << 23), __uint_as_float(((meta >> 8) & 0xffu) << 23),
-                           __uint_as_float(((meta >> 16) & 0xffu) << 23));
-      const uint32_t qhy = (uint32_t)nc4.x, qhz = (uint32_t)nc4.y;
-      const uint32_t qnx = px ? nb4.x : nb4.w, qfx = px ? nb4.w : nb4.x;
-      const uint32_t qny = py ? nb4.y : qhy, qfy = py ? qhy : nb4.y;
-      const uint32_t qnz = pz ? nb4.z : qhz, qfz = pz ? qhz : nb4.z;
-      const float lim = L.best * REL;
-      float key[4];
-      int32_t r[4] = {nc4.z, nc4.w, nd2.x, nd2.y};
-      int h = 0;
-      if (fast) {
-        const float3 A = f3(sc.x * L.inv.x, sc.y * L.inv.y, sc.z * L.inv.z);
-        const float3 Bn = f3((na.x - on.x) * L.inv.x, (na.y - on.y) * L.inv.y, (na.z - on.z) * L.inv.z);
-        const float3 Bf = f3((na.x - of.x) * L.inv.x, (na.y - of.y) * L.inv.y, (na.z - of.z) * L.inv.z);
+    } else if (sp > 0) {
+      const int room = (RQ_STACK - Q4_MAX_STACK - sp) >> 2;
+      int k = sp < WAVE ? sp : WAVE;
+      k = k < room ? k : (room > 1 ? room : 1);
+      float key[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+      int32_t ref[4] = {0, 0, 0, 0};
+      int r = 0;
+      if (lane < k) {
+        const int e = sp - 1 - lane;
+        r = W.own[e];
+        const float lim = cmp_key_d(W.key[r]) * REL;
+        if (lb_unpack(W.t[e]) <= lim) {
+          const QNode4 *np = qn + W.ref[e];
+          const float4 na = np->a;
+          const uint4 nb4 = np->b;
+          const int4 nc4 = np->c;
+          const int2 nd2 = *reinterpret_cast<const int2 *>(&np->d);
+          const float4 ow = W.ow[r], iv = W.iv[r];
+          const bool px = iv.x >= 0.0f, py = iv.y >= 0.0f, pz = iv.z >= 0.0f;
+          // near planes are widened backwards, far planes forwards
+          const float3 on = f3(px ? ow.x + ow.w : ow.x - ow.w, py ? ow.y + ow.w : ow.y - ow.w,
+                               pz ? ow.z + ow.w : ow.z - ow.w);
+          const float3 of = f3(px ? ow.x - ow.w : ow.x + ow.w, py ? ow.y - ow.w : ow.y + ow.w,
+                               pz ? ow.z - ow.w : ow.z + ow.w);
+          const uint32_t meta = __float_as_uint(na.w);
+          const int nc = (int)(meta >> 24);
+          const float3 sc = f3(__uint_as_float((meta & 0xffu) << 23), __uint_as_float(((meta >> 8) & 0xffu) << 23),
+                               __uint_as_float(((meta >> 16) & 0xffu) << 23));
+          const uint32_t qhy = (uint32_t)nc4.x, qhz = (uint32_t)nc4.y;
+          const uint32_t qnx = px ? nb4.x : nb4.w, qfx = px ? nb4.w : nb4.x;
+          const uint32_t qny = py ? nb4.y : qhy, qfy = py ? qhy : nb4.y;
+          const uint32_t qnz = pz ? nb4.z : qhz, qfz = pz ? qhz : nb4.z;
+          ref[0] = nc4.z, ref[1] = nc4.w, ref[2] = nd2.x, ref[3] = nd2.y;
+          if (fast) {
+            const float3 A = f3(sc.x * iv.x, sc.y * iv.y, sc.z * iv.z);
+            const float3 Bn = f3((na.x - on.x) * iv.x, (na.y - on.y) * iv.y, (na.z - on.z) * iv.z);
+            const float3 Bf = f3((na.x - of.x) * iv.x, (na.y - of.y) * iv.y, (na.z - of.z) * iv.z);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float t0 = fmaxf(fmaxf(fmaf(q_byte(qnx, k), A.x, Bn.x), fmaf(q_byte(qny, k), A.y, Bn.y)),
-                                 fmaxf(fmaf(q_byte(qnz, k), A.z, Bn.z), 0.0f));
-          const float t1 = fminf(fminf(fmaf(q_byte(qfx, k), A.x, Bf.x), fmaf(q_byte(qfy, k), A.y, Bf.y)),
-                                 fmaf(q_byte(qfz, k), A.z, Bf.z));
-          const bool hit = k < nc && t0 <= t1 * REL && t0 <= lim;
-          key[k] = hit ? fminf(t0, 3.40282347e+38f) : INFINITY;
-          h += hit ? 1 : 0;
-        }
-      } else {
+            for (int c = 0; c < 4; ++c) {
+              const float t0 = fmaxf(fmaxf(fmaf(q_byte(qnx, c), A.x, Bn.x), fmaf(q_byte(qny, c), A.y, Bn.y)),
+                                     fmaxf(fmaf(q_byte(qnz, c), A.z, Bn.z), 0.0f));
+              const float t1 = fminf(fminf(fmaf(q_byte(qfx, c), A.x, Bf.x), fmaf(q_byte(qfy, c), A.y, Bf.y)),
+                                     fmaf(q_byte(qfz, c), A.z, Bf.z));
+              key[c] = c < nc && t0 <= t1 * REL && t0 <= lim ? fminf(t0, 3.40282347e+38f) : INFINITY;
+            }
+          } else {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float t0 =
-              fmaxf(fmaxf((fmaf(q_byte(qnx, k), sc.x, na.x) - on.x) * L.inv.x,
-                          (fmaf(q_byte(qny, k), sc.y, na.y) - on.y) * L.inv.y),
-                    fmaxf((fmaf(q_byte(qnz, k), sc.z, na.z) - on.z) * L.inv.z, 0.0f));
-          const float t1 = fminf(fminf((fmaf(q_byte(qfx, k), sc.x, na.x) - of.x) * L.inv.x,
-                                       (fmaf(q_byte(qfy, k), sc.y, na.y) - of.y) * L.inv.y),
-                                 (fmaf(q_byte(qfz, k), sc.z, na.z) - of.z) * L.inv.z);
-          const bool hit = k < nc && t0 <= t1 * REL && t0 <= lim;
-          key[k] = hit ? fminf(t0, 3.40282347e+38f) : INFINITY;
-          h += hit ? 1 : 0;
-        }
-      }
-      // Nearest first (misses, keyed +inf, sort last).
+            for (int c = 0; c < 4; ++c) {
+              const float t0 = fmaxf(fmaxf((fmaf(q_byte(qnx, c), sc.x, na.x) - on.x) * iv.x,
+                                           (fmaf(q_byte(qny, c), sc.y, na.y) - on.y) * iv.y),
+                                     fmaxf((fmaf(q_byte(qnz, c), sc.z, na.z) - on.z) * iv.z, 0.0f));
+              const float t1 = fminf(fminf((fmaf(q_byte(qfx, c), sc.x, na.x) - of.x) * iv.x,
+                                           (fmaf(q_byte(qfy, c), sc.y, na.y) - of.y) * iv.y),
+                                     (fmaf(q_byte(qfz, c), sc.z, na.z) - of.z) * iv.z);
+              key[c] = c < nc && t0 <= t1 * REL && t0 <= lim ? fminf(t0, 3.40282347e+38f) : INFINITY;
+            }
+          }
+          // Nearest first (misses, keyed +inf, sort last).
 #define THG_CSWAP(i, j)                                              \
   if (key[j] < key[i]) {                                             \
     const float tk = key[i]; key[i] = key[j]; key[j] = tk;           \
-    const int32_t tr_ = r[i]; r[i] = r[j]; r[j] = tr_;               \
+    const int32_t tr_ = ref[i]; ref[i] = ref[j]; ref[j] = tr_;       \
   }
-      THG_CSWAP(0, 1) THG_CSWAP(2, 3) THG_CSWAP(0, 2) THG_CSWAP(1, 3) THG_CSWAP(1, 2)
+          THG_CSWAP(0, 1) THG_CSWAP(2, 3) THG_CSWAP(0, 2) THG_CSWAP(1, 3) THG_CSWAP(1, 2)
 #undef THG_CSWAP
-      if (h == 0) {
-        node = pop();
-      } else {
-        node = r[0];
-        if (h > 3) push(r[3]);
-        if (h > 2) push(r[2]);
-        if (h > 1) push(r[1]);
+        }
       }
-      if (!POST) {
-        // Leaves are tested as soon as they are met (any hit: the first hit ends the ray).
-        while (node < 0 && node != RAY_DONE) node = run_leaf(node) ? RAY_DONE : pop();
-        continue;
+      sp -= k;
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int c = 3; c >= 0; --c) {
+        const bool in = key[c] < INFINITY;
+        const uint64_t mi = ballot(in && ref[c] >= 0), ml = ballot(in && ref[c] < 0);
+        if (in && ref[c] >= 0) {
+          const int pos = sp + __popcll(mi & lanemask_lt());
+          if (pos < RQ_STACK) {  // always: three entries per level of the deepest path fit
+            W.ref[pos] = ref[c];
+            W.t[pos] = lb_pack(key[c]);
+            W.own[pos] = (uint8_t)r;
+          }
+        }
+        if (in && ref[c] < 0) {
+          const int pos = ln + __popcll(ml & lanemask_lt());
+          W.leaf[pos] = ref[c];
+          W.lown[pos] = (uint8_t)r;
+        }
+        sp += __popcll(mi);
+        if (sp > RQ_STACK) sp = RQ_STACK;
+        ln += __popcll(ml);
       }
-      if (node < 0 && node != RAY_DONE && leaf == 0) {
-        leaf = node;
-        node = pop();
-      }
-      if (__ballot(leaf == 0) == 0) break;
+    } else {
+      break;
     }
-    while (leaf < 0) {
-      if (run_leaf(leaf)) {
-        node = RAY_DONE;
-        leaf = 0;
-        break;
-      }
-      leaf = 0;
-      if (node < 0 && node != RAY_DONE) {
-        leaf = node;
-        node = pop();
-      }
-    }
+    __builtin_amdgcn_wave_barrier();
   }
-  ray_lane_finish<ANY>(L, tr, out_idx, out_t, out_n, out_any);
+  if (!inrange) return;
+  const unsigned long long key = W.key[lane];
+  if (ANY) {
+    out_any[ri] = best_init >= 0.0f && key == ~0ull ? 1 : 0;
+    return;
+  }
+  const int32_t id = (int32_t)(uint32_t)key;
+  const bool hit = best_init >= 0.0f && id != 0x7fffffff;
+  const int32_t e = hit ? W.slot[lane] : 0;
+  out_idx[ri] = hit ? id : -1;
+  if (out_t) {
+    float th = cmp_key_d(key);
+    if (hit && th == 0.0f) {  // the key drops the sign of a zero
+      const RayTri *tp = rt + e;
+      th = tri_ray_e(f3(tp->a.x, tp->a.y, tp->a.z), f3(tp->b.x, tp->b.y, tp->b.z), f3(tp->c.x, tp->c.y, tp->c.z), o, d,
+                     max_time);
+    }
+    out_t[ri] = hit ? th : -1.0f;
+  }
+  if (out_n) {
+    float nx = 0, ny = 0, nz = 0;
+    if (hit) { nx = tr[e].p0.w; ny = tr[e].p1.w; nz = tr[e].p2.w; }
+    out_n[3 * ri] = nx; out_n[3 * ri + 1] = ny; out_n[3 * ri + 2] = nz;
+  }
 }
 
-template <bool ANY, int LST, int OVF, bool POST>
-__global__ void __launch_bounds__(Q_BLOCK) k_ray_q4(const QNode4 *__restrict__ qn, const RayTri *__restrict__ rt,
+template <bool ANY>
+__global__ void __launch_bounds__(WAVE) k_ray_queue(const QNode4 *__restrict__ qn, const RayTri *__restrict__ rt,
                                                     const TriRec *__restrict__ tr, const float *__restrict__ orig,
                                                     const float *__restrict__ dirs, const uint32_t *__restrict__ order,
-                                                    int64_t n, uint32_t nb_real, float best_init, float max_time,
-                                                    float scale, int exact_only, int32_t *__restrict__ out_idx,
+                                                    int64_t n, int lg, uint32_t nb_real, float best_init,
+                                                    float max_time, float scale, int exact_only, int32_t *__restrict__ out_idx,
                                                     float *__restrict__ out_t, float *__restrict__ out_n,
                                                     uint8_t *__restrict__ out_any) {
-  __shared__ int32_t s_ref[LST * Q_BLOCK];
-  bool active;
-  const int64_t ri = query_slot(nb_real, n, order, active);
-  if (!active) return;
-  ray_q4_body<ANY, LST, OVF, POST>(s_ref, qn, rt, tr, orig, dirs, ri, best_init, max_time, scale, exact_only,
-                                   out_idx, out_t, out_n, out_any);
+  __shared__ RayWave s_w;
+  const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
+  if (lb_blk >= nb_real) return;
+  ray_queue_body<ANY>(s_w, qn, rt, tr, orig, dirs, order, n, (int64_t)lb_blk, lg, best_init, max_time, scale, exact_only,
+                      out_idx, out_t, out_n, out_any);
 }
 
-// Many first-hit ray batches in one launch over their meshes' QNode4 trees; one 64-lane block per
-// wave of a segment (SEG_WAVE_QUERIES rays).
-template <int LST, int OVF>
-__global__ void __launch_bounds__(Q_BLOCK) k_ray_q4_multi(const SegDesc *__restrict__ seg, int nseg,
+// Many first-hit ray batches in one launch over their meshes' ray trees; the waves of a segment take
+// 64 >> lanes_log2 rays each.
+__global__ void __launch_bounds__(WAVE) k_ray_queue_multi(const SegDesc *__restrict__ seg, int nseg,
                                                           uint64_t total_waves, uint32_t nb_real) {
-  __shared__ int32_t s_ref[LST * Q_BLOCK];
+  __shared__ RayWave s_w;
   const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
   if (lb_blk >= nb_real || (uint64_t)lb_blk >= total_waves) return;
   const int si = uni(find_segment(seg, nseg, (int64_t)lb_blk));
   const SegDesc &d = seg[si];
-  const int64_t t = ((int64_t)lb_blk - (int64_t)d.wave_begin) * Q_BLOCK + threadIdx.x;
-  if (t >= d.n) return;
-  const int64_t ri = d.order ? (int64_t)d.order[t] : t;
-  ray_q4_body<false, LST, OVF, true>(s_ref, readonly_ptr<QNode4>(d.qnodes), readonly_ptr<RayTri>(d.rays),
-                                     readonly_ptr<TriRec>(d.elems), readonly_ptr<float>(d.q), readonly_ptr<float>(d.q2), ri, d.best_init, d.max_time, d.scale, q4_exact_only(d.scale), d.idx, d.dist,
-                               d.cp, nullptr);
+  ray_queue_body<false>(s_w, readonly_ptr<QNode4>(d.qnodes), readonly_ptr<RayTri>(d.rays),
+                        readonly_ptr<TriRec>(d.elems), readonly_ptr<float>(d.q), readonly_ptr<float>(d.q2),
+                        readonly_ptr<uint32_t>(d.order), d.n, (int64_t)lb_blk - (int64_t)d.wave_begin, d.lanes_log2,
+                        d.best_init, d.max_time, d.scale, q4_exact_only(d.scale), d.idx, d.dist, d.cp, nullptr);
 }
 
 //--------------------------------------------------------------------------------------------------
@@ -2580,6 +2662,35 @@ void order_rays(const Bvh &b, const float *o, const float *d, int64_t n, QuerySc
     return e && std::string(e) == "origin";
   }();
   order_batch(b, o, by_origin ? nullptr : d, n, ws, s);
+}
+
+// Rays by work queue where a mesh has its 4-wide tree and three entries per level fit the kernel's
+// reserve; THG_RAY_Q4=0 and deeper trees take the binary tree, one ray per lane.
+bool use_ray_queue(const Bvh &b) {
+  static const bool q4 = env_int("THG_RAY_Q4", 1) != 0;
+  return q4 && b.qnodes.p != nullptr && q4_stack(b) <= Q4_MAX_STACK;
+}
+
+// log2 of the lanes per ray of the work queue: rays are spread over up to 4,096 waves (what the GPU
+// holds), 8 to 64 per wave. First hits on a torus of 1,048,576 triangles at 64 / 32 / 16 / 8 per wave: 3,000
+// rays 44, 32, 27, 24 us; 20,000 55, 39, 31, 31; 100,000 59, 48, 61, 88; 300,000 102, 99, 130, 219;
+// 1,000,000 210, 255, 388, 691.
+int ray_lanes_log2(int64_t n) {
+  int lg = 0;
+  while (lg < 3 && n <= (4096 * WAVE) >> (lg + 1)) ++lg;
+  return lg;
+}
+
+// Whether a ray batch is sorted first. The queue's steps mix the rays of a wave, so order buys it
+// only cache hits, and in random order its waves are more alike. On trees the caches hold it is not
+// worth the sort (4,000,000 first hits, sorted / as they come: torus of 1,048,576 triangles 1.03 / 0.77 ms,
+// of 4,000,000 1.21 / 0.90; sphere of 1,000,000 1.96 / 2.22), nor for fewer rays on a larger one (1,000,000
+// on a sphere of 4,000,000: 1.68 / 1.62 ms). Beyond both lines it mostly is: 16,000,000 rays on that
+// sphere 16.9 / 23.8 ms, any hit 13.9 / 23.1; on a torus of 16,000,000 5.5 / 4.4, any hit 5.8 / 6.4.
+bool order_ray_batch(const Bvh &b, int64_t n) {
+  if (!use_ray_queue(b)) return true;
+  const int64_t bytes = b.n * (int64_t)sizeof(RayTri) + b.num_qnodes * (int64_t)sizeof(QNode4);
+  return n > ((int64_t)1 << 22) && bytes > ((int64_t)256 << 20);
 }
 
 static float prev_float(float x) { return std::nextafter(x, -INFINITY); }
@@ -2881,20 +2992,17 @@ void launch_knn_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_wav
   launch_check("k_knn_queue_multi");
 }
 
-void launch_ray_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int stack, hipStream_t s,
-                      int q_stack) {
+void launch_ray_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s) {
+  if (nseg <= 0 || total_waves == 0) return;
+  const uint32_t nb = (uint32_t)total_waves;
+  hipLaunchKernelGGL(k_ray_queue_multi, dim3(round_up8(nb)), dim3(WAVE), 0, s, seg_dev, nseg, total_waves, nb);
+  launch_check("k_ray_queue_multi");
+}
+
+void launch_ray_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int stack, hipStream_t s) {
   if (nseg <= 0 || total_waves == 0) return;
   uint32_t nb = (uint32_t)total_waves;
   uint32_t grid = round_up8(nb);
-  if (q_stack > 0) {
-    require(q_stack <= Q4_MAX_STACK, "ray tree too deep for the 4-wide traversal stack");
-    if (q_stack <= 16 + 32)
-      hipLaunchKernelGGL((k_ray_q4_multi<16, 32>), dim3(grid), dim3(Q_BLOCK), 0, s, seg_dev, nseg, total_waves, nb);
-    else
-      hipLaunchKernelGGL((k_ray_q4_multi<16, 96>), dim3(grid), dim3(Q_BLOCK), 0, s, seg_dev, nseg, total_waves, nb);
-    launch_check("k_ray_q4_multi");
-    return;
-  }
   if (stack <= 32) hipLaunchKernelGGL(k_ray_multi<32>, dim3(grid), dim3(Q_BLOCK), 0, s, seg_dev, nseg, total_waves, nb);
   else hipLaunchKernelGGL(k_ray_multi<64>, dim3(grid), dim3(Q_BLOCK), 0, s, seg_dev, nseg, total_waves, nb);
   launch_check("k_ray_multi");
@@ -3010,37 +3118,25 @@ void launch_ray(const Bvh &b, const float *o, const float *d, int64_t n, float m
                 const uint32_t *given_order) {
   if (n <= 0) return;
   require(!b.points && (b.n == 0 || b.rays.p != nullptr), "ray queries need a triangle BVH");
-  if (sort_rays) order_rays(b, o, d, n, ws, s);
-  else ws.order = given_order;
+  if (!sort_rays) ws.order = given_order;
+  else if (order_ray_batch(b, n)) order_rays(b, o, d, n, ws, s);
+  else ws.order = nullptr;
   uint32_t nb = ceil_div(n, Q_BLOCK);
   uint32_t grid = round_up8(nb);
   // Thea accepts only hits strictly before max_time at the structure level (BvhN.hpp:2247-2258).
   float best = max_time >= 0 ? prev_float(max_time) : INFINITY;
   int st = pick_stack(b.max_depth);
   KernelTimer kt(b.ctx, s, any ? "any_hit" : "ray");
-  // Quantized 4-wide tree (k_ray_q4; THG_RAY_Q4=0 selects the binary kernels below) when its stack
-  // bound (three entries per level) fits 16 LDS + 96 private entries.
-  static const bool q4 = env_int("THG_RAY_Q4", 1) != 0;
-  if (q4 && b.qnodes.p && q4_stack(b) <= Q4_MAX_STACK) {
-    const int exact_only = q4_exact_only(b.scale);
-    const bool small = q4_stack(b) <= 16 + 32;
-    // Postponed leaves (while-while) for first hits, leaves tested when met for any hit
-    // (THG_RAY_POST / THG_RAY_ANY_POST override).
-    static const bool post = env_int("THG_RAY_POST", 1) != 0, any_post = env_int("THG_RAY_ANY_POST", 0) != 0;
-#define THG_RQ(A, O, P)                                                                                               \
-  hipLaunchKernelGGL((k_ray_q4<A, 16, O, P>), dim3(grid), dim3(Q_BLOCK), 0, s, b.qnodes.as<QNode4>(),               \
-                     b.rays.as<RayTri>(), b.elems.as<TriRec>(), o, d, ws.order, n, nb, best, max_time, b.scale,     \
-                     exact_only, idx, t, nrm, hit)
-#define THG_RQP(A, O, P) \
-  if (P) { THG_RQ(A, O, true); } else { THG_RQ(A, O, false); }
-    if (any) {
-      if (small) { THG_RQP(true, 32, any_post); } else { THG_RQP(true, 96, any_post); }
-    } else {
-      if (small) { THG_RQP(false, 32, post); } else { THG_RQP(false, 96, post); }
-    }
-#undef THG_RQP
+  if (use_ray_queue(b)) {
+    const int lg = ray_lanes_log2(n);
+    const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE), qgrid = round_up8(qnb);
+#define THG_RQ(A)                                                                                                  \
+  hipLaunchKernelGGL(k_ray_queue<A>, dim3(qgrid), dim3(WAVE), 0, s, b.qnodes.as<QNode4>(), b.rays.as<RayTri>(),    \
+                     b.elems.as<TriRec>(), o, d, ws.order, n, lg, qnb, best, max_time, b.scale,                    \
+                     q4_exact_only(b.scale), idx, t, nrm, hit)
+    if (any) THG_RQ(true); else THG_RQ(false);
 #undef THG_RQ
-    launch_check("k_ray_q4");
+    launch_check("k_ray_queue");
     kt.stop();
     return;
   }

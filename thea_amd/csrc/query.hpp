@@ -137,13 +137,18 @@ void launch_knn_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_wav
 bool use_knn_queue(const Bvh &b, int64_t n, int k);
 int knn_queue_lanes_log2(int64_t n, int k, bool points);
 bool use_wave_traversal(const Bvh &b, int64_t n);
-// stack: the deepest tree among the segments plus one (32 or 64 entries). q_stack > 0 traverses
-// the segments' QNode4 trees instead; it must be at least q4_stack() of every segment's BVH.
-void launch_ray_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int stack, hipStream_t s,
-                      int q_stack = 0);
-// Stack entries a QNode4 traversal of b may need (three per level) and the most the kernels hold.
+// Rays by work queue, segments as above.
+void launch_ray_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s);
+bool use_ray_queue(const Bvh &b);
+int ray_lanes_log2(int64_t n);
+bool order_ray_batch(const Bvh &b, int64_t n);
+// One ray per lane on the binary trees; stack: the deepest among the segments plus one (32 or 64
+// entries).
+void launch_ray_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, int stack, hipStream_t s);
+// Stack entries a QNode4 walk of one ray in b may need (three per level), and the most that the work
+// queue keeps in reserve for it.
 inline int q4_stack(const Bvh &b) { return 3 * b.q_depth + 1; }
-constexpr int Q4_MAX_STACK = 16 + 96;
+constexpr int Q4_MAX_STACK = 112;
 constexpr int SEG_WAVE_QUERIES = 64;  // queries per wave in the multi-batch kernels
 void ray_stats(const Bvh &b, const float *o, const float *d, int64_t n, int32_t *idx, int32_t *counts, hipStream_t s);
 void closest_wave_stats(const Bvh &b, const float *q, int64_t n, unsigned long long *stats, QueryScratch &ws,

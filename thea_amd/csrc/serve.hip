@@ -148,7 +148,7 @@ static void worker_loop(Server *S, int wi) {
           // work queue (2), wave-cooperative (0) or one query per lane (1), as single calls choose
           const bool queue = r.r.type == THG_REQ_CLOSEST ? use_queue_traversal(*r.bvh, r.r.n)
                              : r.r.type == THG_REQ_KNN   ? use_knn_queue(*r.bvh, r.r.n, r.r.k)
-                                                         : false;
+                                                         : use_ray_queue(*r.bvh);
           int lane = queue ? 2 : r.r.type != THG_REQ_RAY && !use_wave_traversal(*r.bvh, r.r.n) ? 1 : 0;
           groups[{r.r.type, lane, kk}].push_back(&r);
         }
@@ -201,7 +201,8 @@ static void worker_loop(Server *S, int wi) {
               d.cp = q.cp;
               d.best_init = bound_to_best(q.bound);
             }
-            if (q.n >= ORDER_MIN_QUERIES && (!queue || q.n > QUEUE_UNSORTED_MAX)) {
+            const bool sorted = type == THG_REQ_RAY ? order_ray_batch(b, q.n) : !queue || q.n > QUEUE_UNSORTED_MAX;
+            if (q.n >= ORDER_MIN_QUERIES && sorted) {
               scratch.emplace_back(new QueryScratch());
               if (type == THG_REQ_RAY) order_rays(b, q.q, q.dirs, q.n, *scratch.back(), s);
               else order_queries(b, q.q, q.n, *scratch.back(), s);
@@ -209,6 +210,7 @@ static void worker_loop(Server *S, int wi) {
             }
             d.lanes_log2 = !queue                    ? 0
                            : type == THG_REQ_CLOSEST ? queue_lanes_log2(total)
+                           : type == THG_REQ_RAY     ? ray_lanes_log2(total)
                                                      : knn_queue_lanes_log2(total, kk.first, false);
             d.wave_begin = waves;
             waves += (uint64_t)(((q.n << d.lanes_log2) + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES);
@@ -224,13 +226,8 @@ static void worker_loop(Server *S, int wi) {
             else if (lane) launch_knn_lane_multi(dd, nseg, waves, kk.first, false, stack, s);
             else launch_knn_multi(dd, nseg, waves, kk.first, false, s);
           } else {
-            int q_stack = 0;
-            bool q4 = true;
-            for (SrvRequest *r : list) {
-              q4 = q4 && r->bvh->qnodes.p != nullptr && q4_stack(*r->bvh) <= Q4_MAX_STACK;
-              q_stack = std::max(q_stack, q4_stack(*r->bvh));
-            }
-            launch_ray_multi(dd, nseg, waves, stack, s, q4 ? q_stack : 0);
+            if (queue) launch_ray_queue_multi(dd, nseg, waves, s);
+            else launch_ray_multi(dd, nseg, waves, stack, s);
           }
         }
       }
