@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "common.hpp"
@@ -348,7 +349,6 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
     for (int a = 0; a < 3; ++a) up[a] = up_in[a] / nn;
   }
   const int nb = (int)((n + ICP_CHUNK - 1) / ICP_CHUNK);
-  AsyncBuf src(n * K * 24, s), cur(K * 96, s), aux(K * 96, s), sums7(K * 56, s), cov(K * 72, s), errs(K * 8, s);
   // qpts: the correspondences of problem k at [k n, (k + 1) n) (kept across iterations whatever the
   // active set); qtmp: the nearest points of one launch over part of the problems, by slot. While every
   // problem is active the launch writes qpts itself (a copy per problem and launch took 0.6 ms of device
@@ -357,53 +357,75 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
   // kept in double; a float BVH with the positions rounded to float.
   const bool f64 = to.f64;
   const int64_t pb = f64 ? 24 : 12;  // bytes per position / correspondence
-  AsyncBuf pos(n * K * pb, s), qpts(n * K * pb, s), qtmp, idx(n * K * 4, s), prob(K * 4, s);
-  AsyncBuf partial((size_t)K * nb * ICP_MAXC * 8, s);
-  hipLaunchKernelGGL(k_icp_init, dim3(ceil_div(n * K, 256)), dim3(256), 0, s, n, K, from, init, src.as<double>());
+  // All arrays in one allocation (the driver spent 2.3 ms per search on giving 18 back), the host's
+  // parameters (cur, aux, prob) and the sums it reads back (sums7, cov, errs) each in one run, so a stage of
+  // the loop takes one copy up and one down: 24 problems of 60,000 points, 4 iterations, 7.2 -> 4.5 ms.
+  Layout lay;
+  const size_t o_src = lay.add(n * K * 24), o_pos = lay.add(n * K * pb), o_q = lay.add(n * K * pb);
+  const size_t o_idx = lay.add(n * K * 4), o_par = lay.add(K * (96 + 96 + 4)), o_res = lay.add(K * (56 + 72 + 8));
+  const size_t o_part = lay.add((size_t)K * nb * ICP_MAXC * 8), o_sort = lay.add(sort_scratch_words(n * K) * 4);
+  Workspace mem;
+  mem.alloc(lay.total, s);
+  double *const src = mem.at<double>(o_src), *const cur = mem.at<double>(o_par), *const aux = cur + 12 * K;
+  int32_t *const prob = reinterpret_cast<int32_t *>(aux + 12 * K);
+  double *const sums7 = mem.at<double>(o_res), *const cov = sums7 + 7 * K, *const errs = cov + 9 * K;
+  double *const partial = mem.at<double>(o_part);
+  int32_t *const idx = mem.at<int32_t>(o_idx);
+  void *const pos = mem.at<char>(o_pos), *const qpts = mem.at<char>(o_q);
+  AsyncBuf qtmp;
+  hipLaunchKernelGGL(k_icp_init, dim3(ceil_div(n * K, 256)), dim3(256), 0, s, n, K, from, init, src);
   launch_check("k_icp_init");
 
   std::vector<IcpProblem> P(K);
   for (auto &p : P) { p.old_tr = p.new_tr = p.cur = xf_identity(); }
-  std::vector<double> h_cur(12 * K), h_aux(12 * K), h_sums(7 * K), h_cov(9 * K), h_err(K);
+  std::vector<double> h_par(24 * K + (K + 1) / 2), h_res(17 * K);
+  double *const h_cur = h_par.data(), *const h_aux = h_cur + 12 * K;
+  const double *const h_sums = h_res.data(), *const h_cov = h_sums + 7 * K, *const h_err = h_cov + 9 * K;
   std::vector<int32_t> active;
-
-  auto upload_cur = [&]() {
-    for (int k = 0; k < K; ++k) std::copy(P[k].cur.m, P[k].cur.m + 12, &h_cur[12 * k]);
-    THG_HIP(hipMemcpyAsync(cur.p, h_cur.data(), 96 * K, hipMemcpyHostToDevice, s));
+  // One upload per stage, before its kernels; the stage ends in download(), which waits for them, so the
+  // parameters are not written again while a copy of them is under way.
+  auto upload = [&]() {
+    for (int k = 0; k < K; ++k) std::copy(P[k].cur.m, P[k].cur.m + 12, h_cur + 12 * k);
+    memcpy(h_aux + 12 * K, active.data(), 4 * active.size());
+    THG_HIP(hipMemcpyAsync(cur, h_par.data(), (size_t)K * (96 + 96 + 4), hipMemcpyHostToDevice, s));
+  };
+  auto download = [&]() {
+    THG_HIP(hipMemcpyAsync(h_res.data(), sums7, (size_t)K * (56 + 72 + 8), hipMemcpyDeviceToHost, s));
+    THG_HIP(hipStreamSynchronize(s));
   };
   auto set_active = [&]() {
     active.clear();
     for (int k = 0; k < K; ++k)
       if (!P[k].done) active.push_back(k);
-    if (!active.empty())
-      THG_HIP(hipMemcpyAsync(prob.p, active.data(), 4 * active.size(), hipMemcpyHostToDevice, s));
   };
   QueryScratch ws;  // sort memory of the nearest-point launches
+  ws.ext = mem.at<uint32_t>(o_sort);
+  ws.ext_cap = n * K;
   // nearest points of the active problems' current positions
   auto nearest = [&]() {
     const int A = (int)active.size();
     const bool all = A == K;
     if (!all) qtmp.ensure(n * K * pb, s);
-    void *out = all ? qpts.p : qtmp.p;
+    void *out = all ? qpts : qtmp.p;
     if (f64) {
-      hipLaunchKernelGGL(k_icp_pos<double>, dim3(ceil_div(n * A, 256)), dim3(256), 0, s, n, A, prob.as<int32_t>(),
-                         src.as<double>(), cur.as<double>(), pos.as<double>());
+      hipLaunchKernelGGL(k_icp_pos<double>, dim3(ceil_div(n * A, 256)), dim3(256), 0, s, n, A, prob, src, cur,
+                         (double *)pos);
       launch_check("k_icp_pos");
-      launch_closest64(to, pos.as<double>(), n * A, -1.0, idx.as<int32_t>(), (double *)out, nullptr, nullptr, ws, s);
+      launch_closest64(to, (double *)pos, n * A, -1.0, idx, (double *)out, nullptr, nullptr, ws, s);
     } else {
-      hipLaunchKernelGGL(k_icp_pos<float>, dim3(ceil_div(n * A, 256)), dim3(256), 0, s, n, A, prob.as<int32_t>(),
-                         src.as<double>(), cur.as<double>(), pos.as<float>());
+      hipLaunchKernelGGL(k_icp_pos<float>, dim3(ceil_div(n * A, 256)), dim3(256), 0, s, n, A, prob, src, cur,
+                         (float *)pos);
       launch_check("k_icp_pos");
-      launch_closest(to, pos.as<float>(), n * A, -1.0, 0, idx.as<int32_t>(), (float *)out, nullptr, nullptr, ws, s);
+      launch_closest(to, (float *)pos, n * A, -1.0, 0, idx, (float *)out, nullptr, nullptr, ws, s);
     }
     if (!all) {
       const dim3 g(ceil_div(3 * n * A, 256));
       if (f64)
-        hipLaunchKernelGGL(k_icp_place<double>, g, dim3(256), 0, s, n, A, prob.as<int32_t>(), qtmp.as<double>(),
-                           qpts.as<double>());
+        hipLaunchKernelGGL(k_icp_place<double>, g, dim3(256), 0, s, n, A, prob, qtmp.as<double>(),
+                           (double *)qpts);
       else
-        hipLaunchKernelGGL(k_icp_place<float>, g, dim3(256), 0, s, n, A, prob.as<int32_t>(), qtmp.as<float>(),
-                           qpts.as<float>());
+        hipLaunchKernelGGL(k_icp_place<float>, g, dim3(256), 0, s, n, A, prob, qtmp.as<float>(),
+                           (float *)qpts);
       launch_check("k_icp_place");
     }
   };
@@ -412,9 +434,8 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
     const int nc = mode == 0 ? 7 : (mode == 1 ? 9 : 1);
     const dim3 g((unsigned)(A * nb));
 #define THG_SUMS(M, QT)                                                                                            \
-  hipLaunchKernelGGL((k_icp_sums<M, QT>), g, dim3(ICP_THREADS), 0, s, n, prob.as<int32_t>(), src.as<double>(),      \
-                     cur.as<double>(), qpts.as<QT>(), wt, wr, sums7.as<double>(), aux.as<double>(), nb,              \
-                     partial.as<double>())
+  hipLaunchKernelGGL((k_icp_sums<M, QT>), g, dim3(ICP_THREADS), 0, s, n, prob, src, cur, (const QT *)qpts, wt, wr,  \
+                     sums7, aux, nb, partial)
     if (f64) {
       if (mode == 0) THG_SUMS(0, double); else if (mode == 1) THG_SUMS(1, double); else THG_SUMS(2, double);
     } else {
@@ -422,24 +443,23 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
     }
 #undef THG_SUMS
     launch_check("k_icp_sums");
-    hipLaunchKernelGGL(k_icp_final, dim3(ceil_div((int64_t)A * nc, 64)), dim3(64), 0, s, A, nb, nc, prob.as<int32_t>(),
-                       partial.as<double>(), stride, dst);
+    hipLaunchKernelGGL(k_icp_final, dim3(ceil_div((int64_t)A * nc, 64)), dim3(64), 0, s, A, nb, nc, prob, partial,
+                       stride, dst);
     launch_check("k_icp_final");
   };
-  // measureError(tr, ...) with the current to_points (Icp3.hpp:422-465): error of L = linear part
-  // of trs[k], translation term |tr p_mean - q_mean|^2 added on the host.
-  auto measure = [&](const std::vector<Xf> &trs) {
-    sums(0, sums7.as<double>(), 7);
+  // measureError(tr, ...) with the current to_points (Icp3.hpp:422-465), found anew if remap: error of
+  // L = linear part of trs[k], translation term |tr p_mean - q_mean|^2 added on the host.
+  auto measure = [&](const std::vector<Xf> &trs, bool remap) {
     for (int k : active) {
-      std::fill(&h_aux[12 * k], &h_aux[12 * k] + 12, 0.0);
+      std::fill(h_aux + 12 * k, h_aux + 12 * k + 12, 0.0);
       for (int i = 0; i < 3; ++i)
         for (int j = 0; j < 3; ++j) h_aux[12 * k + 3 * i + j] = trs[k].m[4 * i + j];
     }
-    THG_HIP(hipMemcpyAsync(aux.p, h_aux.data(), 96 * K, hipMemcpyHostToDevice, s));
-    sums(2, errs.as<double>(), 1);
-    THG_HIP(hipMemcpyAsync(h_sums.data(), sums7.p, 56 * K, hipMemcpyDeviceToHost, s));
-    THG_HIP(hipMemcpyAsync(h_err.data(), errs.p, 8 * K, hipMemcpyDeviceToHost, s));
-    THG_HIP(hipStreamSynchronize(s));
+    upload();
+    if (remap) nearest();
+    sums(0, sums7, 7);
+    sums(2, errs, 1);
+    download();
     std::vector<double> e(K, 0);
     for (int k : active) {
       const double *sm = &h_sums[7 * k];
@@ -455,11 +475,9 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
 
   // initial mapping and error (Icp3.hpp:210-219)
   set_active();
-  upload_cur();
-  nearest();
   {
     std::vector<Xf> ident(K, xf_identity());
-    std::vector<double> e = measure(ident);
+    std::vector<double> e = measure(ident, true);
     for (int k = 0; k < K; ++k) {
       P[k].old_err = P[k].new_err = e[k];
       if (e[k] <= DBL_MIN) {
@@ -473,17 +491,15 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
     set_active();
     if (active.empty()) break;
     // alignOneStep with the mapping of the last measurement (Icp3.hpp:288-375)
-    sums(0, sums7.as<double>(), 7);
     for (int k : active) {
-      std::fill(&h_aux[12 * k], &h_aux[12 * k] + 12, 0.0);
+      std::fill(h_aux + 12 * k, h_aux + 12 * k + 12, 0.0);
       for (int a = 0; a < 3; ++a) h_aux[12 * k + a] = up[a];
       h_aux[12 * k + 3] = has_up ? 1.0 : 0.0;
     }
-    THG_HIP(hipMemcpyAsync(aux.p, h_aux.data(), 96 * K, hipMemcpyHostToDevice, s));
-    sums(1, cov.as<double>(), 9);
-    THG_HIP(hipMemcpyAsync(h_cov.data(), cov.p, 72 * K, hipMemcpyDeviceToHost, s));
-    THG_HIP(hipMemcpyAsync(h_sums.data(), sums7.p, 56 * K, hipMemcpyDeviceToHost, s));
-    THG_HIP(hipStreamSynchronize(s));
+    upload();
+    sums(0, sums7, 7);
+    sums(1, cov, 9);
+    download();
     std::vector<Xf> inc(K, xf_identity());
     for (int k : active) {
       M3 C{};
@@ -507,9 +523,8 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
       P[k].iterations = it + 1;
     }
     // measureError(inc, from_points, to): new mapping at the same positions, error of inc on it
-    if (it > 0) nearest();  // at it == 0 the positions are the initial ones: same mapping
-    std::vector<double> e = measure(inc);
-    bool moved = false;
+    // (at it == 0 the positions are the initial ones: same mapping)
+    std::vector<double> e = measure(inc, it > 0);
     for (int k : active) {
       IcpProblem &p = P[k];
       p.new_err = e[k];
@@ -522,12 +537,10 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
           continue;
         }
         p.cur = p.new_tr;  // from_points = new_tr * from (Icp3.hpp:251-252)
-        moved = true;
       }
       p.old_err = p.new_err;
       p.old_tr = p.new_tr;
     }
-    if (moved) upload_cur();
   }
   for (int k = 0; k < K; ++k) {
     IcpProblem &p = P[k];
@@ -594,17 +607,22 @@ extern "C" int thg_icp_align(thg_bvh to, const double *from, int64_t n, int32_t 
       }
       return;
     }
-    AsyncBuf hf, hi, hwt, hwr;
-    auto stage = [&](AsyncBuf &buf, const double *p, size_t count) -> const double * {
-      if (!p || mem == THG_MEM_DEVICE) return p;
-      buf.ensure(count * 8, s);
-      THG_HIP(hipMemcpyAsync(buf.p, p, count * 8, hipMemcpyHostToDevice, s));
-      return buf.as<double>();
+    // host arrays staged in one allocation
+    const bool host = mem == THG_MEM_HOST;
+    Layout lay;
+    Workspace staged;
+    const size_t o_from = lay.add((size_t)n * 24), o_init = lay.add(initial ? (size_t)K * 96 : 0);
+    const size_t o_wt = lay.add(wt ? (size_t)n * 8 : 0), o_wr = lay.add(wr ? (size_t)n * 8 : 0);
+    if (host) staged.alloc(lay.total, s);
+    auto stage = [&](size_t o, const double *p, size_t count) -> const double * {
+      if (!p || !host) return p;
+      THG_HIP(hipMemcpyAsync(staged.at<double>(o), p, count * 8, hipMemcpyHostToDevice, s));
+      return staged.at<double>(o);
     };
-    const double *d_from = stage(hf, from, (size_t)n * 3);
-    const double *d_init = stage(hi, initial, (size_t)K * 12);
-    const double *d_wt = stage(hwt, wt, (size_t)n);
-    const double *d_wr = stage(hwr, wr, (size_t)n);
+    const double *d_from = stage(o_from, from, (size_t)n * 3);
+    const double *d_init = stage(o_init, initial, (size_t)K * 12);
+    const double *d_wt = stage(o_wt, wt, (size_t)n);
+    const double *d_wr = stage(o_wr, wr, (size_t)n);
     icp_align(*b, d_from, n, K, d_init, thr, min_it, max_it, has_up, up, kabsch, d_wt, d_wr, transforms, errors,
               iterations, s);
     THG_HIP(hipStreamSynchronize(s));

@@ -94,6 +94,14 @@ __global__ void __launch_bounds__(256) k_query_keys64(const double *__restrict__
   keys[i] = (spread10_64(ix) << 2) | (spread10_64(iy) << 1) | spread10_64(iz);
 }
 
+// Squared float distance above which a point cannot beat a lane's best d^2 (-1: the lane admits nothing,
+// +inf: no bound yet). The float coordinates of query and point are within 2^-24 of theirs, and the
+// float arithmetic within 2^-21 of its result: the 2^-12 and the two slacks cover both.
+__device__ __forceinline__ float reject64(double bd, float sl) {
+  const float t = fmaf(2.0f, sl, sqrtf(float_up(bd)) * (1.0f + 1.0f / 4096.0f));
+  return bd < 0.0 ? -1.0f : t * t;
+}
+
 __global__ void __launch_bounds__(B64) k_closest64(const BNode *__restrict__ nodes, const PointRecD *__restrict__ pr,
                                                    const double *__restrict__ q, const uint32_t *__restrict__ order,
                                                    int64_t n, uint32_t nb_real, double best_init, float scale,
@@ -134,6 +142,7 @@ __global__ void __launch_bounds__(B64) k_closest64(const BNode *__restrict__ nod
       if (better64(d, r.id, bd, bi)) { bd = d; bi = r.id; bslot = e; }
     }
   }
+  float rej = reject64(bd, sl);
   int32_t s_ref = 0;
   float s_lx = 0, s_ly = 0, s_lz = 0, s_hx = 0, s_hy = 0, s_hz = 0;
   int32_t sp = 0;
@@ -192,7 +201,13 @@ __global__ void __launch_bounds__(B64) k_closest64(const BNode *__restrict__ nod
         ++sp;
       }
     }
+    // A double distance costs half the float rate and its coordinates six lane reads, so each point is
+    // first held against every lane's bound in float (1,440,000 queries, 80,000 points: 758 -> 712 us).
+    const float pxf = (float)px, pyf = (float)py, pzf = (float)pz;
     for (int32_t j = 0; j < total; ++j) {
+      const float ex = lreadf(pxf, j) - fx, ey = lreadf(pyf, j) - fy, ez = lreadf(pzf, j) - fz;
+      const float df = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
+      if (__ballot(!(df > rej)) == 0) continue;
       const double x = lreadd(px, j), y = lreadd(py, j), z = lreadd(pz, j);
       const int32_t id = lread(pid, j);
       const double dx = x - qx, dy = y - qy, dz = z - qz;
@@ -201,6 +216,7 @@ __global__ void __launch_bounds__(B64) k_closest64(const BNode *__restrict__ nod
         bd = d;
         bi = id;
         bslot = j < lc0 ? lf0 + j : lf1 + (j - lc0);
+        rej = reject64(bd, sl);
       }
     }
     if (next >= 0) { node = next; nd = nd_next; continue; }
