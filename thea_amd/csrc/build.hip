@@ -8,7 +8,8 @@
 //  4. k_karras        binary radix tree over the sorted codes (Karras, "Maximizing Parallelism in
 //                     the Construction of BVHs, Octrees, and k-d Trees", HPG 2012), duplicate codes
 //                     disambiguated by position; nodes of more than leaf_size elements are kept.
-//  5. k_records       element records in leaf order (TriRec with Thea's per-triangle constants,
+//  5. k_tri_records, k_point_records
+//                     element records in leaf order (TriRec with Thea's per-triangle constants,
 //                     RayTri, ScreenRec) and the box pyramid: the boxes of every aligned run of 2^L
 //                     sorted elements, a block's 256 at a time from registers.
 //  6. k_emit          kept nodes compacted into 64-byte BNodes holding both children's boxes. A
