@@ -68,6 +68,34 @@ def test_icp_batch_equals_single_and_oracle(oracle):
         _check(tr[k], err[k], its[k], ref, f"problem {k}")
 
 
+@pytest.mark.parametrize("target", ["points", "mesh"])
+def test_icp_problems_that_end_apart_equal_single(target):
+    """200,000 positions while all four problems run, which are searched in spatial order, and 100,000 or
+    fewer once two have ended, which are searched as they come."""
+    import thea_amd
+    from thea_amd import workloads as W
+    print(f"case icp ending apart {target}", flush=True)
+    g = np.random.default_rng(15)
+    n = 50000
+    if target == "points":
+        to = _ellipsoid(g, n)
+        src = to.astype(np.float64)
+        bvh = thea_amd.PointBvh(to)
+    else:
+        v, t = W.torus(96, 48, R=1.0, r=0.3, amp=0.03, seed=7)
+        src = (v[t[g.integers(0, len(t), n)]] * g.dirichlet([1, 1, 1], n)[:, :, None]).sum(1)
+        bvh = thea_amd.MeshBvh(thea_amd.Mesh(v, t))
+    inits = np.stack([_xf(_axis_rot([1, 2, 3], a), [d, -d, 0.5 * d])
+                      for a, d in ((0.01, 0.002), (0.1, 0.02), (0.3, 0.05), (0.9, 0.1))])
+    icp = thea_amd.Icp3(fractional_error_threshold=0.05, max_iterations=25, kabsch=True)
+    tr, err, its = icp.alignBatch(src, bvh, initial=inits)
+    its = list(its)
+    assert sorted(its)[1] < sorted(its)[3], its  # two or fewer problems search on
+    for k in range(len(inits)):
+        t1, e1, i1 = icp.alignBatch(src, bvh, initial=inits[k:k + 1])
+        assert i1[0] == its[k] and e1[0] == err[k] and np.array_equal(t1[0], tr[k]), f"problem {k}"
+
+
 def test_icp_mesh_weights_up(oracle):
     import thea_amd
     from oracle import icp as I

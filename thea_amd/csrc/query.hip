@@ -2796,6 +2796,7 @@ void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, 
   if (n <= 0) return;
   const bool queue = b.points ? use_knn_queue(b, n, 1) : use_queue_traversal(b, n);
   if (!queue || n > QUEUE_UNSORTED_MAX) order_queries(b, q, n, ws, s);
+  else ws.order = nullptr;  // a reused scratch may hold an earlier batch's order
   uint32_t nb = ceil_div(n, Q_BLOCK);
   uint32_t grid = round_up8(nb);
   float best = bound_to_best(dist_bound);
@@ -3059,6 +3060,7 @@ void launch_knn(const Bvh &b, const float *q, int64_t n, int k, double dist_boun
   if (n <= 0) return;
   const bool queue = use_knn_queue(b, n, k);
   if (!queue || n > QUEUE_UNSORTED_MAX) order_queries(b, q, n, ws, s);
+  else ws.order = nullptr;  // a reused scratch may hold an earlier batch's order
   uint32_t nb = ceil_div(n, Q_BLOCK);
   uint32_t grid = round_up8(nb);
   float best = bound_to_best(dist_bound);
