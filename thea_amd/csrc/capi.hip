@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "block_cache.hpp"
 #include "common.hpp"
 #include "kernels_common.hpp"
 #include "query.hpp"
@@ -51,89 +52,53 @@ __global__ void k_check_tris(const int32_t *__restrict__ tris, int64_t n3, int64
 }
 
 namespace {
-struct DevBlock {
-  void *p;
-  size_t bytes;
-  int device;
+struct HipDriver {
+  using Error = hipError_t;
+  using Stream = hipStream_t;
+  static Error success() { return hipSuccess; }
+  static bool out_of_memory(Error e) {
+    if (e != hipErrorOutOfMemory) return false;
+    (void)hipGetLastError();
+    return true;
+  }
+  static Error alloc(void **p, size_t n) { return hipMalloc(p, n); }
+  static Error alloc_async(void **p, size_t n, Stream s) { return hipMallocAsync(p, n, s); }
+  static void free(void *p) { (void)hipFree(p); }
+  static bool wait(int device) {
+    int cur = device;
+    (void)hipGetDevice(&cur);
+    if (cur != device) (void)hipSetDevice(device);
+    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    if (!idle) (void)hipGetLastError();
+    if (cur != device) (void)hipSetDevice(cur);
+    return idle;
+  }
+  static void trim(int device) {
+    hipMemPool_t pool;
+    if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
+    (void)hipGetLastError();
+  }
 };
-std::mutex g_blocks_mu;
-std::vector<DevBlock> &kept_blocks() {  // oldest first; never destroyed (the driver is gone by then)
-  static auto *v = new std::vector<DevBlock>();
-  return *v;
+BlockCache<HipDriver> &block_cache() {  // never destroyed: the driver may be gone by then
+  static auto *c = new BlockCache<HipDriver>(HipDriver(), DEV_CACHE_BYTES);
+  return *c;
 }
 }  // namespace
 
 hipError_t dev_alloc(void **p, size_t n, size_t *block, int *device) {
-  hipError_t e = hipGetDevice(device);
-  if (e != hipSuccess) return e;
-  {
-    std::lock_guard<std::mutex> g(g_blocks_mu);
-    auto &v = kept_blocks();
-    size_t best = v.size();
-    for (size_t i = 0; i < v.size(); ++i)
-      if (v[i].device == *device && v[i].bytes >= n && v[i].bytes - n <= n / 4 &&
-          (best == v.size() || v[i].bytes < v[best].bytes))
-        best = i;
-    if (best < v.size()) {
-      *p = v[best].p;
-      *block = v[best].bytes;
-      v.erase(v.begin() + best);
-      return hipSuccess;
-    }
-  }
-  e = hipMalloc(p, n);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    dev_cache_release(*device);
-    e = hipMalloc(p, n);
-  }
-  *block = n;
-  return e;
+  const hipError_t e = hipGetDevice(device);
+  return e != hipSuccess ? e : block_cache().alloc(p, n, *device, block);
 }
 
-void dev_free(void *p, size_t block, int device) {
-  if (block > DEV_CACHE_BYTES) {
-    (void)hipFree(p);
-    return;
-  }
-  int cur = device;
-  (void)hipGetDevice(&cur);
-  if (cur != device) (void)hipSetDevice(device);
-  const bool idle = hipDeviceSynchronize() == hipSuccess;
-  if (cur != device) (void)hipSetDevice(cur);
-  std::vector<void *> out;
-  if (idle) {
-    std::lock_guard<std::mutex> g(g_blocks_mu);
-    auto &v = kept_blocks();
-    v.push_back({p, block, device});
-    size_t held = 0;
-    for (const auto &b : v) held += b.device == device ? b.bytes : 0;
-    for (size_t i = 0; i < v.size() && held > DEV_CACHE_BYTES;) {
-      if (v[i].device != device) { ++i; continue; }
-      held -= v[i].bytes;
-      out.push_back(v[i].p);
-      v.erase(v.begin() + i);
-    }
-  } else {
-    (void)hipGetLastError();
-    out.push_back(p);
-  }
-  for (void *q : out) (void)hipFree(q);
+hipError_t dev_alloc_async(void **p, size_t n, hipStream_t s) {
+  int device = 0;
+  const hipError_t e = hipGetDevice(&device);
+  return e != hipSuccess ? e : block_cache().alloc_async(p, n, device, s);
 }
 
-void dev_cache_release(int device) {
-  std::vector<void *> out;
-  {
-    std::lock_guard<std::mutex> g(g_blocks_mu);
-    auto &v = kept_blocks();
-    for (size_t i = 0; i < v.size();) {
-      if (v[i].device != device) { ++i; continue; }
-      out.push_back(v[i].p);
-      v.erase(v.begin() + i);
-    }
-  }
-  for (void *q : out) (void)hipFree(q);
-}
+void dev_free(void *p, size_t block, int device) { block_cache().free(p, block, device); }
+
+void dev_cache_release(int device) { block_cache().release(device); }
 
 // Fails with THG_E_INVALID unless every index of the nt triangles (device memory) is in [0, nv).
 void check_tri_indices(const int32_t *tris, int64_t nt, int64_t nv, hipStream_t s) {

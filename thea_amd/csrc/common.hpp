@@ -47,16 +47,15 @@ inline void require(bool ok, const std::string &msg) {
   if (!ok) fail(THG_E_INVALID, msg);
 }
 
-// Device memory blocks of DevBuf. A freed block is kept for the next allocation of about its size (at
-// least its request, at most a quarter more), up to DEV_CACHE_BYTES per device, oldest given back first;
-// all of a device's blocks are given back when one of its contexts is destroyed and before an
-// allocation is reported as failed. Like hipFree, dev_free waits for the device first, so a kept block
-// is idle and any stream or thread may take it.
+// Device memory of DevBuf and AsyncBuf. A freed DevBuf's block is kept for the next one of about its size
+// (block_cache.hpp), up to DEV_CACHE_BYTES per device; all of a device's blocks are given back when one
+// of its contexts is destroyed and before either kind of allocation is reported as failed.
 // Mapping and unmapping hundreds of megabytes for every mesh of a changing scene took 35 us per
 // hipMalloc and 170 us per hipFree at best, and from run to run 8 ms per build (the driver's share, in
 // whichever call came next).
 constexpr size_t DEV_CACHE_BYTES = (size_t)1 << 30;
 hipError_t dev_alloc(void **p, size_t n, size_t *block, int *device);
+hipError_t dev_alloc_async(void **p, size_t n, hipStream_t s);
 void dev_free(void *p, size_t block, int device);
 void dev_cache_release(int device);
 
@@ -129,7 +128,7 @@ struct AsyncBuf {
     reset();
     s = st;
     if (n == 0) return;
-    hipError_t e = hipMallocAsync(&p, n, s);
+    const hipError_t e = dev_alloc_async(&p, n, s);
     if (e != hipSuccess) {
       p = nullptr;
       (void)hipGetLastError();
