@@ -2,9 +2,20 @@
 // memory on each of two devices. Prints the name of each check that fails; exit status = their number.
 #include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <map>
+#include <new>
 
 #include "block_cache.hpp"
+
+static bool no_memory = false;  // host allocations fail
+void *operator new(std::size_t n) {
+  void *p = no_memory ? nullptr : std::malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, std::size_t) noexcept { std::free(p); }
 
 struct Model {
   size_t capacity = 1000, used[2] = {0, 0}, pooled[2] = {0, 0};
@@ -111,6 +122,20 @@ int main() {
     m.idle = false;
     k.free(p, b, 0);
     check(m.live.empty(), "a block whose device could not be waited for is not kept");
+  }
+  {
+    Model m;
+    Cache k(ModelDriver{&m}, 600);
+    k.alloc(&p, 100, 0, &b);
+    no_memory = true;
+    bool threw = false;
+    try {
+      k.free(p, b, 0);
+    } catch (const std::bad_alloc &) {
+      threw = true;
+    }
+    no_memory = false;
+    check(!threw && m.live.empty(), "without host memory to note a block, it is given back");
   }
   return bad;
 }

@@ -10,6 +10,7 @@
 
 #include <cstddef>
 #include <mutex>
+#include <new>
 #include <vector>
 
 namespace thg {
@@ -42,14 +43,11 @@ template <class Driver> class BlockCache {
     return e;
   }
 
-  void free(void *p, size_t block, int device) {
-    if (block > limit_ || !drv.wait(device)) {
+  // Called from destructors: nothing leaves it.
+  void free(void *p, size_t block, int device) noexcept {
+    if (block > limit_ || !drv.wait(device) || !keep(p, block, device)) {
       drv.free(p);
       return;
-    }
-    {
-      std::lock_guard<std::mutex> g(mu);
-      kept.push_back({p, block, device});
     }
     give_back(device, limit_);
   }
@@ -72,6 +70,17 @@ template <class Driver> class BlockCache {
   const size_t limit_;
   std::mutex mu;
   std::vector<Block> kept;  // oldest first
+
+  // False if there is no host memory to note the block.
+  bool keep(void *p, size_t block, int device) {
+    std::lock_guard<std::mutex> g(mu);
+    try {
+      kept.push_back({p, block, device});
+    } catch (const std::bad_alloc &) {
+      return false;
+    }
+    return true;
+  }
 
   bool take(void **p, size_t n, int device, size_t *block) {
     std::lock_guard<std::mutex> g(mu);
