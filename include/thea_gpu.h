@@ -65,6 +65,11 @@ const char *thg_version(void);
  * typical. Thea has no analogue (its queries run on the calling CPU thread). */
 int thg_ctx_create(int32_t device, thg_ctx *out);
 int thg_ctx_destroy(thg_ctx ctx);
+/* Gives back the device memory that the library holds but does not use on the context's device: the
+ * blocks of destroyed meshes and BVHs that it keeps for the next ones (at most 1 GiB; destroying a
+ * context gives them back too) and the idle part of the stream-ordered pool. For programs that
+ * rebuild rarely or whose other allocators need the memory. */
+int thg_ctx_trim(thg_ctx ctx);
 
 /* Upload a triangle mesh: `verts` = nv float3 (x,y,z interleaved), `tris` = nt int32 triplets of
  * vertex indices. Replaces MeshBvh::add / addTriangles and MeshTriangles::add

@@ -135,6 +135,8 @@ class Context {
   Context(const Context &) = delete;
   Context &operator=(const Context &) = delete;
   thg_ctx handle() const { return h_; }
+  // Gives back the device memory that is kept for the next meshes and BVHs.
+  void trim() { check(thg_ctx_trim(h_)); }
 
  private:
   thg_ctx h_ = nullptr;

@@ -81,6 +81,7 @@ def test_null_handles_of_the_feature_entry_points():
     assert lib.thg_proximity_graph(None, None, None, 1, None, None, None, None, None) == E
     assert lib.thg_icp_align(None, None, 0, 1, None, None, 1, None, None, None, None) == E
     assert lib.thg_bvh_bounds(None, None, None) == E
+    assert lib.thg_ctx_trim(None) == E
 
 
 def test_file_entry_points_report_errors(tmp_path):

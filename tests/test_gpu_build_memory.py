@@ -87,3 +87,32 @@ def test_blocks_are_given_back_with_a_context():
     ctx.close()
     # what is left: the stream-ordered pool's share of the build's temporaries (256 MB at most)
     assert free0 - torch.cuda.mem_get_info()[0] <= 300 << 20
+
+
+def test_trim_gives_back_kept_memory():
+    """The default context, which lives as long as the process, gives back what it keeps on request."""
+    import torch
+    import thea_amd
+    ctx = thea_amd.default_context()
+    v, t = _mesh(300_000, 1)
+
+    def build():
+        m = thea_amd.Mesh(v, t)
+        b = thea_amd.MeshBvh(m)
+        r = b.closestPoint(v[:1000])
+        b.close()
+        m.close()
+        return r
+
+    want = build()
+    ctx.trim()
+    free0 = torch.cuda.mem_get_info()[0]
+    build()
+    held = free0 - torch.cuda.mem_get_info()[0]
+    ctx.trim()
+    left = free0 - torch.cuda.mem_get_info()[0]
+    print(f"held {held >> 20} MB, after trim {left >> 20} MB", flush=True)
+    assert held >= 64 << 20  # the arrays over elements alone are 72 MB
+    assert left <= 8 << 20
+    for a, b in zip(build(), want):
+        assert np.array_equal(a, b)

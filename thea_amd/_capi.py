@@ -77,6 +77,7 @@ SIGNATURES = {
     "thg_version": (C.c_char_p, []),
     "thg_ctx_create": (C.c_int, [i32, C.POINTER(vp)]),
     "thg_ctx_destroy": (C.c_int, [vp]),
+    "thg_ctx_trim": (C.c_int, [vp]),
     "thg_mesh_create": (C.c_int, [vp, vp, i64, vp, i64, i32, C.POINTER(vp)]),
     "thg_mesh_destroy": (C.c_int, [vp]),
     "thg_mesh_num_triangles": (i64, [vp]),

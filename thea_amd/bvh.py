@@ -94,6 +94,10 @@ class Context:
         except Exception:
             pass
 
+    def trim(self):
+        """Give back the device memory that is kept for the next meshes and BVHs."""
+        capi.check(capi.lib().thg_ctx_trim(self.h))
+
     def set_timing(self, enable=True):
         """Record HIP events around every query/sampling kernel launched through this context."""
         capi.check(capi.lib().thg_ctx_set_timing(self.h, 1 if enable else 0))

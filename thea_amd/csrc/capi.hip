@@ -100,6 +100,8 @@ void dev_free(void *p, size_t block, int device) { block_cache().free(p, block, 
 
 void dev_cache_release(int device) { block_cache().release(device); }
 
+void dev_cache_reclaim(int device) { block_cache().reclaim(device); }
+
 // Fails with THG_E_INVALID unless every index of the nt triangles (device memory) is in [0, nv).
 void check_tri_indices(const int32_t *tris, int64_t nt, int64_t nv, hipStream_t s) {
   if (nt <= 0) return;
@@ -189,6 +191,14 @@ int thg_ctx_destroy(thg_ctx ctx) {
     const int device = c->device;
     delete c;
     dev_cache_release(device);
+  });
+}
+
+int thg_ctx_trim(thg_ctx ctx) {
+  return guarded([&] {
+    require(ctx != nullptr, "ctx is NULL");
+    set_device(reinterpret_cast<Ctx *>(ctx));
+    dev_cache_reclaim(reinterpret_cast<Ctx *>(ctx)->device);
   });
 }
 

@@ -49,7 +49,8 @@ inline void require(bool ok, const std::string &msg) {
 
 // Device memory of DevBuf and AsyncBuf. A freed DevBuf's block is kept for the next one of about its size
 // (block_cache.hpp), up to DEV_CACHE_BYTES per device; all of a device's blocks are given back when one
-// of its contexts is destroyed and before either kind of allocation is reported as failed.
+// of its contexts is destroyed, by thg_ctx_trim and before either kind of allocation is reported as
+// failed.
 // Mapping and unmapping hundreds of megabytes for every mesh of a changing scene took 35 us per
 // hipMalloc and 170 us per hipFree at best, and from run to run 8 ms per build (the driver's share, in
 // whichever call came next).
@@ -58,6 +59,7 @@ hipError_t dev_alloc(void **p, size_t n, size_t *block, int *device);
 hipError_t dev_alloc_async(void **p, size_t n, hipStream_t s);
 void dev_free(void *p, size_t block, int device);
 void dev_cache_release(int device);
+void dev_cache_reclaim(int device);  // the idle pool too
 
 // Owning device allocation, or a view into another one (view()).
 struct DevBuf {
