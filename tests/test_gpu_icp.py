@@ -96,6 +96,40 @@ def test_icp_problems_that_end_apart_equal_single(target):
         assert i1[0] == its[k] and e1[0] == err[k] and np.array_equal(t1[0], tr[k]), f"problem {k}"
 
 
+def test_icp_leaves_other_streams_running():
+    """Whatever its arrays take (340 MB here), an alignment waits for its own stream only."""
+    import time
+    import torch
+    import thea_amd
+    print("case icp beside another stream", flush=True)
+    g = np.random.default_rng(16)
+    src = _ellipsoid(g, 500_000).astype(np.float64)
+    bvh = thea_amd.PointBvh(_ellipsoid(g, 1000))
+    inits = np.repeat(_xf(np.eye(3), [0, 0, 0])[None], 10, 0)
+    icp = thea_amd.Icp3(min_iterations=1, max_iterations=1, kabsch=True)
+    icp.alignBatch(src, bvh, initial=inits)  # memory and code in place
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    torch.cuda._sleep(10_000_000)
+    torch.cuda.synchronize()
+    cycles = int(10_000_000 / (time.perf_counter() - t0))  # in one second, roughly
+    for _ in range(8):
+        s = torch.cuda.Stream()
+        done = torch.cuda.Event()
+        with torch.cuda.stream(s):
+            torch.cuda._sleep(cycles)
+            done.record()
+        bvh.closestPoint(np.zeros((1, 3), np.float32))
+        if done.query():  # shares a hardware queue with the default stream
+            continue
+        icp.alignBatch(src, bvh, initial=inits)
+        beside = not done.query()
+        torch.cuda.synchronize()
+        assert beside
+        return
+    pytest.skip("no stream runs beside the default stream")
+
+
 def test_icp_mesh_weights_up(oracle):
     import thea_amd
     from oracle import icp as I

@@ -144,6 +144,7 @@ struct AsyncBuf {
     bytes = 0;
   }
   template <typename T> T *as() const { return static_cast<T *>(p); }
+  template <typename T> T *at(size_t o) const { return reinterpret_cast<T *>(static_cast<char *>(p) + o); }
 };
 
 // Sizes of several arrays laid out in one allocation (each 256-byte aligned): add() every array, then
@@ -158,7 +159,8 @@ struct Layout {
 };
 
 // One allocation for a build's some 15 temporary arrays: up to WORKSPACE_POOL bytes from the device's
-// stream-ordered pool, more, which would stay in the pool, as a block of their own.
+// stream-ordered pool, more, which would stay in the pool, as a block of their own (whose release waits
+// for the device, as that of a build's temporaries always did).
 constexpr size_t WORKSPACE_POOL = (size_t)256 << 20;
 struct Workspace {
   AsyncBuf pooled;

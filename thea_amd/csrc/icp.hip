@@ -364,8 +364,7 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
   const size_t o_src = lay.add(n * K * 24), o_pos = lay.add(n * K * pb), o_q = lay.add(n * K * pb);
   const size_t o_idx = lay.add(n * K * 4), o_par = lay.add(K * (96 + 96 + 4)), o_res = lay.add(K * (56 + 72 + 8));
   const size_t o_part = lay.add((size_t)K * nb * ICP_MAXC * 8), o_sort = lay.add(sort_scratch_words(n * K) * 4);
-  Workspace mem;
-  mem.alloc(lay.total, s);
+  AsyncBuf mem(lay.total, s);  // stream-ordered whatever its size: freeing it waits for no other stream
   double *const src = mem.at<double>(o_src), *const cur = mem.at<double>(o_par), *const aux = cur + 12 * K;
   int32_t *const prob = reinterpret_cast<int32_t *>(aux + 12 * K);
   double *const sums7 = mem.at<double>(o_res), *const cov = sums7 + 7 * K, *const errs = cov + 9 * K;
@@ -610,10 +609,10 @@ extern "C" int thg_icp_align(thg_bvh to, const double *from, int64_t n, int32_t 
     // host arrays staged in one allocation
     const bool host = mem == THG_MEM_HOST;
     Layout lay;
-    Workspace staged;
+    AsyncBuf staged;
     const size_t o_from = lay.add((size_t)n * 24), o_init = lay.add(initial ? (size_t)K * 96 : 0);
     const size_t o_wt = lay.add(wt ? (size_t)n * 8 : 0), o_wr = lay.add(wr ? (size_t)n * 8 : 0);
-    if (host) staged.alloc(lay.total, s);
+    if (host) staged.ensure(lay.total, s);
     auto stage = [&](size_t o, const double *p, size_t count) -> const double * {
       if (!p || !host) return p;
       THG_HIP(hipMemcpyAsync(staged.at<double>(o), p, count * 8, hipMemcpyHostToDevice, s));
