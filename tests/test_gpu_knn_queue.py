@@ -88,3 +88,29 @@ def test_points_equal_wave_walk(leaf):
         _equal(b.closest(q[:n], want_d2=True), [x[:n] for x in ref], f"closest n={n}")
         _equal(b.kClosestElements(q[:n], 6, want_d2=True), [x[:n] for x in refk], f"k-NN n={n}")
     assert (b.closest(q[:50], dist_bound=0.0)[0] == -1).all()
+
+
+def test_more_threads_than_one_launch_holds():
+    """From 2^29 queries on, the 8 threads that a query of a list of more than 16 takes add up to more
+    than the 2^32 of one launch (51 GB here: 6 of queries, 37 of indices, 9 to sort them)."""
+    import torch
+    import thea_amd
+    from thea_amd import _capi as capi
+    n, k = (1 << 29) + 1_001, 17
+    if torch.cuda.mem_get_info()[0] < 80 << 30:
+        pytest.skip("needs 80 GB of device memory")
+    b = thea_amd.PointBvh(np.random.default_rng(1).random((40, 3), dtype=np.float32))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.rand(n, 3, generator=g, device="cuda")
+    idx = torch.full((n, k), -2, dtype=torch.int32, device="cuda")
+    print(f"case n={n} k={k}", flush=True)
+    stream = torch.cuda.current_stream().cuda_stream
+    capi.check(capi.lib().thg_k_closest(b.h, q.data_ptr(), n, k, -1.0, 0, idx.data_ptr(), None, None,
+                                        capi.THG_MEM_DEVICE, stream))
+    for a in range(0, n, 1 << 27):
+        assert bool((idx[a:a + (1 << 27)] >= 0).all()), a
+    for a in (0, (1 << 28) - 500, (1 << 29) - 500, n - 1_000):
+        assert torch.equal(idx[a:a + 1_000], b.kClosestElements(q[a:a + 1_000].contiguous(), k)[0]), a
+    del q, idx
+    torch.cuda.empty_cache()
+    b.ctx.trim()

@@ -1133,28 +1133,29 @@ __global__ void __launch_bounds__(WAVE) k_closest_queue(const BNode *__restrict_
                                                         const ScreenRec *__restrict__ scr,
                                                         const LeafBound *__restrict__ lbnd,
                                                         const float *__restrict__ q, const uint32_t *__restrict__ order,
-                                                        int64_t n, int lg, uint32_t nb_real, float best_init,
-                                                        float scale, int exclude_self, int32_t *__restrict__ out_idx,
-                                                        float *__restrict__ out_cp, float *__restrict__ out_dist,
-                                                        float *__restrict__ out_d2) {
+                                                        int64_t n, int lg, uint32_t nb_real, uint32_t wave0,
+                                                        float best_init, float scale, int exclude_self,
+                                                        int32_t *__restrict__ out_idx, float *__restrict__ out_cp,
+                                                        float *__restrict__ out_dist, float *__restrict__ out_d2) {
   __shared__ QueueWave s_w;
   const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
   if (lb_blk >= nb_real) return;
-  closest_queue_body(s_w, nodes, tr, scr, lbnd, q, order, n, (int64_t)lb_blk, lg, best_init, scale, exclude_self,
+  closest_queue_body(s_w, nodes, tr, scr, lbnd, q, order, n, (int64_t)wave0 + lb_blk, lg, best_init, scale, exclude_self,
                      out_idx, out_cp, out_dist, out_d2, 0);
 }
 
 // Many batches in one launch; the waves of a segment take 64 >> lanes_log2 queries each.
 __global__ void __launch_bounds__(WAVE) k_closest_queue_multi(const SegDesc *__restrict__ seg, int nseg,
-                                                              uint64_t total_waves, uint32_t nb_real) {
+                                                              uint32_t nb_real, uint32_t wave0) {
   __shared__ QueueWave s_w;
   const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
-  if (lb_blk >= nb_real || (uint64_t)lb_blk >= total_waves) return;
-  const int si = uni(find_segment(seg, nseg, (int64_t)lb_blk));
+  if (lb_blk >= nb_real) return;
+  const int64_t wave = (int64_t)wave0 + lb_blk;
+  const int si = uni(find_segment(seg, nseg, wave));
   const SegDesc &d = seg[si];
   closest_queue_body(s_w, readonly_ptr<BNode>(d.nodes), readonly_ptr<TriRec>(d.elems),
                      readonly_ptr<ScreenRec>(d.screen), readonly_ptr<LeafBound>(d.lbounds), readonly_ptr<float>(d.q),
-                     readonly_ptr<uint32_t>(d.order), d.n, (int64_t)lb_blk - (int64_t)d.wave_begin, d.lanes_log2,
+                     readonly_ptr<uint32_t>(d.order), d.n, wave - (int64_t)d.wave_begin, d.lanes_log2,
                      d.best_init, d.scale, d.exclude_self, d.idx, d.cp, d.dist, d.d2, d.root);
 }
 
@@ -1379,28 +1380,29 @@ __global__ void __launch_bounds__(WAVE) k_knn_queue(const BNode *__restrict__ no
                                                     const ScreenRec *__restrict__ scr,
                                                     const LeafBound *__restrict__ lbnd, const float *__restrict__ q,
                                                     const uint32_t *__restrict__ order, int64_t n, int lg,
-                                                    uint32_t nb_real, int k, float best_init, float scale,
-                                                    int exclude_self, int32_t *__restrict__ out_idx,
+                                                    uint32_t nb_real, uint32_t wave0, int k, float best_init,
+                                                    float scale, int exclude_self, int32_t *__restrict__ out_idx,
                                                     float *__restrict__ out_cp, float *__restrict__ out_dist,
                                                     float *__restrict__ out_d2, int32_t nelem) {
   __shared__ KnnWave s_w;
   const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
   if (lb_blk >= nb_real) return;
-  knn_queue_body<POINTS>(s_w, nodes, elems, scr, lbnd, q, order, n, (int64_t)lb_blk, lg, k, best_init, scale,
-                         exclude_self, out_idx, out_cp, out_dist, out_d2, nelem, 0);
+  knn_queue_body<POINTS>(s_w, nodes, elems, scr, lbnd, q, order, n, (int64_t)wave0 + lb_blk, lg, k, best_init,
+                         scale, exclude_self, out_idx, out_cp, out_dist, out_d2, nelem, 0);
 }
 
 // Many batches over mesh BVHs in one launch; the waves of a segment take 64 >> lanes_log2 queries each.
 __global__ void __launch_bounds__(WAVE) k_knn_queue_multi(const SegDesc *__restrict__ seg, int nseg,
-                                                          uint64_t total_waves, uint32_t nb_real) {
+                                                          uint32_t nb_real, uint32_t wave0) {
   __shared__ KnnWave s_w;
   const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
-  if (lb_blk >= nb_real || (uint64_t)lb_blk >= total_waves) return;
-  const int si = uni(find_segment(seg, nseg, (int64_t)lb_blk));
+  if (lb_blk >= nb_real) return;
+  const int64_t wave = (int64_t)wave0 + lb_blk;
+  const int si = uni(find_segment(seg, nseg, wave));
   const SegDesc &d = seg[si];
   knn_queue_body<false>(s_w, readonly_ptr<BNode>(d.nodes), readonly_ptr<TriRec>(d.elems),
                         readonly_ptr<ScreenRec>(d.screen), readonly_ptr<LeafBound>(d.lbounds), readonly_ptr<float>(d.q),
-                        readonly_ptr<uint32_t>(d.order), d.n, (int64_t)lb_blk - (int64_t)d.wave_begin, d.lanes_log2,
+                        readonly_ptr<uint32_t>(d.order), d.n, wave - (int64_t)d.wave_begin, d.lanes_log2,
                         d.k, d.best_init, d.scale, d.exclude_self, d.idx, nullptr, d.dist, d.d2, d.nelem, d.root);
 }
 
@@ -2511,29 +2513,31 @@ template <bool ANY>
 __global__ void __launch_bounds__(WAVE) k_ray_queue(const QNode4 *__restrict__ qn, const RayTri *__restrict__ rt,
                                                     const TriRec *__restrict__ tr, const float *__restrict__ orig,
                                                     const float *__restrict__ dirs, const uint32_t *__restrict__ order,
-                                                    int64_t n, int lg, uint32_t nb_real, float best_init,
-                                                    float max_time, float scale, int exact_only, int32_t *__restrict__ out_idx,
+                                                    int64_t n, int lg, uint32_t nb_real, uint32_t wave0,
+                                                    float best_init, float max_time, float scale, int exact_only,
+                                                    int32_t *__restrict__ out_idx,
                                                     float *__restrict__ out_t, float *__restrict__ out_n,
                                                     uint8_t *__restrict__ out_any) {
   __shared__ RayWave s_w;
   const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
   if (lb_blk >= nb_real) return;
-  ray_queue_body<ANY>(s_w, qn, rt, tr, orig, dirs, order, n, (int64_t)lb_blk, lg, best_init, max_time, scale, exact_only,
-                      out_idx, out_t, out_n, out_any);
+  ray_queue_body<ANY>(s_w, qn, rt, tr, orig, dirs, order, n, (int64_t)wave0 + lb_blk, lg, best_init, max_time, scale,
+                      exact_only, out_idx, out_t, out_n, out_any);
 }
 
 // Many first-hit ray batches in one launch over their meshes' ray trees; the waves of a segment take
 // 64 >> lanes_log2 rays each.
 __global__ void __launch_bounds__(WAVE) k_ray_queue_multi(const SegDesc *__restrict__ seg, int nseg,
-                                                          uint64_t total_waves, uint32_t nb_real) {
+                                                          uint32_t nb_real, uint32_t wave0) {
   __shared__ RayWave s_w;
   const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
-  if (lb_blk >= nb_real || (uint64_t)lb_blk >= total_waves) return;
-  const int si = uni(find_segment(seg, nseg, (int64_t)lb_blk));
+  if (lb_blk >= nb_real) return;
+  const int64_t wave = (int64_t)wave0 + lb_blk;
+  const int si = uni(find_segment(seg, nseg, wave));
   const SegDesc &d = seg[si];
   ray_queue_body<false>(s_w, readonly_ptr<QNode4>(d.qnodes), readonly_ptr<RayTri>(d.rays),
                         readonly_ptr<TriRec>(d.elems), readonly_ptr<float>(d.q), readonly_ptr<float>(d.q2),
-                        readonly_ptr<uint32_t>(d.order), d.n, (int64_t)lb_blk - (int64_t)d.wave_begin, d.lanes_log2,
+                        readonly_ptr<uint32_t>(d.order), d.n, wave - (int64_t)d.wave_begin, d.lanes_log2,
                         d.best_init, d.max_time, d.scale, q4_exact_only(d.scale), d.idx, d.dist, d.cp, nullptr);
 }
 
@@ -2791,6 +2795,18 @@ float bound_to_best(double dist_bound) {
   return prev_float(f);
 }
 
+// Launches of a work queue's waves, one workgroup each: launch(grid, waves, first wave). A launch holds
+// fewer than 2^32 threads per dimension, and a wave takes as few as 8 queries of a long k-NN list, so
+// from 2^29 queries on there are several.
+template <typename F> static void launch_queue(uint64_t waves, F launch) {
+  constexpr uint64_t MOST = (uint64_t)1 << 25;
+  for (uint64_t w = 0; w < waves; w += MOST) {
+    const uint32_t nb = (uint32_t)std::min(MOST, waves - w);
+    launch(dim3(round_up8(nb)), nb, (uint32_t)w);
+  }
+}
+static uint64_t queue_waves(int64_t n, int lg) { return (((uint64_t)n << lg) + WAVE - 1) / WAVE; }
+
 void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, int exclude_self, int32_t *idx,
                     float *cp, float *dist, float *d2, QueryScratch &ws, hipStream_t s) {
   if (n <= 0) return;
@@ -2802,22 +2818,23 @@ void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, 
   float best = bound_to_best(dist_bound);
   if (queue && !b.points) {
     const int lg = queue_lanes_log2(n);
-    const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE);
     KernelTimer kt(ws.timer_ctx(b.ctx), s, "closest");
-    hipLaunchKernelGGL(k_closest_queue, dim3(round_up8(qnb)), dim3(WAVE), 0, s, b.nodes.as<BNode>(),
-                       b.elems.as<TriRec>(), b.screen.as<ScreenRec>(), b.lbounds.as<LeafBound>(), q, ws.order, n, lg,
-                       qnb, best, b.scale, exclude_self, idx, cp, dist, d2);
+    launch_queue(queue_waves(n, lg), [&](dim3 g, uint32_t qnb, uint32_t w0) {
+      hipLaunchKernelGGL(k_closest_queue, g, dim3(WAVE), 0, s, b.nodes.as<BNode>(), b.elems.as<TriRec>(),
+                         b.screen.as<ScreenRec>(), b.lbounds.as<LeafBound>(), q, ws.order, n, lg, qnb, w0, best, b.scale,
+                         exclude_self, idx, cp, dist, d2);
+    });
     launch_check("k_closest_queue");
     kt.stop();
     return;
   }
   if (queue) {
     const int lg = knn_queue_lanes_log2(n, 1, true);
-    const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE);
     KernelTimer kt(ws.timer_ctx(b.ctx), s, "closest");
-    hipLaunchKernelGGL(k_knn_queue<true>, dim3(round_up8(qnb)), dim3(WAVE), 0, s, b.nodes.as<BNode>(), b.elems.p,
-                       nullptr, nullptr, q, ws.order, n, lg, qnb, 1, best, b.scale, exclude_self, idx, cp, dist, d2,
-                       (int32_t)b.n);
+    launch_queue(queue_waves(n, lg), [&](dim3 g, uint32_t qnb, uint32_t w0) {
+      hipLaunchKernelGGL(k_knn_queue<true>, g, dim3(WAVE), 0, s, b.nodes.as<BNode>(), b.elems.p, nullptr, nullptr, q,
+                         ws.order, n, lg, qnb, w0, 1, best, b.scale, exclude_self, idx, cp, dist, d2, (int32_t)b.n);
+    });
     launch_check("k_knn_queue");
     kt.stop();
     return;
@@ -2981,22 +2998,25 @@ void launch_knn_lane_multi(const SegDesc *seg_dev, int nseg, uint64_t total_wave
 
 void launch_closest_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s) {
   if (nseg <= 0 || total_waves == 0) return;
-  const uint32_t nb = (uint32_t)total_waves;
-  hipLaunchKernelGGL(k_closest_queue_multi, dim3(round_up8(nb)), dim3(WAVE), 0, s, seg_dev, nseg, total_waves, nb);
+  launch_queue(total_waves, [&](dim3 g, uint32_t nb, uint32_t w0) {
+    hipLaunchKernelGGL(k_closest_queue_multi, g, dim3(WAVE), 0, s, seg_dev, nseg, nb, w0);
+  });
   launch_check("k_closest_queue_multi");
 }
 
 void launch_knn_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s) {
   if (nseg <= 0 || total_waves == 0) return;
-  const uint32_t nb = (uint32_t)total_waves;
-  hipLaunchKernelGGL(k_knn_queue_multi, dim3(round_up8(nb)), dim3(WAVE), 0, s, seg_dev, nseg, total_waves, nb);
+  launch_queue(total_waves, [&](dim3 g, uint32_t nb, uint32_t w0) {
+    hipLaunchKernelGGL(k_knn_queue_multi, g, dim3(WAVE), 0, s, seg_dev, nseg, nb, w0);
+  });
   launch_check("k_knn_queue_multi");
 }
 
 void launch_ray_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s) {
   if (nseg <= 0 || total_waves == 0) return;
-  const uint32_t nb = (uint32_t)total_waves;
-  hipLaunchKernelGGL(k_ray_queue_multi, dim3(round_up8(nb)), dim3(WAVE), 0, s, seg_dev, nseg, total_waves, nb);
+  launch_queue(total_waves, [&](dim3 g, uint32_t nb, uint32_t w0) {
+    hipLaunchKernelGGL(k_ray_queue_multi, g, dim3(WAVE), 0, s, seg_dev, nseg, nb, w0);
+  });
   launch_check("k_ray_queue_multi");
 }
 
@@ -3066,16 +3086,17 @@ void launch_knn(const Bvh &b, const float *q, int64_t n, int k, double dist_boun
   float best = bound_to_best(dist_bound);
   if (queue) {
     const int lg = knn_queue_lanes_log2(n, k, b.points);
-    const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE);
     KernelTimer kt(b.ctx, s, "knn");
-    if (b.points)
-      hipLaunchKernelGGL(k_knn_queue<true>, dim3(round_up8(qnb)), dim3(WAVE), 0, s, b.nodes.as<BNode>(), b.elems.p,
-                         nullptr, nullptr, q, ws.order, n, lg, qnb, k, best, b.scale, exclude_self, idx, nullptr, dist,
-                         d2, (int32_t)b.n);
-    else
-      hipLaunchKernelGGL(k_knn_queue<false>, dim3(round_up8(qnb)), dim3(WAVE), 0, s, b.nodes.as<BNode>(), b.elems.p,
-                         b.screen.as<ScreenRec>(), b.lbounds.as<LeafBound>(), q, ws.order, n, lg, qnb, k, best, b.scale,
-                         exclude_self, idx, nullptr, dist, d2, (int32_t)b.n);
+    launch_queue(queue_waves(n, lg), [&](dim3 g, uint32_t qnb, uint32_t w0) {
+      if (b.points)
+        hipLaunchKernelGGL(k_knn_queue<true>, g, dim3(WAVE), 0, s, b.nodes.as<BNode>(), b.elems.p, nullptr, nullptr, q,
+                           ws.order, n, lg, qnb, w0, k, best, b.scale, exclude_self, idx, nullptr, dist, d2,
+                           (int32_t)b.n);
+      else
+        hipLaunchKernelGGL(k_knn_queue<false>, g, dim3(WAVE), 0, s, b.nodes.as<BNode>(), b.elems.p,
+                           b.screen.as<ScreenRec>(), b.lbounds.as<LeafBound>(), q, ws.order, n, lg, qnb, w0, k, best,
+                           b.scale, exclude_self, idx, nullptr, dist, d2, (int32_t)b.n);
+    });
     launch_check("k_knn_queue");
     kt.stop();
     return;
@@ -3131,13 +3152,14 @@ void launch_ray(const Bvh &b, const float *o, const float *d, int64_t n, float m
   KernelTimer kt(b.ctx, s, any ? "any_hit" : "ray");
   if (use_ray_queue(b)) {
     const int lg = ray_lanes_log2(n);
-    const uint32_t qnb = (uint32_t)ceil_div(n << lg, WAVE), qgrid = round_up8(qnb);
-#define THG_RQ(A)                                                                                                  \
-  hipLaunchKernelGGL(k_ray_queue<A>, dim3(qgrid), dim3(WAVE), 0, s, b.qnodes.as<QNode4>(), b.rays.as<RayTri>(),    \
-                     b.elems.as<TriRec>(), o, d, ws.order, n, lg, qnb, best, max_time, b.scale,                    \
+    launch_queue(queue_waves(n, lg), [&](dim3 g, uint32_t qnb, uint32_t w0) {
+#define THG_RQ(A)                                                                                            \
+  hipLaunchKernelGGL(k_ray_queue<A>, g, dim3(WAVE), 0, s, b.qnodes.as<QNode4>(), b.rays.as<RayTri>(),        \
+                     b.elems.as<TriRec>(), o, d, ws.order, n, lg, qnb, w0, best, max_time, b.scale,          \
                      q4_exact_only(b.scale), idx, t, nrm, hit)
-    if (any) THG_RQ(true); else THG_RQ(false);
+      if (any) THG_RQ(true); else THG_RQ(false);
 #undef THG_RQ
+    });
     launch_check("k_ray_queue");
     kt.stop();
     return;
