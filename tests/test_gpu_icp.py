@@ -96,6 +96,29 @@ def test_icp_problems_that_end_apart_equal_single(target):
         assert i1[0] == its[k] and e1[0] == err[k] and np.array_equal(t1[0], tr[k]), f"problem {k}"
 
 
+def test_icp_more_coordinates_than_one_launch_holds():
+    """63 of 64 problems search on with 23,000,000 points each: 1.45e9 correspondences, whose coordinates
+    are more than the 2^32 threads of one launch (118 GB)."""
+    import torch
+    import thea_amd
+    if torch.cuda.mem_get_info()[0] < 150 << 30:
+        pytest.skip("needs 150 GB of device memory")
+    print("case icp 63 x 23,000,000", flush=True)
+    g = np.random.default_rng(17)
+    to = _ellipsoid(g, 40)
+    src = to[np.arange(23_000_000) % len(to)].astype(np.float64)
+    move = _xf(_axis_rot([1, 2, 3], 0.9), [0.1, -0.1, 0.05])
+    inits = np.stack([_xf(np.eye(3), [0, 0, 0])] + 63 * [move])
+    bvh = thea_amd.PointBvh(to)
+    icp = thea_amd.Icp3(min_iterations=2, max_iterations=2, kabsch=True)
+    tr, err, its = icp.alignBatch(src, bvh, initial=inits)
+    t1, e1, i1 = icp.alignBatch(src, bvh, initial=inits[1:2])
+    torch.cuda.synchronize()
+    bvh.ctx.trim()
+    assert its[0] == 0 and i1[0] == 2 and np.all(its[1:] == 2)
+    assert np.all(err[1:] == e1[0]) and np.all(tr[1:] == t1[0])
+
+
 def test_icp_leaves_other_streams_running():
     """Whatever its arrays take (340 MB here), an alignment waits for its own stream only."""
     import time

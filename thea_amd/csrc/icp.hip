@@ -83,14 +83,16 @@ __global__ void __launch_bounds__(256) k_icp_pos(int64_t n, int A, const int32_t
   pos[3 * i + 2] = (T)z;
 }
 
-// q[prob[s] n + j] = tmp[s n + j]: the correspondences of a launch over part of the problems.
+// q[prob[s] n + j] = tmp[s n + j]: the correspondences of a launch over part of the problems, one thread
+// each like the searches (one per coordinate would exceed a launch's 2^32 threads three times as soon).
 template <typename T>
 __global__ void __launch_bounds__(256) k_icp_place(int64_t n, int A, const int32_t *__restrict__ prob,
                                                    const T *__restrict__ tmp, T *__restrict__ q) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= 3 * n * A) return;
-  const int64_t s = i / (3 * n);
-  q[3 * n * prob[s] + (i - s * 3 * n)] = tmp[i];
+  if (i >= n * A) return;
+  const int64_t s = i / n, o = n * prob[s] + (i - s * n);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) q[3 * o + a] = tmp[3 * i + a];
 }
 
 // Sums over the points of each active problem, with q the correspondences by problem (q[k n + j]).
@@ -418,7 +420,7 @@ void icp_align(const Bvh &to, const double *from, int64_t n, int K, const double
       launch_closest(to, (float *)pos, n * A, -1.0, 0, idx, (float *)out, nullptr, nullptr, ws, s);
     }
     if (!all) {
-      const dim3 g(ceil_div(3 * n * A, 256));
+      const dim3 g(ceil_div(n * A, 256));
       if (f64)
         hipLaunchKernelGGL(k_icp_place<double>, g, dim3(256), 0, s, n, A, prob, qtmp.as<double>(),
                            (double *)qpts);
