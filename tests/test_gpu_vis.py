@@ -42,3 +42,25 @@ def test_visibility_device_and_chunks(oracle):
     many = b.visibility(pos[:1700], num_rays=10000, seed=4, scale=2.0)
     assert np.array_equal(many, oracle.visibility(oracle.KdTree(v, t), pos[:1700], 10000, 2.0, 4))
     assert len(b.visibility(np.zeros((0, 3), np.float32))) == 0
+
+
+def test_one_ray_per_lane_sorts_its_rays(oracle):
+    """Where the work queue is not used (THG_RAY_Q4=0, read once per process), the rays are put in order,
+    one sort per chunk, and the fractions stay the same."""
+    import os
+    import subprocess
+    import sys
+    import thea_amd
+    from thea_amd import workloads as W
+    print("case visibility one ray per lane", flush=True)
+    code = ("import sys, numpy as np, thea_amd; from thea_amd import workloads as W;"
+            "v, t = W.torus(64, 32, seed=1); b = thea_amd.MeshBvh(thea_amd.Mesh(v, t)); b.ctx.set_timing(True);"
+            "x = b.visibility(v[:500], num_rays=64, seed=3);"
+            "print(b.ctx.kernel_time('order')[1], b.ctx.kernel_time('any_hit')[1], x.tobytes().hex())")
+    out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, THG_RAY_Q4="0"), capture_output=True,
+                         text=True, timeout=120, check=True,
+                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__)))).stdout.split()
+    assert out[0] == "1" and out[1] == "1"
+    v, t = W.torus(64, 32, seed=1)
+    b = thea_amd.MeshBvh(thea_amd.Mesh(v, t))
+    assert bytes.fromhex(out[2]) == b.visibility(v[:500], num_rays=64, seed=3).tobytes()

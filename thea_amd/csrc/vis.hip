@@ -125,9 +125,9 @@ extern "C" int thg_visibility(thg_bvh mesh_bvh, const float *positions, int64_t 
       launch_check("k_vis_rays");
       // In point order: neighbouring rays share their origin, which serves the work queue as well as a
       // sort by octant and origin did (1,000,000 points, 100 rays each, torus of 1,000,000 triangles: 28.3
-      // against 29.0 ms with the sort; one ray per lane, sorted, 34.1 ms).
+      // against 29.0 ms with the sort). One ray per lane is better sorted (65.2 against 72.2 ms there).
       launch_ray(*b, org.as<float>(), dir.as<float>(), m, -1.0f, true, nullptr, nullptr, nullptr, hit.as<uint8_t>(), ws,
-                 s, /*sort_rays=*/false);
+                 s, /*sort_rays=*/!use_ray_queue(*b));
       hipLaunchKernelGGL(k_vis_count, dim3(ceil_div(np, 256)), dim3(256), 0, s, hit.as<uint8_t>(), np, R,
                          d_vis + p0);
       launch_check("k_vis_count");
