@@ -2210,54 +2210,8 @@ __global__ void __launch_bounds__(Q_BLOCK) k_ray_multi(const SegDesc *__restrict
                                                  nullptr, d.root);
 }
 
-// Per-lane state of a ray (one ray per lane) and its set-up and output.
-struct RayLane {
-  float3 o, d, inv;
-  float3 olo, ohi;  // o + w and o - w: the widened slab planes are (lo - olo) * inv, (hi - ohi) * inv
-  float best;
-  int32_t bidx, bslot;
-  int64_t ri;
-};
-
-__device__ __forceinline__ void ray_lane_init(RayLane &L, const float *__restrict__ orig,
-                                              const float *__restrict__ dirs, int64_t ri, float best_init,
-                                              float scale) {
-  L.ri = ri;
-  L.o = load_q(orig, ri);
-  L.d = load_q(dirs, ri);
-  L.inv = f3(1.0f / L.d.x, 1.0f / L.d.y, 1.0f / L.d.z);
-  const float m = fmaxf(scale, fmaxf(fabsf(L.o.x), fmaxf(fabsf(L.o.y), fabsf(L.o.z))));
-  const float w = m * SLACK_REL;
-  L.olo = f3(L.o.x + w, L.o.y + w, L.o.z + w);
-  L.ohi = f3(L.o.x - w, L.o.y - w, L.o.z - w);
-  L.best = best_init;
-  L.bidx = 0x7fffffff;
-  L.bslot = -1;
-}
-
-template <bool ANY>
-__device__ __forceinline__ void ray_lane_finish(const RayLane &L, const TriRec *__restrict__ tr,
-                                                int32_t *__restrict__ out_idx, float *__restrict__ out_t,
-                                                float *__restrict__ out_n, uint8_t *__restrict__ out_any) {
-  const bool hit = L.bidx != 0x7fffffff;
-  if (ANY) {
-    out_any[L.ri] = hit ? 1 : 0;
-    return;
-  }
-  out_idx[L.ri] = hit ? L.bidx : -1;
-  if (out_t) out_t[L.ri] = hit ? L.best : -1.0f;
-  if (out_n) {
-    float nx = 0, ny = 0, nz = 0;
-    if (hit) { nx = tr[L.bslot].p0.w; ny = tr[L.bslot].p1.w; nz = tr[L.bslot].p2.w; }
-    out_n[3 * L.ri] = nx; out_n[3 * L.ri + 1] = ny; out_n[3 * L.ri + 2] = nz;
-  }
-}
-
 // Leaf end flag of a RayTri (int bits of b.w).
 __device__ __forceinline__ bool raytri_last(const float4 &b) { return __float_as_int(b.w) != 0; }
-
-// Node reference that ends a lane's traversal (~RAY_DONE would be leaf INT32_MAX: never a real one).
-constexpr int32_t RAY_DONE = INT32_MIN;
 
 __device__ __forceinline__ float q_byte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xffu); }
 
@@ -3137,12 +3091,10 @@ void launch_knn(const Bvh &b, const float *q, int64_t n, int k, double dist_boun
 }
 
 void launch_ray(const Bvh &b, const float *o, const float *d, int64_t n, float max_time, bool any, int32_t *idx,
-                float *t, float *nrm, uint8_t *hit, QueryScratch &ws, hipStream_t s, bool sort_rays,
-                const uint32_t *given_order) {
+                float *t, float *nrm, uint8_t *hit, QueryScratch &ws, hipStream_t s, bool sort_rays) {
   if (n <= 0) return;
   require(!b.points && (b.n == 0 || b.rays.p != nullptr), "ray queries need a triangle BVH");
-  if (!sort_rays) ws.order = given_order;
-  else if (order_ray_batch(b, n)) order_rays(b, o, d, n, ws, s);
+  if (sort_rays && order_ray_batch(b, n)) order_rays(b, o, d, n, ws, s);
   else ws.order = nullptr;
   uint32_t nb = ceil_div(n, Q_BLOCK);
   uint32_t grid = round_up8(nb);

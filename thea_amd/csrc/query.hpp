@@ -158,12 +158,10 @@ void launch_knn(const Bvh &b, const float *q, int64_t n, int k, double dist_boun
 // Per-wave statistics of the 16-nearest wave kernel on a point BVH (4 int64 per 64-query wave).
 void knn_wave_stats(const Bvh &b, const float *q, int64_t n, int exclude_self, int64_t *wstats, QueryScratch &ws,
                     hipStream_t s);
-// sort_rays = false traces the rays in the order given by given_order (ray given_order[j] in slot j;
-// nullptr: input order), for callers that make the rays coherent themselves. Results are always
-// written at the rays' input indices.
+// sort_rays = false traces the rays in input order, for callers whose rays are coherent as they come.
+// Results are always written at the rays' input indices.
 void launch_ray(const Bvh &b, const float *o, const float *d, int64_t n, float max_time, bool any, int32_t *idx,
-                float *t, float *nrm, uint8_t *hit, QueryScratch &ws, hipStream_t s, bool sort_rays = true,
-                const uint32_t *given_order = nullptr);
+                float *t, float *nrm, uint8_t *hit, QueryScratch &ws, hipStream_t s, bool sort_rays = true);
 
 // Sampler
 void mesh_cdf(Mesh &m, hipStream_t s);
