@@ -526,11 +526,7 @@ __device__ __forceinline__ void cmp_flush(CmpWave &W, const TriRec *__restrict__
   __builtin_amdgcn_wave_barrier();
 }
 
-// PF (batches too small to fill the GPU): a leaf's screening data (bounding spheres, normals and
-// plane offsets) arrives with one vector load per lane and is read per triangle with v_readlane, so
-// a wave waits once per leaf instead of once per triangle; large batches hide that latency with
-// other waves and keep the scalar loads, which cost no vector instructions.
-template <bool STATS, bool PF = false, bool LB = false>
+template <bool STATS, bool LB = false>
 __device__ __forceinline__ void closest_cmp_body(CmpWave &W, const BNode *__restrict__ nodes,
                                                  const TriRec *__restrict__ tr, const float *__restrict__ q,
                                                  const uint32_t *__restrict__ order, int64_t n, int64_t wave,
@@ -630,33 +626,16 @@ __device__ __forceinline__ void closest_cmp_body(CmpWave &W, const BNode *__rest
           ml &= ballot(!(leaf_lb2(dc2, sd, lt, lr, sl) > rej2));
           if (ml == 0) continue;
         }
-        float4 lsb = make_float4(0.0f, 0.0f, 0.0f, 0.0f), lpl = lsb;  // PF: lane j holds triangle f + j's
-        if (PF && lane < cnt) {
-          const ScreenRec *sj = scr + f + lane;
-          lsb = sj->c;
-          lpl = sj->n;
-        }
         for (int32_t k = f; k < f + cnt; ++k) {
           const ScreenRec *sk = scr + k;
           if (STATS) st_loaded++;
-          const int jl = k - f;
-          const float4 sbv = PF ? make_float4(lane_readf(lsb.x, jl), lane_readf(lsb.y, jl), lane_readf(lsb.z, jl),
-                                              lane_readf(lsb.w, jl))
-                                : make_float4(unif(sk->c.x), unif(sk->c.y), unif(sk->c.z), unif(sk->c.w));
+          const float4 sbv = make_float4(unif(sk->c.x), unif(sk->c.y), unif(sk->c.z), unif(sk->c.w));
           // conservative reject (fused multiply-adds: the slack dwarfs their rounding): the plane
-          // and disc bound. Large batches apply it alone (a bounding-sphere test first, to skip the
-          // plane's scalar loads, cost more than it saved: C3 18.1 against 19.4 ms per launch);
-          // prefetched leaves test the sphere first, which skips the plane's four lane reads when
-          // no lane passes (C1: 1.45 against 1.57 ms). sqrt(rej2) widened by 2^-20 covers the
-          // hardware square root's rounding.
+          // and disc bound alone (a bounding-sphere test first, to skip the plane's scalar loads,
+          // cost more than it saved: C3 18.1 against 19.4 ms per launch)
           const float dx = p.x - sbv.x, dy = p.y - sbv.y, dz = p.z - sbv.z;
           const float dc2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-          if (PF) {
-            const float T = fmaf(__builtin_amdgcn_sqrtf(rej2), 1.0f + 1.0f / 1048576.0f, fabsf(sbv.w));
-            if ((ballot(!(dc2 > T * T)) & ml) == 0) continue;
-          }
-          const float nx = PF ? lane_readf(lpl.x, jl) : unif(sk->n.x), ny = PF ? lane_readf(lpl.y, jl) : unif(sk->n.y);
-          const float nz = PF ? lane_readf(lpl.z, jl) : unif(sk->n.z);
+          const float nx = unif(sk->n.x), ny = unif(sk->n.y), nz = unif(sk->n.z);
           const float sd = fmaf(dx, nx, fmaf(dy, ny, dz * nz));
           // every lane computes the bound (no divergence); lanes that did not admit the leaf are
           // masked out of the ballot
@@ -740,7 +719,7 @@ __device__ __forceinline__ void closest_cmp_body(CmpWave &W, const BNode *__rest
 }
 
 // WAVES: resident waves per SIMD to compile for (1: the compiler's choice, 6 here, no spill).
-template <bool STATS = false, int WAVES = 1, bool PF = false>
+template <bool STATS = false, int WAVES = 1>
 __global__ void __launch_bounds__(W_BLOCK, WAVES) k_closest_cmp(const BNode *__restrict__ nodes, const TriRec *__restrict__ tr,
                                                          const float *__restrict__ q, const uint32_t *__restrict__ order,
                                                          int64_t n, uint32_t nb_real, float best_init, float scale,
@@ -754,9 +733,9 @@ __global__ void __launch_bounds__(W_BLOCK, WAVES) k_closest_cmp(const BNode *__r
   __shared__ CmpWave s_w[W_WAVES];
   const uint32_t lb_blk = xcd_remap(blockIdx.x, gridDim.x);
   const int64_t wave = (int64_t)lb_blk * W_WAVES + (threadIdx.x / WAVE);
-  closest_cmp_body<STATS, PF, true>(s_w[threadIdx.x / WAVE], nodes, tr, q, order, n, wave, lb_blk < nb_real,
-                                    best_init, scale, exclude_self, out_idx, out_cp, out_dist, out_d2, stats, 0,
-                                    child_order, lbnd, scr);
+  closest_cmp_body<STATS, true>(s_w[threadIdx.x / WAVE], nodes, tr, q, order, n, wave, lb_blk < nb_real,
+                               best_init, scale, exclude_self, out_idx, out_cp, out_dist, out_d2, stats, 0,
+                               child_order, lbnd, scr);
 }
 
 template <bool POINTS, int G, bool PRE, bool STATS = false>
@@ -2799,35 +2778,10 @@ void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, 
     uint32_t wgrid = round_up8(wnb);
     KernelTimer kt(ws.timer_ctx(b.ctx), s, "closest");
     if (wc.cmp && !b.points) {
-      // A batch whose waves all fit at once at 6 per SIMD gains nothing from more resident waves and
-      // would only pay the 8-wave build's spill (C1, 100k queries: 1.56 against 1.64 ms).
-      const bool one_round = ceil_div(n, (uint64_t)WAVE) <= (uint64_t)b.ctx->num_cus * 4 * 6;
       const uint32_t cgrid = round_up8(ceil_div(n, (uint64_t)W_BLOCK)), cnb = (uint32_t)ceil_div(n, (uint64_t)W_BLOCK);
-      // When every wave is resident at once, the walk's load latency is exposed: prefetch leaves
-      // (PF; C1, 100k queries: 1.55 -> 1.34 ms; 300k: 1.61 -> 1.36 ms). THG_LEAF_PREFETCH=0 or 1
-      // overrides, for either build.
-      static const int pf_env = env_int("THG_LEAF_PREFETCH", -1);
-      const bool pf = pf_env >= 0 ? pf_env != 0 : one_round;
-      if (!one_round && pf)
-        hipLaunchKernelGGL((k_closest_cmp<false, CMP_WAVES, true>), dim3(cgrid), dim3(W_BLOCK), 0, s,
-                           b.nodes.as<BNode>(), b.elems.as<TriRec>(), q, ws.order, n, cnb, best, b.scale, exclude_self,
-                           idx, cp, dist, d2, nullptr, b.child_order, b.lbounds.as<LeafBound>(),
-                           b.screen.as<ScreenRec>());
-      else if (one_round && pf)
-        hipLaunchKernelGGL((k_closest_cmp<false, 1, true>), dim3(cgrid), dim3(W_BLOCK), 0, s, b.nodes.as<BNode>(),
-                           b.elems.as<TriRec>(), q, ws.order, n, cnb, best, b.scale, exclude_self, idx, cp, dist, d2,
-                           nullptr, b.child_order, b.lbounds.as<LeafBound>(),
-                           b.screen.as<ScreenRec>());
-      else if (one_round)
-        hipLaunchKernelGGL((k_closest_cmp<false, 1>), dim3(cgrid), dim3(W_BLOCK), 0, s, b.nodes.as<BNode>(),
-                           b.elems.as<TriRec>(), q, ws.order, n, cnb, best, b.scale, exclude_self, idx, cp, dist, d2,
-                           nullptr, b.child_order, b.lbounds.as<LeafBound>(),
-                           b.screen.as<ScreenRec>());
-      else
-        hipLaunchKernelGGL((k_closest_cmp<false, CMP_WAVES>), dim3(cgrid), dim3(W_BLOCK), 0, s, b.nodes.as<BNode>(),
-                           b.elems.as<TriRec>(), q, ws.order, n, cnb, best, b.scale, exclude_self, idx, cp, dist, d2,
-                           nullptr, b.child_order, b.lbounds.as<LeafBound>(),
-                           b.screen.as<ScreenRec>());
+      hipLaunchKernelGGL((k_closest_cmp<false, CMP_WAVES>), dim3(cgrid), dim3(W_BLOCK), 0, s, b.nodes.as<BNode>(),
+                         b.elems.as<TriRec>(), q, ws.order, n, cnb, best, b.scale, exclude_self, idx, cp, dist, d2,
+                         nullptr, b.child_order, b.lbounds.as<LeafBound>(), b.screen.as<ScreenRec>());
       launch_check("k_closest_cmp");
       kt.stop();
       return;
