@@ -1016,9 +1016,12 @@ __device__ __forceinline__ void queue_screen(W_ &W, int lane, const ScreenRec *_
 }
 
 // Position in the batch of a lane's query. In a sorted batch below WQ_SPREAD_N queries, groups of
-// WQ_SPREAD waves deal their queries out like cards, so a cluster of hard queries falls on many waves
-// (150,000 queries in the box, torus of 1,048,576 triangles 958 -> 745 us; near the surface 230 ->
-// 238 us). From 500,000 on there are waves enough, and dealing only costs locality.
+// WQ_SPREAD waves deal their queries out like cards, so a cluster of hard queries falls on many waves.
+// Kernel time without and with dealing: queries in the box of a torus of 1,048,576 triangles 758 / 723 us
+// (150,000 of them), 1,030 / 1,015 (262,143), 1,393 / 1,422 (400,000), 2,455 / 2,455 (700,000); near its
+// surface 182 / 187, 283 / 279, 385 / 397, 483 / 498: there the gain ends at the line. A sphere of 20,480
+// triangles, whose hard queries lie together at its centre, gains on both sides of it: 1,018 / 597 us,
+// 1,170 / 758, 1,510 / 877, 2,588 / 1,391.
 constexpr int64_t WQ_SPREAD = 16, WQ_SPREAD_N = (int64_t)1 << 18;
 __device__ __forceinline__ int64_t queue_slot(int64_t wave, int lane, int Q, int64_t n, bool sorted) {
   if (!sorted || n >= WQ_SPREAD_N) return wave * Q + lane;
@@ -2312,7 +2315,7 @@ __device__ __forceinline__ void ray_queue_body(RayWave &W, const QNode4 *__restr
           } while (!last && !(ANY && bslot >= 0));
           if (bslot >= 0) {
             if (ANY) {
-              W.key[r] = ~0ull;  // negative bound: the ray's other pairs drop out
+              W.key[r] = ~0ull;  // a NaN bound: every compare with it fails, so the ray's other pairs drop out
             } else {
               atomicMin(&W.key[r], best);
               __builtin_amdgcn_wave_barrier();
@@ -2632,19 +2635,13 @@ bool order_ray_batch(const Bvh &b, int64_t n) {
 
 static float prev_float(float x) { return std::nextafter(x, -INFINITY); }
 
-// Traversal strategy for a batch of n point-proximity queries. One wave walking the tree for 64
-// sorted queries pays for the union of their search regions, which stays small only when the batch
-// is dense: at least about one query per 8 leaves (measured on spheres and tori of 0.1M-4M
-// triangles with queries uniform in the inflated box, where the cheaper of the two strategies
-// changes between 1/4 and 1/16 of a query per leaf). Sparser batches, and batches too small to be
-// spatially sorted, walk one query per lane. THG_TRAVERSAL=lane or =wave forces a strategy; trees
-// deeper than the lane-distributed stack always use lanes.
-bool use_wave_traversal(const Bvh &b, int64_t n) {
+// Point queries that do not take the work queue: one walk per wave, whose 64 sorted queries pay for the
+// union of their search regions (the queue's rules below leave it the dense batches, where that union
+// is small), or one query per lane. THG_TRAVERSAL=lane or =wave forces one; trees deeper than the
+// lane-distributed stack always use lanes.
+bool use_wave_traversal(const Bvh &b) {
   static const char *env = getenv("THG_TRAVERSAL");
-  if (b.max_depth >= W_STACK) return false;
-  if (env && std::string(env) == "lane") return false;
-  if (env && std::string(env) == "wave") return true;
-  return n >= ORDER_MIN_QUERIES && n >= b.num_leaves / 8;
+  return b.max_depth < W_STACK && !(env && std::string(env) == "lane");
 }
 
 // Closest triangles: the work-queue kernel or the compacted wave walk. One walk for 64 queries needs
@@ -2772,7 +2769,7 @@ void launch_closest(const Bvh &b, const float *q, int64_t n, double dist_bound, 
     kt.stop();
     return;
   }
-  if (use_wave_traversal(b, n)) {
+  if (use_wave_traversal(b)) {
     const WaveConfig wc = wave_config(b);
     uint32_t wnb = ceil_div(n, (uint64_t)W_WAVES * (WAVE / wc.g));
     uint32_t wgrid = round_up8(wnb);
@@ -3009,7 +3006,7 @@ void launch_knn(const Bvh &b, const float *q, int64_t n, int k, double dist_boun
     kt.stop();
     return;
   }
-  if (k <= 16 && use_wave_traversal(b, n)) {
+  if (k <= 16 && use_wave_traversal(b)) {
     uint32_t wnb = ceil_div(n, W_BLOCK);
     uint32_t wgrid = round_up8(wnb);
     KernelTimer kt(b.ctx, s, "knn");

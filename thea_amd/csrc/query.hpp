@@ -136,7 +136,7 @@ int queue_lanes_log2(int64_t n);
 void launch_knn_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s);
 bool use_knn_queue(const Bvh &b, int64_t n, int k);
 int knn_queue_lanes_log2(int64_t n, int k, bool points);
-bool use_wave_traversal(const Bvh &b, int64_t n);
+bool use_wave_traversal(const Bvh &b);
 // Rays by work queue, segments as above.
 void launch_ray_queue_multi(const SegDesc *seg_dev, int nseg, uint64_t total_waves, hipStream_t s);
 bool use_ray_queue(const Bvh &b);

@@ -149,7 +149,7 @@ static void worker_loop(Server *S, int wi) {
           const bool queue = r.r.type == THG_REQ_CLOSEST ? use_queue_traversal(*r.bvh, r.r.n)
                              : r.r.type == THG_REQ_KNN   ? use_knn_queue(*r.bvh, r.r.n, r.r.k)
                                                          : use_ray_queue(*r.bvh);
-          int lane = queue ? 2 : r.r.type != THG_REQ_RAY && !use_wave_traversal(*r.bvh, r.r.n) ? 1 : 0;
+          int lane = queue ? 2 : r.r.type != THG_REQ_RAY && !use_wave_traversal(*r.bvh) ? 1 : 0;
           groups[{r.r.type, lane, kk}].push_back(&r);
         }
       }
