@@ -250,16 +250,16 @@ int thg_batch_plan_run(thg_batch_plan plan, const float *verts, const int32_t *t
                        int32_t *idx, float *dist, void *stream, double timings_ms[2]);
 int thg_batch_plan_destroy(thg_batch_plan plan);
 /* Leaf size per mesh chosen by measurement: for each size class (floor(log2(triangles))) the
- * plan's closest-point kernel is timed on up to two of its meshes for leaf sizes 2..16 and the
+ * closest-point kernel that the plan runs there is timed on up to two of its meshes for leaf sizes 2..16 and the
  * fastest is kept (cached for the process). Same inputs as thg_batch_closest; writes leaf_sizes[nm]. */
 int thg_autotune_leaf(thg_ctx ctx, int32_t nm, const int64_t *nv, const int64_t *nt, const int64_t *nq,
                       const float *verts, const int32_t *tris, const float *queries, int32_t *leaf_sizes);
 /* Leaf size and child visiting order per mesh, and the launch shape of the plan, chosen by
- * measurement. Per size class, as thg_autotune_leaf, then at that leaf size the child order
- * (child_orders[m]: 0 = the child most of a wave's queries find nearer, 1 = the child with the least
+ * measurement. Per size class, as thg_autotune_leaf, then at that leaf size the child order, for meshes
+ * whose queries are dense enough for the wave walk that has one (child_orders[m]: 0 = the child most of a wave's queries find nearer, 1 = the child with the least
  * lower bound over the wave's queries, 2 = the build's order; cached per class). Then launch[0] =
  * waves per workgroup of the query launch (1, 2, 4, 8) and launch[1] = 1 for the build compiled for 8
- * resident waves per SIMD (0: the spill-free one), the fastest summed over the sampled meshes.
+ * resident waves per SIMD (0: the spill-free one), the fastest summed over those sampled meshes.
  * Results never depend on these choices, only the time does. No counterpart in Thea. */
 int thg_autotune_plan(thg_ctx ctx, int32_t nm, const int64_t *nv, const int64_t *nt, const int64_t *nq,
                       const float *verts, const int32_t *tris, const float *queries, int32_t *leaf_sizes,

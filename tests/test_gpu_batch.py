@@ -93,6 +93,32 @@ def test_autotune_and_one_shot():
     print(f"autotuned leaf sizes {leaf.tolist()}")
 
 
+def test_autotune_times_the_kernel_that_the_plan_runs():
+    """Visiting orders and launch shapes belong to the wave walk: a plan whose meshes all take the work
+    queue keeps the defaults instead of picking among equal timings; a mesh with 800,000 queries takes
+    the wave walk and is tuned apart from one of its size class that does not."""
+    import torch
+    from thea_amd.batch import BatchPlan, autotune_plan, concat
+    print("case batch autotune by kernel", flush=True)
+    sizes = [400, 900, 1800, 3600, 7200, 14400]
+    meshes, queries = _batch(7, sizes, [30_000] * len(sizes))
+    nv, nt, nq, verts, tris, qs = concat(meshes, queries)
+    V, T, Q = (torch.from_numpy(x).cuda() for x in (verts, tris, qs))
+    leaf, order, launch = autotune_plan(nv, nt, nq, V, T, Q)
+    assert np.all((leaf >= 2) & (leaf <= 16)) and not order.any() and launch == (4, 1), (order, launch)
+    meshes, queries = _batch(8, [900, 930], [800_000, 3_000])
+    nv, nt, nq, verts, tris, qs = concat(meshes, queries)
+    V, T, Q = (torch.from_numpy(x).cuda() for x in (verts, tris, qs))
+    leaf, order, launch = autotune_plan(nv, nt, nq, V, T, Q)
+    assert order[1] == 0
+    plan = BatchPlan(nv, nt, nq, leaf_sizes=leaf, child_orders=order, launch=launch)
+    for _ in range(2):
+        idx, dist = plan.run(V, T, Q)
+        torch.cuda.synchronize()
+        _check(meshes, queries, idx.cpu().numpy(), dist.cpu().numpy())
+    plan.close()
+
+
 def test_c4_full_size_oracle(oracle):
     """The 512-mesh workload the benchmark runs (42.7M triangles, 20.4M queries), autotuned leaf sizes,
     through the captured graph: the first 256 queries of every mesh bit-exact against the oracle's
@@ -138,11 +164,12 @@ def test_c4_full_size_oracle(oracle):
 
 
 def test_child_orders_and_launch_shapes_change_no_result():
-    """Every child visiting order and query launch shape the tuner may pick gives the same bits."""
+    """Every child visiting order and query launch shape the tuner may pick gives the same bits (the
+    800,000 queries on 1,000 triangles take the wave walk, which has them)."""
     import torch
     from thea_amd.batch import BatchPlan, concat
     sizes = [17, 1000, 5000, 20000, 60000, 300]
-    qsizes = [1000, 5000, 20000, 30000, 40000, 1]
+    qsizes = [1000, 800_000, 20000, 30000, 40000, 1]
     print("case batch orders and shapes", flush=True)
     meshes, queries = _batch(3, sizes, qsizes)
     nv, nt, nq, verts, tris, qs = concat(meshes, queries)

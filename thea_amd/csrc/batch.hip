@@ -418,13 +418,13 @@ static void check_batch_indices(const int32_t *tris, int nm, const int64_t *nv, 
 static std::mutex g_tune_mu;
 static std::map<int, int> g_tuned_leaf, g_tuned_order;
 
-// The plan's query launch for one mesh alone: its queries spatially sorted, one segment, the given
-// visiting order and launch shape; returns the average time of `reps` launches after one warm-up.
-static double time_plan_kernel(const Bvh &b, const float *q, int64_t n, int child_order, int block_waves, bool spill,
-                               int reps, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+// The plan's query launch for one mesh alone: by work queue or by wave walk (with the given visiting
+// order and launch shape), one segment, its queries sorted as the plan sorts them; returns the average
+// time of `reps` launches after one warm-up.
+static double time_plan_kernel(const Bvh &b, const float *q, int64_t n, bool queue, int child_order, int block_waves,
+                               bool spill, int reps, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
   QueryScratch ws;
   ws.timed = false;
-  const bool queue = use_queue(n, b.n, 0);
   if (!queue || n > QUEUE_UNSORTED_MAX) order_queries(b, q, n, ws, s);
   AsyncBuf oi(n * 4, s), od(n * 4, s), dseg(sizeof(SegDesc), s);
   SegDesc d{};
@@ -444,7 +444,7 @@ static double time_plan_kernel(const Bvh &b, const float *q, int64_t n, int chil
   THG_HIP(hipMemcpyAsync(dseg.p, &d, sizeof(SegDesc), hipMemcpyHostToDevice, s));
   const uint64_t waves = (uint64_t)(((n << d.lanes_log2) + SEG_WAVE_QUERIES - 1) / SEG_WAVE_QUERIES);
   auto launch = [&] {
-    if (d.lanes_log2) launch_closest_queue_multi(dseg.as<SegDesc>(), 1, waves, s);
+    if (queue) launch_closest_queue_multi(dseg.as<SegDesc>(), 1, waves, s);
     else launch_closest_multi(dseg.as<SegDesc>(), 1, waves, false, s, false, block_waves, spill);
   };
   launch();
@@ -627,12 +627,13 @@ int thg_batch_plan_run(thg_batch_plan plan, const float *verts, const int32_t *t
 
 namespace thg {
 
-// Per size class (floor(log2 triangles)): the leaf size (2..16), then at that leaf size the child
-// visiting order (CHILD_*), each the fastest for the plan's query kernel on up to two sampled
-// meshes of the class (the largest query batches, up to 262,144 queries each); both cached for the
-// process. Then, if `launch` is given, the launch shape of the whole plan (waves per workgroup 1, 2,
-// 4 or 8; the spill-free or the 8-resident-wave build), the fastest summed over every class's sampled
-// meshes at their tuned leaf sizes and orders. A leaf size whose tree is too deep for the query
+// Per size class (floor(log2 triangles)) and kernel that the plan runs on the mesh (use_queue): the leaf
+// size (2..16), then at that leaf size the child visiting order (CHILD_*), each the fastest for that
+// kernel on up to two sampled meshes of the class (the largest query batches, up to 262,144 queries
+// each); both cached for the process. Then, if `launch` is given, the launch shape of the whole plan
+// (waves per workgroup 1, 2, 4 or 8; the spill-free or the 8-resident-wave build), the fastest summed over
+// every class's sampled meshes at their tuned leaf sizes and orders. Visiting order and launch shape
+// belong to the wave walk: meshes of the work queue keep CHILD_MAJORITY and do not vote on the shape. A leaf size whose tree is too deep for the query
 // kernel's 64-entry stack on a sampled mesh is not a candidate.
 static void autotune_plan(Ctx *c, int32_t nm, const int64_t *nv, const int64_t *nt, const int64_t *nq,
                           const float *verts, const int32_t *tris, const float *queries, int32_t *leaf_sizes,
@@ -645,7 +646,7 @@ static void autotune_plan(Ctx *c, int32_t nm, const int64_t *nv, const int64_t *
     if (nt[m] <= 0) continue;
     int b = 0;
     while ((int64_t(1) << (b + 1)) <= nt[m]) ++b;
-    buckets[b].push_back(m);
+    buckets[2 * b + (use_queue(nq[m], nt[m], 0) ? 1 : 0)].push_back(m);
   }
   const int leaves[] = {2, 4, 6, 8, 12, 16};
   const int REPS = 3;
@@ -678,13 +679,14 @@ static void autotune_plan(Ctx *c, int32_t nm, const int64_t *nv, const int64_t *
     return b;
   };
   for (auto &kv : buckets) {
-    int best_leaf = 0, best_order = -1;
+    const bool queue = kv.first & 1;
+    int best_leaf = 0, best_order = queue ? CHILD_MAJORITY : -1;
     {
       std::lock_guard<std::mutex> g(g_tune_mu);
       auto it = g_tuned_leaf.find(kv.first);
       if (it != g_tuned_leaf.end()) best_leaf = it->second;
       auto io = g_tuned_order.find(kv.first);
-      if (io != g_tuned_order.end()) best_order = io->second;
+      if (!queue && io != g_tuned_order.end()) best_order = io->second;
     }
     std::vector<int> ms = kv.second;
     ms.erase(std::remove_if(ms.begin(), ms.end(), [&](int m) { return nq[m] <= 0; }), ms.end());
@@ -699,8 +701,8 @@ static void autotune_plan(Ctx *c, int32_t nm, const int64_t *nv, const int64_t *
         for (int m : ms) {
           std::unique_ptr<Bvh> b = build(m, leaf);
           if (b->max_depth >= 64) { timed_all = false; break; }
-          tot += time_plan_kernel(*b, queries + 3 * qo[m], std::min<int64_t>(nq[m], 262144), CHILD_MAJORITY, 4, true,
-                                  REPS, s, R.e0, R.e1);
+          tot += time_plan_kernel(*b, queries + 3 * qo[m], std::min<int64_t>(nq[m], 262144), queue, CHILD_MAJORITY, 4,
+                                  true, REPS, s, R.e0, R.e1);
         }
         if (timed_all && tot < best_ms) { best_ms = tot; best_leaf = leaf; }
       }
@@ -709,7 +711,7 @@ static void autotune_plan(Ctx *c, int32_t nm, const int64_t *nv, const int64_t *
       g_tuned_leaf[kv.first] = best_leaf;
     }
     std::vector<Sampled> here;
-    if ((child_orders && best_order < 0) || launch) {
+    if (!queue && ((child_orders && best_order < 0) || launch)) {
       for (int m : ms) {
         std::unique_ptr<Bvh> b = build(m, best_leaf);
         if (b->max_depth >= 64) continue;
@@ -721,7 +723,7 @@ static void autotune_plan(Ctx *c, int32_t nm, const int64_t *nv, const int64_t *
       for (int order : {CHILD_MAJORITY, CHILD_LEADER, CHILD_BUILD}) {
         double tot = 0;
         for (auto &x : here)
-          tot += time_plan_kernel(*x.b, queries + 3 * qo[x.m], x.n, order, 4, true, REPS, s, R.e0, R.e1);
+          tot += time_plan_kernel(*x.b, queries + 3 * qo[x.m], x.n, false, order, 4, true, REPS, s, R.e0, R.e1);
         if (tot < best_ms) { best_ms = tot; best_order = order; }
       }
       if (here.empty()) best_order = CHILD_MAJORITY;
@@ -749,7 +751,8 @@ static void autotune_plan(Ctx *c, int32_t nm, const int64_t *nv, const int64_t *
       for (int bw : {1, 2, 4, 8}) {
         double tot = 0;
         for (auto &x : all)
-          tot += time_plan_kernel(*x.b, queries + 3 * qo[x.m], x.n, x.order, bw, spill != 0, REPS, s, R.e0, R.e1);
+          tot += time_plan_kernel(*x.b, queries + 3 * qo[x.m], x.n, false, x.order, bw, spill != 0, REPS, s, R.e0,
+                                  R.e1);
         if (!all.empty() && tot < best_ms) {
           best_ms = tot;
           launch[0] = bw;
