@@ -1,9 +1,8 @@
 """GPU tests of the BVH build: the exported tree is a partition of the elements into leaves, and
 every child box is exactly the union of what it holds (tight, so it both contains its elements and
-adds nothing). Covers the span-local and straddling parts of the refit (trees larger than one
-1024-element span, many spans, duplicate Morton codes) and the serial atomic refit it replaces."""
-import os
-
+adds nothing). Sizes from a single leaf to 4.6M elements, with duplicate Morton codes and a 1,048,576
+triangle mesh: boxes come from the aligned runs of sorted elements that tile a node's range, whose
+levels above the eighth are made by launches of their own."""
 import numpy as np
 import pytest
 
@@ -85,9 +84,7 @@ def test_point_tree_with_duplicates():
     _check_tree(b, p, p)
 
 
-def test_c3_tree_exact_and_refits_agree():
-    import subprocess
-    import sys
+def test_c3_tree_exact():
     import thea_amd
     from thea_amd import workloads as W
     print("case build C3 torus", flush=True)
@@ -95,24 +92,13 @@ def test_c3_tree_exact_and_refits_agree():
     b = thea_amd.MeshBvh(thea_amd.Mesh(v, t))
     elo, ehi = _tri_boxes(v, t)
     _check_tree(b, elo, ehi)
-    # the serial atomic refit (THG_REFIT=1, read once per process) builds the same tree
-    code = ("import sys, numpy as np, thea_amd; from thea_amd import workloads as W;"
-            "v,t,_,_,_=W.torus_c3(n_queries=0,n_rays=0); b=thea_amd.MeshBvh(thea_amd.Mesh(v,t));"
-            "f,i,ids=b.export(); np.save(sys.stdout.buffer, i, allow_pickle=False)")
-    env = dict(os.environ, THG_REFIT="1")
-    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, timeout=120, check=True,
-                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__)))).stdout
-    import io
-    other = np.load(io.BytesIO(out), allow_pickle=False)
-    f, i, _ = b.export()
-    assert np.array_equal(other, i)
 
 
-def test_level_refit_large_point_tree():
-    """Over 4M elements (4096 spans of 1024) the refit finishes the top tree level by level, one
-    launch per level; clustered and duplicated points make the tree unbalanced and deep."""
+def test_large_point_tree():
+    """4.6M elements take 22 levels of runs (two launches above the record kernel's eight); clustered and
+    duplicated points make the tree unbalanced and deep."""
     import thea_amd
-    print("case build 4.6M points (level refit)", flush=True)
+    print("case build 4.6M points", flush=True)
     g = np.random.default_rng(23)
     n = 4_600_000
     p = g.random((n, 3)).astype(np.float32)

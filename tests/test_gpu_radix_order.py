@@ -3,7 +3,9 @@
 Build: a point BVH's leaf order is the stable order of the points' 30-bit Morton codes, so it must
 equal numpy's stable argsort of codes computed with the same float operations. Queries: a batch and
 its reverse visit different orders of the same queries, so every query's answer must be the same
-bits either way (an order that lost or repeated a query would leave one unanswered).
+bits either way (an order that lost or repeated a query would leave one unanswered). Float batches are
+sorted above 131,072 queries, double ones from 4,096 on; ray batches only above 2^22 on trees of more
+than 256 MB (test_gpu_ray_queue.py).
 """
 import numpy as np
 import pytest
@@ -37,7 +39,7 @@ def test_build_order_is_the_stable_morton_order(n):
     assert np.array_equal(ids, np.argsort(_morton(p), kind="stable").astype(np.int32))
 
 
-@pytest.mark.parametrize("n", [4_096, 4_097, 100_001, (1 << 18) - 1, 1 << 18, (1 << 20) + 1, 2_500_001])
+@pytest.mark.parametrize("n", [131_073, 200_001, (1 << 18) - 1, 1 << 18, 786_433, 1 << 20, (1 << 20) + 1, 2_500_001])
 def test_query_order_answers_every_query(n):
     import torch
     import thea_amd
@@ -46,11 +48,16 @@ def test_query_order_answers_every_query(n):
     bvh = thea_amd.MeshBvh(thea_amd.Mesh(v, t))
     g = torch.Generator(device="cuda").manual_seed(n)
     q = (torch.rand(n, 3, generator=g, device="cuda") - 0.5) * 3.5
-    d = torch.randn(n, 3, generator=g, device="cuda")
-    i0, t0, _ = bvh.rayStructureIntersection(q, d, want_normal=False)
-    i1, t1, _ = bvh.rayStructureIntersection(q.flip(0), d.flip(0), want_normal=False)
-    assert torch.equal(i0, i1.flip(0)) and torch.equal(t0, t1.flip(0))
-    if n <= 1 << 20:
-        i0, d0 = bvh.closestElementWithDistance(q)
-        i1, d1 = bvh.closestElementWithDistance(q.flip(0))
-        assert torch.equal(i0, i1.flip(0)) and torch.equal(d0, d1.flip(0))
+    i0, d0 = bvh.closestElementWithDistance(q)
+    i1, d1 = bvh.closestElementWithDistance(q.flip(0))
+    assert torch.equal(i0, i1.flip(0)) and torch.equal(d0, d1.flip(0))
+
+
+@pytest.mark.parametrize("n", [4_096, 4_097, 65_537, 100_001, (1 << 20) + 1])
+def test_double_query_order_answers_every_query(n):
+    import thea_amd
+    g = np.random.default_rng(n)
+    bvh = thea_amd.PointBvhF64(g.normal(size=(5_000, 3)))
+    q = g.normal(size=(n, 3))
+    for a, b in zip(bvh.closest(q)[:3], bvh.closest(q[::-1])[:3]):
+        assert np.array_equal(a, b[::-1])

@@ -3,9 +3,9 @@
 Bar: indices, closest points, distances and squared distances bit-identical to the allocating entry
 point on the same inputs. Calls run back to back on one stream, each on a batch smaller than or
 different from the one before, so a result that depended on what an earlier call left in the
-shared sort memory would differ. Covers the sorted wave path at 8 and at 1 resident waves per SIMD
-(batches above and below 256 CUs x 24 waves x 64 queries), a bounded search, an unsorted sparse
-batch, a point BVH, and the size limit.
+shared sort memory would differ. Covers the sorted wave walk (more than 1.25 queries per triangle), the
+work queue sorted and as they come (up to 131,072 queries), a bounded search, a point BVH (a wave walk
+above 131,072 queries here), and the size limit.
 """
 import ctypes as C
 
@@ -53,9 +53,10 @@ def test_noalloc_equals_closest_point():
     b = thea_amd.MeshBvh(thea_amd.Mesh(v, t), leaf_size=8)
     qd = torch.from_numpy(q).cuda()
     stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    # (first query, count, bound): 8-wave sorted batch, then smaller and different ones
-    cases = [(0, 1_000_000, -1.0), (1_000_000, 150_000, -1.0), (1_150_000, 300_000, 0.05), (1_450_000, 2_000, -1.0),
-             (1_452_000, 4_096, -1.0)]
+    # (first query, count, bound): wave walk, then smaller and different batches
+    cases = [(0, 1_320_000, -1.0), (1_320_000, 150_000, -1.0), (1_470_000, 200_000, 0.05), (1_670_000, 2_000, -1.0),
+             (1_672_000, 4_096, -1.0)]
+    assert cases[0][1] > 1.25 * len(t)
     for first, n, bound in cases:
         label = f"C3 torus leaf 8, queries [{first}, {first + n}), bound {bound}"
         print(f"case {label}", flush=True)
@@ -73,11 +74,11 @@ def test_noalloc_point_bvh_and_empty_batch():
     thea_amd.default_context(0)
     g = np.random.default_rng(5)
     pts = g.normal(size=(200_000, 3)).astype(np.float32)
-    q = g.uniform(-2, 2, size=(120_000, 3)).astype(np.float32)
+    q = g.uniform(-2, 2, size=(140_000, 3)).astype(np.float32)
     b = thea_amd.PointBvh(pts, leaf_size=4)
     qd = torch.from_numpy(q).cuda()
     stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    for n in (120_000, 50_000):
+    for n in (140_000, 50_000):
         print(f"case point BVH 200k points x {n} queries", flush=True)
         got = _call(L, "noalloc", b, qd[:n], n, -1.0, stream)
         want = _call(L, "alloc", b, qd[:n], n, -1.0, stream)
