@@ -119,7 +119,7 @@ def test_slivers_and_near_collinear(oracle, nq):
     perturbed by float rounding), thin slivers and ordinary ones, far from the origin as well, with
     queries on and just off them: the plane-and-disc pruning bound must fall back to the bounding
     sphere wherever the stored plane is not tight. 790,000 queries take the wave walk (more than
-    786,432), 30,000 the work queue; their 6 nearest likewise (more than 262,144)."""
+    449,536 on 6,000 triangles), 30,000 the work queue; their 6 nearest likewise (more than 242,304)."""
     g = np.random.default_rng(19)
     n = 6000
     off = np.repeat(g.choice([0.0, 1.0, 300.0], size=(n // 3, 1)), 3, axis=0) * g.normal(size=(n, 3))

@@ -1,7 +1,8 @@
 """The work-queue closest-triangle kernel against the compacted wave walk and the oracle.
 
-Batches of up to max(1.25 queries per triangle, 786,432) take the queue, larger ones the wave walk,
-and both must give the canonical bits. Sizes are the edges of its waves (1 to 32 queries per wave)
+Batches of up to 1.25 queries per triangle take the queue, and on small meshes up to 65,536 + 64 per
+triangle (at least 131,072, at most 786,432); larger ones take the wave walk, and both must give the
+canonical bits. Sizes are the edges of its waves (1 to 32 queries per wave)
 and of its rule; the equidistant sphere makes every query at its centre meet the whole tree, so the
 stack runs into its throttle.
 """
@@ -10,7 +11,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-WAVE_N = 786_433  # the smallest batch of a small mesh that takes the wave walk
+WAVE_N = 786_433  # takes the wave walk on every mesh of fewer than 629,146 triangles
 
 
 def _equal(a, b, label):
@@ -22,7 +23,7 @@ def _equal(a, b, label):
 def torus(request):
     import thea_amd
     from thea_amd import workloads as W
-    v, t = W.torus(64, 32)
+    v, t = W.torus(128, 64)  # 16,384 triangles: the queue up to WAVE_N - 1
     b = thea_amd.MeshBvh(thea_amd.Mesh(v, t), leaf_size=request.param)
     g = np.random.default_rng(7)
     lo, hi = W.inflated_box(v, 1.2)

@@ -1,8 +1,8 @@
 """The work-queue k-NN kernel (and closest points of point BVHs) against the wave walk and the oracle.
 
 A batch of more than max(4 queries per triangle, 2^18) on a mesh, or max(1 per 2 points, 2^17) on
-points, takes the wave walk up to k = 16; smaller ones, and every k above 16, take the queue. Both
-must give the canonical lists. Sizes are the edges of its waves (1 to 32 queries each, by k), k the
+points, takes the wave walk up to k = 16; smaller ones, down to lower lines on trees of fewer than
+8,000 elements, and every k above 16, take the queue. Both must give the canonical lists. Sizes are the edges of its waves (1 to 32 queries each, by k), k the
 edges of its list widths, and trees of fewer elements than k leave slots empty.
 """
 import numpy as np
@@ -20,7 +20,7 @@ def _equal(a, b, label):
 def mesh_case():
     import thea_amd
     from thea_amd import workloads as W
-    v, t = W.torus(40, 20)
+    v, t = W.torus(90, 45)  # 8,100 triangles: the queue up to 2^18
     g = np.random.default_rng(11)
     lo, hi = W.inflated_box(v, 1.2)
     q = g.uniform(lo, hi, size=((1 << 18) + 1, 3)).astype(np.float32)

@@ -2646,17 +2646,24 @@ bool use_wave_traversal(const Bvh &b) {
 
 // Closest triangles: the work-queue kernel or the compacted wave walk. One walk for 64 queries needs
 // the fewest loads where its queries are close together, from about 1.25 queries per triangle on;
-// below that, and below 3 2^18 queries on any mesh (where the longest walk bounds the launch), the
-// queue is faster. Torus of 1,048,576 triangles, queries uniform in the box, queue against wave:
-// 500,000 2.1 / 4.1 ms, 1,000,000 3.7 / 4.7 ms, 10,000,000 21.8 / 13.2 ms; of 100,000 triangles:
-// 500,000 0.84 / 1.31 ms, 1,000,000 1.45 / 1.54 ms. THG_TRAVERSAL=queue or =wave forces one; trees
-// deeper than 63 levels take one query per lane.
+// below that, and below `small` queries (where the longest walk bounds the launch), the queue is
+// faster. Torus of 1,048,576 triangles, queries uniform in the box, queue against wave: 500,000
+// 2.1 / 4.1 ms, 1,000,000 3.7 / 4.7 ms, 10,000,000 21.8 / 13.2 ms; of 100,000 triangles: 500,000
+// 0.84 / 1.31 ms, 1,000,000 1.45 / 1.54 ms. `small` grows with the tree, since the whole of a small one
+// lies close together; whole calls near the surface / in the box, queue against wave: 8,100 triangles,
+// 524,288 queries 296 / 351 and 502 / 574 us; 4,096 triangles, 262,144 212 / 221 and 289 / 390, 524,288
+// 276 / 259 and 438 / 434; 1,024 triangles, 131,072 (as they come) 78 / 132, 196,608 157 / 135 and
+// 184 / 234, 262,144 188 / 156. THG_TRAVERSAL=queue or =wave forces one; trees deeper than 63 levels take
+// one query per lane. Queries that all lie far from the mesh share one walk far better than either
+// line allows for (20 box sizes away: 200,000 on the large torus 1.70 / 1.39 ms, 1,000,000
+// 6.8 / 4.2 ms); no size tells them apart.
 bool use_queue(int64_t n, int64_t triangles, int max_depth) {
   static const char *env = getenv("THG_TRAVERSAL");
   if (max_depth + 1 > W_STACK || (env && std::string(env) == "lane")) return false;
   if (env && std::string(env) == "wave") return n < ORDER_MIN_QUERIES;
   if (env && std::string(env) == "queue") return true;
-  return n <= std::max<int64_t>(triangles + triangles / 4, (int64_t)3 << 18);
+  const int64_t small = std::max<int64_t>((int64_t)1 << 17, ((int64_t)1 << 16) + 64 * triangles);
+  return n <= std::max<int64_t>(triangles + triangles / 4, std::min<int64_t>(small, (int64_t)3 << 18));
 }
 bool use_queue_traversal(const Bvh &b, int64_t n) { return !b.points && use_queue(n, b.n, b.max_depth); }
 
@@ -2675,16 +2682,27 @@ int queue_lanes_log2(int64_t n) {
 // 1,000,000 queries in the box 80 against 13.6 ms; 200,000 points, each one's 32 nearest, 2.84 against
 // 1.04 ms). Shorter ones share the wave walk with advantage from about 4 queries per triangle (8-NN on
 // the torus, queue / wave: 2,000,000 13.3 / 14.3 ms, 4,000,000 24.9 / 22.3 ms) or 1 per 2 points (8-NN
-// over 1,000,000 points, 500,000 of them 0.63 / 0.65 ms, all 1.08 / 0.94 ms), and always where a few
-// thousand waves would be too few to fill the GPU.
+// over 1,000,000 points, 500,000 of them 0.63 / 0.65 ms, all 1.08 / 0.94 ms), but not below `small`
+// queries, where a few thousand waves would be too few to fill the GPU: the line grows with the tree, as
+// in use_queue, and falls with the list, whose insertions the queue makes one after another. 8-NN near
+// the surface, queue against wave: 8,100 triangles, 262,144 queries 606 / 686 us; 4,096 triangles, 196,608
+// 433 / 432, 262,144 551 / 416 (in the box 496 / 600, 646 / 584); 1,024 triangles, 131,072 260 / 265,
+// 160,000 346 / 234. Points: 4 nearest of 1,000, 131,072 queries 114 / 130; 8 nearest, 100,000 160 / 154;
+// 16 nearest, 65,536 184 / 198, 100,000 278 / 211, but of 6,000 131,072 342 / 400. As there, queries that all
+// lie far from the scene or in one spot are better walked together (200,000, 20 box sizes from a sphere of
+// 20,480 triangles: 8-NN 1.92 / 0.93 ms), and no size tells them apart.
 bool use_knn_queue(const Bvh &b, int64_t n, int k) {
   static const char *env = getenv("THG_TRAVERSAL");
   if (b.max_depth + 1 > W_STACK || (env && std::string(env) == "lane")) return false;
   if (k > 16) return true;
   if (env && std::string(env) == "wave") return n < ORDER_MIN_QUERIES;
   if (env && std::string(env) == "queue") return true;
-  if (b.points) return n <= std::max<int64_t>(b.n / 2, (int64_t)1 << 17);
-  return n <= std::max<int64_t>(4 * b.n, (int64_t)1 << 18);
+  if (b.points) {
+    const int64_t small = (k <= 4 ? (int64_t)4 << 15 : k <= 8 ? (int64_t)3 << 15 : (int64_t)2 << 15) + 11 * b.n;
+    return n <= std::max<int64_t>(b.n / 2, std::min<int64_t>(small, (int64_t)1 << 17));
+  }
+  const int64_t small = (k == 1 ? (int64_t)4 << 15 : (int64_t)3 << 15) + 24 * b.n;
+  return n <= std::max<int64_t>(4 * b.n, std::min<int64_t>(small, (int64_t)1 << 18));
 }
 
 // log2 of the lanes per query: as queue_lanes_log2, with at most WQ_LIST keys per wave, and twice as
