@@ -239,8 +239,8 @@ int thg_ray_stats(thg_bvh bvh, const float *origins, const float *dirs, int64_t 
  * arrays). Results use local triangle indices. All array pointers are device pointers.
  *
  * A plan sizes every buffer once; its whole pipeline (all meshes' bounds, one Morton sort over all
- * meshes, per-mesh radix trees, one refit, one compaction, records, query sort, and one
- * multi-segment closest-point launch) has no host synchronisation, so the first run captures it into
+ * meshes, per-mesh radix trees, records and boxes, one compaction, a query sort where a mesh's batch
+ * needs one, and one multi-segment closest-point launch per kernel) has no host synchronisation, so the first run captures it into
  * a HIP graph and later runs replay it. leaf_sizes: per mesh, 1..16 (NULL = 4).
  * timings_ms (nullable): when given, the run is eager (not graph) and reports [build, query] ms. */
 typedef struct thg_batch_plan_s *thg_batch_plan;
