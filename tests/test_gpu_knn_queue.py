@@ -1,7 +1,7 @@
 """The work-queue k-NN kernel (and closest points of point BVHs) against the wave walk and the oracle.
 
 A batch of more than max(4 queries per triangle, 2^18) on a mesh, or max(1 per 2 points, 2^17) on
-points, takes the wave walk up to k = 16; smaller ones, down to lower lines on trees of fewer than
+points and any of more than 2^19 there, takes the wave walk up to k = 16; smaller ones, down to lower lines on trees of fewer than
 8,000 elements, and every k above 16, take the queue. Both must give the canonical lists. Sizes are the edges of its waves (1 to 32 queries each, by k), k the
 edges of its list widths, and trees of fewer elements than k leave slots empty.
 """
@@ -88,6 +88,23 @@ def test_points_equal_wave_walk(leaf):
         _equal(b.closest(q[:n], want_d2=True), [x[:n] for x in ref], f"closest n={n}")
         _equal(b.kClosestElements(q[:n], 6, want_d2=True), [x[:n] for x in refk], f"k-NN n={n}")
     assert (b.closest(q[:50], dist_bound=0.0)[0] == -1).all()
+
+
+@pytest.mark.parametrize("k", [1, 6])
+def test_large_point_sets_at_the_line(k):
+    """2^19 queries of 1,100,000 points take the queue, one more the wave walk."""
+    import torch
+    import thea_amd
+    g = torch.Generator(device="cuda").manual_seed(k)
+    p = torch.randn(1_100_000, 3, generator=g, device="cuda")
+    b = thea_amd.PointBvh(p)
+    q = torch.randn((1 << 19) + 1, 3, generator=g, device="cuda") * 1.3
+    q[:1000] = p[:1000]
+    for x, y in zip(b.kClosestElements(q, k, want_d2=True), b.kClosestElements(q[:-1], k, want_d2=True)):
+        assert torch.equal(x[:-1], y)
+    if k == 1:
+        for x, y in zip(b.closestPoint(q), b.closestPoint(q[:-1])):
+            assert torch.equal(x[:-1], y)
 
 
 def test_more_threads_than_one_launch_holds():

@@ -2682,7 +2682,10 @@ int queue_lanes_log2(int64_t n) {
 // 1,000,000 queries in the box 80 against 13.6 ms; 200,000 points, each one's 32 nearest, 2.84 against
 // 1.04 ms). Shorter ones share the wave walk with advantage from about 4 queries per triangle (8-NN on
 // the torus, queue / wave: 2,000,000 13.3 / 14.3 ms, 4,000,000 24.9 / 22.3 ms) or 1 per 2 points (8-NN
-// over 1,000,000 points, 500,000 of them 0.63 / 0.65 ms, all 1.08 / 0.94 ms), but not below `small`
+// over 1,000,000 points, 500,000 of them 0.63 / 0.65 ms, all 1.08 / 0.94 ms), and from 2^19 queries on
+// however many points there are (4,000,000 on a torus, queries in its box / near it: closest of 524,288
+// 810 / 699 and 356 / 647 us; 8-NN of 1,000,000 3.8 / 2.6 and 1.6 / 2.9 ms, of 2,000,000 6.3 / 3.5 and
+// 3.1 / 3.8 ms), but not below `small`
 // queries, where a few thousand waves would be too few to fill the GPU: the line grows with the tree, as
 // in use_queue, and falls with the list, whose insertions the queue makes one after another. 8-NN near
 // the surface, queue against wave: 8,100 triangles, 262,144 queries 606 / 686 us; 4,096 triangles, 196,608
@@ -2699,7 +2702,7 @@ bool use_knn_queue(const Bvh &b, int64_t n, int k) {
   if (env && std::string(env) == "queue") return true;
   if (b.points) {
     const int64_t small = (k <= 4 ? (int64_t)4 << 15 : k <= 8 ? (int64_t)3 << 15 : (int64_t)2 << 15) + 11 * b.n;
-    return n <= std::max<int64_t>(b.n / 2, std::min<int64_t>(small, (int64_t)1 << 17));
+    return n <= std::max<int64_t>(std::min<int64_t>(b.n / 2, (int64_t)1 << 19), std::min<int64_t>(small, (int64_t)1 << 17));
   }
   const int64_t small = (k == 1 ? (int64_t)4 << 15 : (int64_t)3 << 15) + 24 * b.n;
   return n <= std::max<int64_t>(4 * b.n, std::min<int64_t>(small, (int64_t)1 << 18));
