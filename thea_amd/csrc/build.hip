@@ -81,14 +81,17 @@ __global__ void __launch_bounds__(B_BLOCK) k_elem_prep(const float *__restrict__
 }
 
 // One wave per slot: the min (lo slots) or max (hi slots) of the block partials.
-// Also clears the depth, sets the node count of a single-leaf tree and marks node 0 as the root.
+// Also clears the depth, sets the words of a single-leaf tree (one: its node count and even-depth flag,
+// zero: the flag's scan and the position of a lone element) and marks node 0 as the root.
 __global__ void __launch_bounds__(12 * WAVE) k_bounds_reduce(const int *__restrict__ part, int nb,
                                                              BoundsAcc *__restrict__ acc, int32_t *__restrict__ depth,
-                                                             uint32_t *__restrict__ one, int32_t *__restrict__ parent) {
+                                                             uint32_t *__restrict__ one, uint32_t *__restrict__ zero,
+                                                             int32_t *__restrict__ parent) {
   const int k = threadIdx.x / WAVE, lane = lane_id();
   if (threadIdx.x == 0) {
     *depth = 0;
     *one = 1;
+    *zero = 0;
     parent[0] = -1;
   }
   const bool lo_slot = k < 3 || (k >= 6 && k < 9);
@@ -510,7 +513,9 @@ void launch_node_depth(int64_t max_nodes, int64_t first, const uint32_t *count, 
 }
 
 // Host driver shared by mesh and point builds. Two waits: for the bounds and the kept node count, which
-// size the nodes, and for the depth and the ray tree's node count, which sizes that.
+// size the nodes, and for the depth and the ray tree's node count, which sizes that. A tree of one leaf
+// knows the latter, and one element needs no sort (one point 163 -> 78 us, four 166 -> 133; with its mesh,
+// one triangle 317 -> 176, four 305 -> 217).
 void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool points, int leaf_size, hipStream_t s) {
   b.points = points;
   b.n = n;
@@ -539,7 +544,7 @@ void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool 
   struct Counts {  // device words read by the host
     BoundsAcc bounds;
     int32_t depth;
-    uint32_t one;
+    uint32_t one, zero;
   };
   Layout lay;
   const size_t o_cnt = lay.add(sizeof(Counts)), o_part = lay.add((size_t)grid * 12 * sizeof(int)),
@@ -562,17 +567,21 @@ void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool 
                      ws.at<int>(o_part));
   launch_check("k_elem_prep");
   hipLaunchKernelGGL(k_bounds_reduce, dim3(1), dim3(12 * WAVE), 0, s, ws.at<int>(o_part), (int)grid, &cnt->bounds,
-                     &cnt->depth, &cnt->one, parent);
+                     &cnt->depth, &cnt->one, &cnt->zero, parent);
   launch_check("k_bounds_reduce");
-  const uint32_t tiles = radix_tiles(n);
-  if (radix_items(n) == RS_ITEMS_SMALL)
-    hipLaunchKernelGGL(k_morton<RS_ITEMS_SMALL>, dim3(tiles), dim3(RS_BLOCK), 0, s, center, n, &cnt->bounds, tiles,
-                       keys, hist);
-  else
-    hipLaunchKernelGGL(k_morton<RS_ITEMS_LARGE>, dim3(tiles), dim3(RS_BLOCK), 0, s, center, n, &cnt->bounds, tiles,
-                       keys, hist);
-  launch_check("k_morton");
-  radix_sort_iota(keys, vals, ws.at<uint32_t>(o_tk), ws.at<uint32_t>(o_tv), hist, n, 0, 32, true, s);
+  if (n == 1) {
+    vals = &cnt->zero;
+  } else {
+    const uint32_t tiles = radix_tiles(n);
+    if (radix_items(n) == RS_ITEMS_SMALL)
+      hipLaunchKernelGGL(k_morton<RS_ITEMS_SMALL>, dim3(tiles), dim3(RS_BLOCK), 0, s, center, n, &cnt->bounds, tiles,
+                         keys, hist);
+    else
+      hipLaunchKernelGGL(k_morton<RS_ITEMS_LARGE>, dim3(tiles), dim3(RS_BLOCK), 0, s, center, n, &cnt->bounds, tiles,
+                         keys, hist);
+    launch_check("k_morton");
+    radix_sort_iota(keys, vals, ws.at<uint32_t>(o_tk), ws.at<uint32_t>(o_tv), hist, n, 0, 32, true, s);
+  }
 
   const BoxLevels P = box_levels(n, ws.at<float4>(o_box));
   if (points)
@@ -606,7 +615,6 @@ void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool 
   b.nodes.alloc((size_t)kept * sizeof(BNode));
   b.num_nodes = kept;
   b.num_leaves = single ? 1 : (int64_t)kept + 1;  // a full binary tree
-  const uint32_t *count = single ? &cnt->one : fidx + ni;
   if (single) {
     hipLaunchKernelGGL(k_single_leaf, dim3(1), dim3(1), 0, s, n, b.lo, b.hi, b.nodes.as<BNode>());
     launch_check("k_single_leaf");
@@ -615,22 +623,31 @@ void build_bvh(Bvh &b, const float *verts, const int32_t *tris, int64_t n, bool 
                 b.nodes.as<BNode>(), parent, s);
   }
   // even-depth flags of the nodes and their scan, for the ray tree (in the pyramid's place)
-  uint32_t *even = points ? nullptr : ws.at<uint32_t>(o_box), *qidx = keep;  // keep: ni >= kept words
-  launch_node_depth(kept, 0, count, parent, &cnt->depth, even, s);
-  uint32_t nq = 0;
+  const uint32_t *even = &cnt->one, *qidx = &cnt->zero;
+  uint32_t nq = 1;
+  if (!single) {
+    uint32_t *flags = points ? nullptr : ws.at<uint32_t>(o_box);
+    launch_node_depth(kept, 0, fidx + ni, parent, &cnt->depth, flags, s);
+    if (!points) {
+      uint32_t *scan = ws.at<uint32_t>(o_first);  // the ranges are no longer needed; o_last follows for the total
+      scan_excl_u32(flags, scan, kept, stmp, s);
+      THG_HIP(hipMemcpyAsync(&nq, scan + kept, 4, hipMemcpyDeviceToHost, s));
+      even = flags;
+      qidx = scan;
+    }
+  }
   if (!points) {
-    qidx = ws.at<uint32_t>(o_first);  // the ranges are no longer needed; o_last follows for the total
-    scan_excl_u32(even, qidx, kept, stmp, s);
-    THG_HIP(hipMemcpyAsync(&nq, qidx + kept, 4, hipMemcpyDeviceToHost, s));
     hipLaunchKernelGGL(k_leaf_ends, dim3(ceil_div(kept, B_BLOCK)), dim3(B_BLOCK), 0, s, b.nodes.as<BNode>(),
                        (int64_t)kept, b.rays.as<RayTri>());
     launch_check("k_leaf_ends");
     launch_leaf_bounds(b.nodes.as<BNode>(), (int64_t)kept, nullptr, (int64_t)kept, b.elems.as<TriRec>(),
                        b.lbounds.as<LeafBound>(), s);
   }
-  int32_t depth = 0;
-  THG_HIP(hipMemcpyAsync(&depth, &cnt->depth, 4, hipMemcpyDeviceToHost, s));
-  THG_HIP(hipStreamSynchronize(s));
+  int32_t depth = 1;
+  if (!single) {
+    THG_HIP(hipMemcpyAsync(&depth, &cnt->depth, 4, hipMemcpyDeviceToHost, s));
+    THG_HIP(hipStreamSynchronize(s));
+  }
   b.max_depth = depth;
   if (!points) build_qbvh4(b, even, qidx, nq, s);
   THG_HIP(hipStreamSynchronize(s));
